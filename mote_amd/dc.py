@@ -229,12 +229,15 @@ def _dechunk_setup(ctx, inputs, output):
     ctx.eps = eps
     ctx.has_init = init is not None
     ctx.save_for_backward(hidden, prob, perm, num, mask, cum, output[1])
+    ctx.set_materialize_grads(False)  # w has no gradient: no [B, M, D] fp32 zeros for it
 
 
 def _dechunk_backward(ctx, dout, _dz):
     if ctx.has_init:
         raise RuntimeError("mote::dechunk has no backward with a carried value (the decode-state form)")
     hidden, prob, perm, num, mask, cum, w = ctx.saved_tensors
+    if dout is None:
+        dout = torch.zeros(mask.shape[0], mask.shape[1], hidden.shape[2], device=hidden.device, dtype=hidden.dtype)
     dh, dp = dechunk_bwd(dout, hidden, prob, perm, num, mask, cum, w, ctx.eps)
     return dh, dp, None, None, None, None, None, None
 

@@ -163,10 +163,14 @@ def _setup_context(ctx, inputs, output):
     y, g, ibar, lse = output
     ctx.save_for_backward(p1, p2, info, ibar, lse, g)
     ctx.tau_s, ctx.q_start = tau_s, q_start
+    # no zero tensors for the outputs without a gradient (g, ibar, lse: the last as large as Y in fp32)
+    ctx.set_materialize_grads(False)
 
 
 def _backward(ctx, dy, _dg, _dibar, _dlse):
     p1, p2, info, ibar, lse, g = ctx.saved_tensors
+    if dy is None:  # only g, ibar or lse was differentiated: no gradient flows through them
+        dy = torch.zeros(p1.shape, device=p1.device, dtype=p1.dtype)
     dp1, dp2, dinfo, dlam = _relation_bwd(p1, p2, info, ibar, lse, g, dy, ctx.tau_s, ctx.q_start)
     return dp1, dp2, dinfo, dlam, None, None
 

@@ -123,6 +123,8 @@ def _setup(ctx, inputs, output):
     ctx.has_res = residual is not None
     ctx.res_dtype = residual.dtype if residual is not None else x.dtype
     ctx.w_dtype = weight.dtype
+    # no zero tensors for rstd, or for the stream when it is not differentiated
+    ctx.set_materialize_grads(False)
 
 
 def _backward(ctx, dy, ds_out, _drstd):

@@ -164,6 +164,7 @@ def _rg_setup(ctx, inputs, output):
     ctx.save_for_backward(qkv, inv_freq, theta)
     ctx.has_theta = theta is not None
     ctx.n_heads, ctx.parity, ctx.pos0 = n_heads, parity, pos0
+    ctx.set_materialize_grads(False)  # the backward takes a missing gradient as zeros
 
 
 def _rg_backward(ctx, dp1, dp2, dinfo):
@@ -297,6 +298,7 @@ def _qr_setup(ctx, inputs, output):
     ctx.norm = norm_w1 is not None
     ctx.keep = keep_info
     ctx.n_heads, ctx.parity, ctx.pos0, ctx.eps = n_heads, parity, pos0, norm_eps
+    ctx.set_materialize_grads(False)  # the kept projections have no gradient: no zero tensors for them
 
 
 @torch.library.custom_op("mote::head_rms_norm_bwd_", mutates_args=("dqkv",))
@@ -481,11 +483,13 @@ def _out_gate_fake(x, wg, y):
 def _og_setup(ctx, inputs, output):
     x, wg, y = inputs
     ctx.save_for_backward(x, wg, y, output[1])
+    ctx.set_materialize_grads(False)  # s has no gradient: no zero tensor for it
 
 
 def _og_backward(ctx, dz, _ds):
     """z = y s, s = sigmoid(g), g = x wg^T: dy = dz s, dg = dz y s (1 - s), dx = dg wg, dwg = dg^T x."""
     x, wg, y, s = ctx.saved_tensors
+    dz = torch.zeros_like(y) if dz is None else dz
     dzf, sf = dz.float(), s.float()
     dy = (dzf * sf).to(y.dtype)
     dg = (dzf * y.float() * sf * (1.0 - sf)).to(x.dtype)
