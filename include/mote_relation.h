@@ -447,6 +447,22 @@ typedef struct mote_wgrad_args {
 size_t mote_wgrad_workspace(const mote_wgrad_args* args);
 int mote_wgrad(const mote_wgrad_args* args, void* stream);
 
+/* The same product for widths that are multiples of 64, dW in bf16 or fp32 (dw_dtype: the fp32 sums
+ * unrounded, for fp32 master weights). Workspace, strides and M == 0 as above. */
+typedef struct mote_linear_wgrad_args {
+  int dtype;               /* MOTE_BF16: a and x */
+  int dw_dtype;            /* MOTE_BF16 or MOTE_F32 */
+  int M, N, K;
+  const void* a; int64_t a_sr;
+  const void* x; int64_t x_sr;
+  void* dw; int64_t dw_sr;
+  void* workspace;
+  size_t workspace_bytes;
+} mote_linear_wgrad_args;
+
+size_t mote_linear_wgrad_workspace(const mote_linear_wgrad_args* args);
+int mote_linear_wgrad(const mote_linear_wgrad_args* args, void* stream);
+
 /* ------------------------------------------------------------------------------------------------
  * Skinny product for the decode engine's per-token projections (bf16, fp32 accumulation):
  * y [B, N] = x [B, K] W[N, K]^T rounded to bf16, B <= 16 rows (one new chunk per sequence), N a

@@ -29,6 +29,8 @@ int check_launch(const char* what) {
 // wgrad.hip (kept out of params.hpp, whose text every recorded kernel profile is tied to)
 size_t wgrad_workspace_bytes(const mote_wgrad_args* a);
 int launch_wgrad(const mote_wgrad_args* a, hipStream_t stream);
+size_t linear_wgrad_workspace_bytes(const mote_linear_wgrad_args* a);
+int launch_linear_wgrad(const mote_linear_wgrad_args* a, hipStream_t stream);
 
 }  // namespace mote
 
@@ -120,6 +122,15 @@ int mote_arena_page_copy(const mote_page_copy_args* args, void* stream) {
 int mote_skinny_gemm(const mote_skinny_gemm_args* args, void* stream) {
   mote::g_err[0] = 0;
   return mote::launch_skinny_gemm(args, reinterpret_cast<hipStream_t>(stream));
+}
+
+size_t mote_linear_wgrad_workspace(const mote_linear_wgrad_args* args) {
+  return args ? mote::linear_wgrad_workspace_bytes(args) : 0;
+}
+
+int mote_linear_wgrad(const mote_linear_wgrad_args* args, void* stream) {
+  mote::g_err[0] = 0;
+  return mote::launch_linear_wgrad(args, reinterpret_cast<hipStream_t>(stream));
 }
 
 size_t mote_wgrad_workspace(const mote_wgrad_args* args) { return args ? mote::wgrad_workspace_bytes(args) : 0; }

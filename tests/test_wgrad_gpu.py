@@ -54,6 +54,27 @@ def test_wgrad_matches_float64(cuda, M, N, K):
     assert torch.equal(dw, again), "bitwise reproducible"
 
 
+# widths off 128 (64-wide tiles on either side or both), both output types, one split and many, ragged
+# last stages, an empty reduction. fp32 dW: sums of products of bf16 values in fp32 over M rows, so M
+# roundings of 2^-24 against a sum whose terms reach about M^(1/2) times less than their absolute sum:
+# 1e-5 of the largest element holds with room for every M here.
+@pytest.mark.parametrize("M,N,K", [(0, 64, 64), (1, 64, 192), (65, 192, 64), (300, 576, 192), (1241, 192, 128), (9929, 320, 192),
+                                   (4964, 256, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_linear_wgrad_widths_and_types(cuda, M, N, K, dtype):
+    from mote_amd.relation import _linear_wgrad
+
+    print(f"case linear_wgrad M={M} N={N} K={K} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(M, N + 8, generator=g).bfloat16().to(cuda)[:, :N]  # row stride above the width
+    x = torch.randn(M, K, generator=g).bfloat16().to(cuda)
+    dw = _linear_wgrad(a, x, dtype)
+    ref = a.double().t().contiguous() @ x.double()
+    assert dw.shape == (N, K) and dw.dtype == dtype
+    assert rel_err(dw, ref) < (1e-5 if dtype == torch.float32 else 4e-3), rel_err(dw, ref)
+    assert torch.equal(dw, _linear_wgrad(a, x, dtype)), "bitwise reproducible"
+
+
 def test_wgrad_strided_rows(cuda):
     """Operands and output as column windows of wider row-major tensors (row strides above the
     widths): only the window is read and written."""
