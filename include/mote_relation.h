@@ -424,6 +424,20 @@ typedef struct mote_gate_product_args {
 
 int mote_gate_product(const mote_gate_product_args* args, void* stream);
 
+/* The elementwise half of the gate's backward: dy = dz s, dg = dz y s (1 - s) over n contiguous bf16
+ * elements (n a multiple of 8, every pointer 16-byte aligned), fp32 arithmetic, one rounding each. */
+typedef struct mote_gate_bwd_args {
+  int dtype;               /* MOTE_BF16 */
+  int64_t n;
+  const void* dz;
+  const void* y;
+  const void* s;
+  void* dy;
+  void* dg;
+} mote_gate_bwd_args;
+
+int mote_gate_bwd(const mote_gate_bwd_args* args, void* stream);
+
 /* ------------------------------------------------------------------------------------------------
  * Weight gradient of a projection (bf16, fp32 accumulation): dW [N, K] = A^T X, A [M, N] (the
  * output gradient) and X [M, K] (the projection's input) token-major, summed over the M rows and

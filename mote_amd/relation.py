@@ -520,14 +520,32 @@ def _og_setup(ctx, inputs, output):
     ctx.set_materialize_grads(False)  # s has no gradient: no zero tensor for it
 
 
+@torch.library.custom_op("mote::gate_bwd", mutates_args=())
+def _gate_bwd(dz: torch.Tensor, y: torch.Tensor, s: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """bf16 (dy, dg) = (dz s, dz y s (1 - s)) of equally shaped bf16 tensors whose last axis is a multiple
+    of 8, contiguous results."""
+    if not dz.is_cuda:
+        raise RuntimeError("mote::gate_bwd needs the HIP library and an MI355X")
+    # the kernel walks flat memory in 16-byte chunks: copies of views in another order or off a chunk
+    dz, y, s = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (t.contiguous() for t in (dz, y, s)))
+    dy, dg = torch.empty_like(y), torch.empty_like(y)
+    a = L.GateBwdArgs()
+    a.dtype, a.n = L.dtype_code(dz), dz.numel()
+    a.dz, a.y, a.s, a.dy, a.dg = dz.data_ptr(), y.data_ptr(), s.data_ptr(), dy.data_ptr(), dg.data_ptr()
+    L.check(L.lib().mote_gate_bwd(a, L.stream_of(dz)), "mote_gate_bwd")
+    return dy, dg
+
+
+@_gate_bwd.register_fake
+def _gate_bwd_fake(dz, y, s):
+    return dz.new_empty(dz.shape), dz.new_empty(dz.shape)
+
+
 def _og_backward(ctx, dz, _ds):
     """z = y s, s = sigmoid(g), g = x wg^T: dy = dz s, dg = dz y s (1 - s), dx = dg wg, dwg = dg^T x."""
     x, wg, y, s = ctx.saved_tensors
     dz = torch.zeros_like(y) if dz is None else dz
-    dzf, sf = dz.float(), s.float()
-    dy = (dzf * sf).to(y.dtype)
-    dg = (dzf * y.float() * sf * (1.0 - sf)).to(x.dtype)
-    D = x.shape[-1]
+    dy, dg = _gate_bwd(dz, y, s)
     dx = torch.matmul(dg, wg)
     dwg = weight_grad(dg, x)
     return dx, dwg, dy

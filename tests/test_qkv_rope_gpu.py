@@ -357,6 +357,27 @@ def test_out_gate_tilings_agree_bitwise(cuda):
     assert torch.equal(z, torch.cat([z0, z1], 1)) and torch.equal(s, torch.cat([s0, s1], 1))
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 128), (2, 3, 128), (1, 517, 256)])
+def test_gate_backward_elementwise_bits(cuda, shape):
+    """mote::gate_bwd against the eager expressions it replaces, bit for bit: contiguous, transposed and
+    misaligned inputs, zero and saturated gates."""
+    from mote_amd.relation import _gate_bwd
+
+    print(f"case gate_bwd {shape}", flush=True)
+    g = torch.Generator().manual_seed(shape[1])
+    dz, y = (torch.randn(shape, generator=g).bfloat16().to(cuda) for _ in range(2))
+    s = torch.sigmoid(torch.randn(shape, generator=g) * 4).bfloat16()
+    s.view(-1)[:2] = torch.tensor([0.0, 1.0])
+    s = s.to(cuda)
+    off = torch.empty(dz.numel() + 3, device=cuda, dtype=torch.bfloat16)[3:].view(shape).copy_(dz)
+    turned = y.transpose(0, 1).contiguous().transpose(0, 1)
+    for a, b in ((dz, y), (off, turned)):
+        dy, dg = _gate_bwd(a, b, s)
+        dzf, sf = a.float(), s.float()
+        assert torch.equal(dy, (dzf * sf).bfloat16())
+        assert torch.equal(dg, (dzf * b.float() * sf * (1.0 - sf)).bfloat16())
+
+
 def test_out_gate_and_qk_norm_ops_pass_opcheck(cuda):
     from mote_amd.relation import rope_inv_freq
 
