@@ -108,9 +108,9 @@ int mote_relation_fwd(const mote_relation_fwd_args* args, void* stream);
  * Inputs are the forward's inputs and saved statistics (ibar, lse, g as produced by
  * mote_relation_fwd, dense layout) and dy ([B, H, TQ, D], any strides). Outputs dp1 [B,H,TQ,D],
  * dp2 and dinfo [B,H,TK,D] in `dtype` (any strides) and dlam (one fp32, overwritten).
- * bf16 with D in {32, 64, 96, 128} runs atomic-free kernels (key-stationary dp2/dinfo, then
+ * bf16 (row strides below 2^24 elements) runs atomic-free kernels (key-stationary dp2/dinfo, then
  * query-stationary dp1): every result is bitwise reproducible whatever `deterministic` says.
- * Other shapes (fp32, padded head dims): `deterministic` != 0 selects the atomic-free pair of
+ * Other shapes (fp32, longer row strides): `deterministic` != 0 selects the atomic-free pair of
  * kernels (the reference's MOTE_DETERMINISTIC_RELATION, flash_relation.py:51), 0 the one-pass
  * kernel with fp32 atomics for dp1.
  * The workspace is caller-allocated device memory of at least mote_relation_bwd_workspace()

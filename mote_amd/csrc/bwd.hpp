@@ -85,7 +85,7 @@ __device__ __forceinline__ void dlam_sum(const float* part, int n, float* out, f
   if (threadIdx.x == 0) *out = red[0];
 }
 
-// bf16 with D in {32, 64, 96, 128}: the atomic-free tile kernels (dP2 / dI~ key-stationary, then dP1
+// bf16: the atomic-free tile kernels (dP2 / dI~ key-stationary, then dP1
 // query-stationary), for the stages selected in `stages` (MOTE_BWD_KEYS, MOTE_BWD_QUERIES).
 void launch_bwd_tiles(const BwdParams& p, int stages, hipStream_t stream);
 

@@ -742,9 +742,11 @@ static bool fused_bwd_wanted(const mote_relation_bwd_args* a) {
   return !(e && e[0] == '0');
 }
 
-// bf16 with a head dim the tile kernels are compiled for: the atomic-free tile path.
+// bf16: the atomic-free tile path, head dims off {32, 64, 96, 128} padded to the next of them (dh 48,
+// H 4, B 16, T 1241: 194 us register-staged, 109 here; dh 88, H 2, T 3000: 244 and 85; dh 104, B 2,
+// H 8, T 1000: 148 and 58; dh 48, B 2, H 4, T 256: 27 and 19).
 static bool use_tiles(const mote_relation_bwd_args* a) {
-  return a->dtype == MOTE_BF16 && padded_dim(a->D) == a->D && tile_strides_ok(a->p1, a->p2, a->info);
+  return a->dtype == MOTE_BF16 && tile_strides_ok(a->p1, a->p2, a->info);
 }
 
 static WsLayout ws_layout(const mote_relation_bwd_args* a) {
@@ -777,7 +779,7 @@ static WsLayout ws_layout(const mote_relation_bwd_args* a) {
 
 size_t bwd_workspace_bytes(const mote_relation_bwd_args* a) { return ws_layout(a).total; }
 
-// Register-staged kernels (fp32, and bf16 head dims that need padding).
+// Register-staged kernels (fp32, and bf16 rows too far apart for the tile kernels).
 template <typename T, int DP>
 static void launch_bwd_t(const BwdParams& p, bool deterministic, int stages, hipStream_t stream) {
   const int BH = p.B * p.H;

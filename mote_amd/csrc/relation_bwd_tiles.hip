@@ -1,4 +1,4 @@
-// Atomic-free Relation backward for bf16, D in {32, 64, 96, 128} (mote/model/flash_relation.py:10-15
+// Atomic-free Relation backward for bf16, D in {32, 64, 96, 128} or padded to one of them (mote/model/flash_relation.py:10-15
 // for the algebra; the reference's two-pass `_bwd_kv_kernel` / `_bwd_q_kernel`, :370-460, has the
 // same split of the work).
 //
@@ -205,7 +205,10 @@ struct KvShape {
 // The key work of one (batch x head) bh and key block kb: 64 keys, 4 waves. FUSED (the fused launch):
 // the query blocks are walked from the last down, so the pairs of the longest query blocks are stored
 // first, and the dU quadrants of each query block are counted in the kvq counts once stored.
-template <int DP, bool FUSED>
+// PAD: head dims below DP (p.D, a multiple of 8): the key tiles' columns past D are zeroed in LDS and the
+// dI-bar rows' are zero in memory, so the staged copies in the query tile stay out of U and dW; gradient
+// columns past D are not stored.
+template <int DP, bool FUSED, bool PAD>
 __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const int kb, bf16_t* smem) {
   using E = Elem<bf16_t>;
   using Frag = E::Frag;
@@ -238,8 +241,9 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
 
   const bf16_t* srcs[2] = {qbase, dbase};
   const int64_t strides[2] = {p.q_sr, DP};
-  TileStager<DP, 4, 2> st;
-  st.init(wave, lane, strides);
+  TileStager<DP, 4, 2, PAD> st;
+  const int qdims[2] = {p.D, DP};
+  st.init(wave, lane, strides, qdims);
   auto issue = [&](int qb, int stage) {
     bf16_t* dst = smem + stage * STAGE;
     st.issue(dst, srcs, strides, qb * 64, p.TQ - 1, wave, lane);
@@ -266,13 +270,22 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
     // the key rows once (rows past the keys: finite copies whose results are never stored)
     const bf16_t* ksrc[2] = {kbase, vbase};
     const int64_t kstr[2] = {p.k_sr, p.v_sr};
-    TileStager<DP, 4, 2> kst;
-    kst.init(wave, lane, kstr);
+    TileStager<DP, 4, 2, PAD> kst;
+    const int kdims[2] = {p.D, p.D};
+    kst.init(wave, lane, kstr, kdims);
     kst.issue(kvs, ksrc, kstr, k0, p.TK - 1, wave, lane);
   }
   if (qb_lo < nqb) issue(qb_first, 0);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
+  if constexpr (PAD) {
+    const int nc = CPR - p.D / 8;  // chunks past D of a row, in both tiles
+    for (int q = tid; q < 128 * nc; q += 256) {
+      const int row = (q / nc) & 63, c = p.D / 8 + q % nc;
+      *reinterpret_cast<bf16x8*>(kvs + q / nc / 64 * TILE + row * DP + (c ^ tile_swz<DP>(row)) * 8) = bf16x8{};
+    }
+    __syncthreads();
+  }
   // FUSED: the count of a block's four dU quadrants is one atomic add by wave 0, issued right after
   // the transfers two blocks later: the waits of the next two blocks leave it in flight, so it costs
   // no wait of its own (an add waited for at the end of the next block, against the transfers, ran
@@ -392,7 +405,7 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
   for (int item = tid; item < 64 * CPR; item += 256) {
     const int row = item / CPR, d0 = (item % CPR) * 8;
     const int j = k0 + row;
-    if (j >= p.TK) continue;
+    if (j >= p.TK || (PAD && d0 >= p.D)) continue;
     float dv[8], dk[8];
 #pragma unroll
     for (int e = 0; e < 8; e += 4) {
@@ -421,12 +434,12 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
   }
 }
 
-template <int DP>
+template <int DP, bool PAD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DP <= 96 ? 2 : 1)))
 bwd_kv_kernel(const BwdParams p) {
   __shared__ __align__(16) bf16_t smem[KvShape<DP>::LDS];
   const int BH = p.B * p.H;
-  kv_job<DP, false>(p, blockIdx.x % BH, blockIdx.x / BH, smem);  // key block 0 sees the most queries: longest first
+  kv_job<DP, false, PAD>(p, blockIdx.x % BH, blockIdx.x / BH, smem);  // key block 0 sees the most queries: longest first
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -453,7 +466,7 @@ struct DqShape {
   static constexpr int LDS = NS * SLOT;
 };
 
-template <int DP, int NW, bool FUSED>
+template <int DP, int NW, bool FUSED, bool PAD>
 __device__ __forceinline__ void dq_job(const BwdParams& p, const int bh, const int qtop, bf16_t* ring) {
   using E = Elem<bf16_t>;
   using Frag = E::Frag;
@@ -461,7 +474,7 @@ __device__ __forceinline__ void dq_job(const BwdParams& p, const int bh, const i
   static_assert(!FUSED || NW == 4, "the fused launch runs four-wave jobs");
   constexpr int NQB = Q::NQB, SLOT = Q::SLOT, NS = Q::NS;
   constexpr int DT = DP / 16, CPR = DP / 8, TILE = Q::TILE;
-  using Stager = TileStager<DP, NW, 1>;
+  using Stager = TileStager<DP, NW, 1, PAD>;
   constexpr int PER = Stager::PER;        // P2 transfers per block of the busiest waves
   constexpr int RSF = DP + 4;             // fp32 row stride of the reduction buffer: an odd count of
                                           // 16-byte chunks, so a lane group's rows fall on distinct banks
@@ -505,13 +518,15 @@ __device__ __forceinline__ void dq_job(const BwdParams& p, const int bh, const i
     const int item = tid + 64 * NW * it;
     const int i = min(max(ibase + item / CPR, 0), p.TQ - 1);
     us_pre[it] = p.duii[int64_t(bh) * p.TQp + i];
-    k8_pre[it] = E::load8(kbase + int64_t(p.q_start + i) * p.k_sr + (item % CPR) * 8);
+    const int d0 = (item % CPR) * 8;
+    k8_pre[it] = E::load8(kbase + int64_t(p.q_start + i) * p.k_sr + (PAD ? min(d0, p.D - 8) : d0));
   }
 
   const bf16_t* srcs[1] = {kbase};
   const int64_t strides[1] = {p.k_sr};
   Stager st;
-  st.init(wave, lane, strides);
+  const int dims[1] = {p.D};
+  st.init(wave, lane, strides, dims);
   // Block kb: P2 rows (the staging instructions dealt over the waves) and the wave's fragments into
   // ring slot kb % NS, issued NS - 1 steps ahead; blocks past the end are not issued. A wave past its
   // own block's last key block reloads that block's last fragments (valid addresses, no products).
@@ -629,7 +644,7 @@ __device__ __forceinline__ void dq_job(const BwdParams& p, const int bh, const i
     const int item = tid + 64 * NW * it;
     const int row = item / CPR, d0 = (item % CPR) * 8;
     const int i = ibase + row;
-    if (i < 0 || i >= p.TQ) continue;
+    if (i < 0 || i >= p.TQ || (PAD && d0 >= p.D)) continue;
     const float us = us_pre[it];
     const Frag k8 = k8_pre[it];
     float o[8];
@@ -645,11 +660,11 @@ __device__ __forceinline__ void dq_job(const BwdParams& p, const int bh, const i
   }
 }
 
-template <int DP>
+template <int DP, bool PAD>
 __global__ void __launch_bounds__(512) bwd_dq_kernel(const BwdParams p) {
   __shared__ __align__(16) bf16_t ring[DqShape<DP, 8>::LDS];
   const int BH = p.B * p.H, nqb = p.TQp / 64;
-  dq_job<DP, 8, false>(p, blockIdx.x % BH, nqb - 1 - 2 * (blockIdx.x / BH), ring);  // the pair's later query block
+  dq_job<DP, 8, false, PAD>(p, blockIdx.x % BH, nqb - 1 - 2 * (blockIdx.x / BH), ring);  // the pair's later query block
   // the last workgroup (the lowest pair, the shortest) also sums dlam: the rows stage has written
   // every partial before this launch
   if (blockIdx.x == gridDim.x - 1) {
@@ -674,7 +689,7 @@ __global__ void __launch_bounds__(512) bwd_dq_kernel(const BwdParams p) {
 // work no longer fills. (With one job per workgroup instead, the dispatcher places workgroups in
 // order, round-robin over the XCDs, and one XCD without a free slot holds back every later
 // workgroup: a third of the slots stood empty through the second half of the launch.)
-template <int DP>
+template <int DP, bool PAD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) bwd_kvq_kernel(const BwdParams p) {
   constexpr int LDS = KvShape<DP>::LDS > DqShape<DP, 4>::LDS ? KvShape<DP>::LDS : DqShape<DP, 4>::LDS;
   static_assert(LDS * 2 <= 80 * 1024, "two workgroups per CU");
@@ -691,10 +706,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
     const int job = __builtin_amdgcn_readfirstlane(s_job);
     if (job >= nkey + nqj) break;
     if (job < nkey) {
-      kv_job<DP, true>(p, queue + nq * (job % hq), job / hq, lds);
+      kv_job<DP, true, PAD>(p, queue + nq * (job % hq), job / hq, lds);
     } else {
       const int j = job - nkey;
-      dq_job<DP, 4, true>(p, queue + nq * (j % hq), nqb - 1 - j / hq, lds);
+      dq_job<DP, 4, true, PAD>(p, queue + nq * (j % hq), nqb - 1 - j / hq, lds);
       if (queue == 0 && j == nqj - 1) {
         // queue 0's last job (its shortest) also sums dlam: the rows stage has written every partial
         __syncthreads();
@@ -727,7 +742,7 @@ __global__ void __launch_bounds__(256) kvq_clear_kernel(int* kvq, int n) {
     __hip_atomic_store(kvq + i, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int DP>
+template <int DP, bool PAD>
 static void launch_tiles_dp(const BwdParams& p, int stages, hipStream_t stream) {
   const int BH = p.B * p.H;
   if constexpr (DP <= 96) {
@@ -746,26 +761,33 @@ static void launch_tiles_dp(const BwdParams& p, int stages, hipStream_t stream) 
       const int resident = 2 * device_cu_count();
       const int jobs = nqb >= 12 ? nkb * BH : (nkb + nqb) * BH;
       const int grid = (jobs < resident ? jobs : resident) / p.kvq_nq * p.kvq_nq;
-      hipLaunchKernelGGL((bwd_kvq_kernel<DP>), dim3(grid > 0 ? grid : p.kvq_nq), dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((bwd_kvq_kernel<DP, PAD>), dim3(grid > 0 ? grid : p.kvq_nq), dim3(256), 0, stream, p);
       return;
     }
   }
   if (stages & MOTE_BWD_KEYS) {
     const int nkb = (p.TK + 63) / 64;
-    hipLaunchKernelGGL((bwd_kv_kernel<DP>), dim3(nkb * BH), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((bwd_kv_kernel<DP, PAD>), dim3(nkb * BH), dim3(256), 0, stream, p);
   }
   if (stages & MOTE_BWD_QUERIES) {
     const int npq = (p.TQp / 64 + 1) / 2;  // query-block pairs
-    hipLaunchKernelGGL((bwd_dq_kernel<DP>), dim3(npq * BH), dim3(512), 0, stream, p);
+    hipLaunchKernelGGL((bwd_dq_kernel<DP, PAD>), dim3(npq * BH), dim3(512), 0, stream, p);
   }
 }
 
 void launch_bwd_tiles(const BwdParams& p, int stages, hipStream_t stream) {
   switch (p.D) {
-    case 32: launch_tiles_dp<32>(p, stages, stream); break;
-    case 64: launch_tiles_dp<64>(p, stages, stream); break;
-    case 96: launch_tiles_dp<96>(p, stages, stream); break;
-    default: launch_tiles_dp<128>(p, stages, stream); break;
+    case 32: launch_tiles_dp<32, false>(p, stages, stream); return;
+    case 64: launch_tiles_dp<64, false>(p, stages, stream); return;
+    case 96: launch_tiles_dp<96, false>(p, stages, stream); return;
+    case 128: launch_tiles_dp<128, false>(p, stages, stream); return;
+    default: break;
+  }
+  switch (padded_dim(p.D)) {
+    case 32: launch_tiles_dp<32, true>(p, stages, stream); break;
+    case 64: launch_tiles_dp<64, true>(p, stages, stream); break;
+    case 96: launch_tiles_dp<96, true>(p, stages, stream); break;
+    default: launch_tiles_dp<128, true>(p, stages, stream); break;
   }
 }
 

@@ -505,7 +505,9 @@ struct FwdTileShape {
 // One (query block, sequence, head) of the tile forward (or one key-range half of it when split),
 // by its block id (the launch order: head fastest, then (when split) the halves, then query blocks
 // longest first); every wave of the workgroup calls it.
-template <int DP>
+// PAD: head dims below DP (p.D, a multiple of 8). The queries' columns past D are zero, which keeps the
+// staged copies there (TileStager) out of the scores; I-bar columns past D are not stored.
+template <int DP, bool PAD>
 __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, bf16_t* smem) {
   using E = Elem<bf16_t>;
   using Frag = E::Frag;
@@ -560,7 +562,7 @@ __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, 
     const int qi = q0 + 16 * s + li;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
-      qf[s][ks] = qi < TQs ? E::load8(qbase + int64_t(qi) * p.q_sr + 32 * ks + 8 * lg) : E::zero();
+      qf[s][ks] = qi < TQs && (!PAD || 32 * ks + 8 * lg < p.D) ? E::load8(qbase + int64_t(qi) * p.q_sr + 32 * ks + 8 * lg) : E::zero();
     qabs[s] = qs + qi;
   }
   const int qlast = min(TQs, qb * 64 + 64) - 1;
@@ -574,8 +576,9 @@ __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, 
 
   const bf16_t* srcs[2] = {kbase, vbase};
   const int64_t strides[2] = {p.k_sr, p.v_sr};
-  TileStager<DP, 4, 2> st;
-  st.init(wave, lane, strides);
+  TileStager<DP, 4, 2, PAD> st;
+  const int dims[2] = {p.D, p.D};
+  st.init(wave, lane, strides, dims);
   const float c2 = p.scale * kLog2e;
   float m_run[2] = {0.f, 0.f};
   f32x4 lacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
@@ -708,6 +711,7 @@ __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, 
     if (qv) {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
+        if (PAD && 32 * ks + 8 * lg >= p.D) continue;
         const Frag kr = E::load8(kbase + int64_t(qa) * p.k_sr + 32 * ks + 8 * lg);
 #pragma unroll
         for (int j = 0; j < 8; ++j) ud = fmaf((float)qf[s][ks].v[j], (float)kr.v[j], ud);
@@ -720,10 +724,11 @@ __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, 
     if (!qv) continue;
     const bf16_t* irow = vbase + int64_t(qa) * p.v_sr;
     bf16_t* yrow = ybase + int64_t(qi) * p.y_sr;
-    float* brow = p.ibar + (soff + qi) * int64_t(DP);
+    float* brow = p.ibar + (soff + qi) * int64_t(PAD ? p.D : DP);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       const int d0 = 16 * dt + 4 * lg;
+      if (PAD && d0 >= p.D) continue;
       const uint2 iv = *reinterpret_cast<const uint2*>(irow + d0);
       const float ivf[4] = {bf2f(iv.x & 0xffffu), bf2f(iv.x >> 16), bf2f(iv.y & 0xffffu), bf2f(iv.y >> 16)};
       float ib[4], yv[4];
@@ -745,11 +750,11 @@ __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, 
   }
 }
 
-template <int DP>
+template <int DP, bool PAD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 relation_fwd_tile_kernel(const FwdParams p) {
   __shared__ __align__(16) bf16_t smem[FwdTileShape<DP>::LDS];
-  fwd_tile_job<DP>(p, blockIdx.x, smem);
+  fwd_tile_job<DP, PAD>(p, blockIdx.x, smem);
 }
 
 // The same jobs taken by persistent workgroups (two per CU) from per-queue counters: queue q holds the
@@ -762,7 +767,7 @@ relation_fwd_tile_kernel(const FwdParams p) {
 // parameters reach each job through an opaque pointer to the kernel argument: the compiler then reads
 // them (scalar loads) inside each job instead of holding every value it derives from them across the
 // loop (61 scalar registers spilled, 6 now).
-template <int DP>
+template <int DP, bool PAD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 relation_fwd_tile_persistent_kernel(const FwdParams p) {
   __shared__ __align__(16) bf16_t smem[FwdTileShape<DP>::LDS];
@@ -781,7 +786,7 @@ relation_fwd_tile_persistent_kernel(const FwdParams p) {
     ConstFwdParams pp = (ConstFwdParams)__builtin_amdgcn_kernarg_segment_ptr();  // the kernel's one argument
     asm volatile("" : "+s"(pp));
     const FwdParams& q = *(const FwdParams*)pp;
-    fwd_tile_job<DP>(q, h + q.H * rest, smem);
+    fwd_tile_job<DP, PAD>(q, h + q.H * rest, smem);
     __syncthreads();  // the next job reuses the LDS and s_job
   }
 }
@@ -792,7 +797,7 @@ __global__ void __launch_bounds__(64) fwd_jobs_clear_kernel(int* jobs) {
 
 // Merge of the two halves of a split query block, then the epilogue of relation_fwd_tile_kernel:
 // four threads per row, each owning DP / 4 head-dim elements.
-template <int DP>
+template <int DP, bool PAD>
 __global__ void __launch_bounds__(256) relation_fwd_merge_kernel(const FwdParams p) {
   constexpr int PER = DP / 4;  // elements per thread
   const int tid = threadIdx.x;
@@ -847,6 +852,7 @@ __global__ void __launch_bounds__(256) relation_fwd_merge_kernel(const FwdParams
   if (qv) {
 #pragma unroll
     for (int c = 0; c < PER; c += 8) {
+      if (PAD && d0 + c >= p.D) break;
       const bf16x8 q8 = *reinterpret_cast<const bf16x8*>(qrow + d0 + c);
       const bf16x8 k8 = *reinterpret_cast<const bf16x8*>(krow + d0 + c);
 #pragma unroll
@@ -860,9 +866,10 @@ __global__ void __launch_bounds__(256) relation_fwd_merge_kernel(const FwdParams
   if (!qv) return;
   const bf16_t* irow = reinterpret_cast<const bf16_t*>(p.info) + voff + int64_t(h) * p.v_sh + int64_t(qa) * p.v_sr;
   bf16_t* yrow = reinterpret_cast<bf16_t*>(p.y) + yoff + int64_t(h) * p.y_sh + int64_t(qi) * p.y_sr;
-  float* brow = p.ibar + (soff + qi) * int64_t(DP);
+  float* brow = p.ibar + (soff + qi) * int64_t(PAD ? p.D : DP);
 #pragma unroll
   for (int c = 0; c < PER; c += 8) {
+    if (PAD && d0 + c >= p.D) break;
     const bf16x8 i8 = *reinterpret_cast<const bf16x8*>(irow + d0 + c);
     float ib[8], yv[8];
 #pragma unroll
@@ -906,9 +913,12 @@ static void launch_fwd_dp(const FwdParams& fp, int DP, int nblocks, hipStream_t 
 
 static bool view_ok(const mote_view& v) { return v.data != nullptr; }
 
-// The tile kernel serves bf16 with D in {32, 64, 96, 128} and row strides below 2^24.
+// The tile kernel serves bf16 with row strides below 2^24: D in {32, 64, 96, 128} as they are, other head
+// dims padded to the next of these. Padded it beats the register-staged kernel, which pays a transpose
+// and two barriers a block, at every size tried (dh 48, H 4, B 16, T 1241: 59.3 -> 42.8 us; dh 88, H 2,
+// T 3000: 146 -> 42; dh 104, B 2, H 8, T 1000: 63 -> 26; dh 48, B 2, H 4, T 256: 14.5 -> 9.2).
 static bool fwd_tiles(const mote_relation_fwd_args* a) {
-  return a->dtype == MOTE_BF16 && padded_dim(a->D) == a->D && tile_strides_ok(a->p1, a->p2, a->info);
+  return a->dtype == MOTE_BF16 && tile_strides_ok(a->p1, a->p2, a->info);
 }
 
 // Key blocks of the longest query block; query blocks with more than split_c of them run as halves.
@@ -944,7 +954,7 @@ size_t fwd_workspace_bytes(const mote_relation_fwd_args* a) {
   if (!a || a->TQ <= 0 || a->D <= 0 || a->D > 128 || !fwd_tiles(a)) return 0;
   if (fwd_split_c(a) >= (1 << 30)) return fwd_persistent(a) ? kFwdJobBytes : 0;
   const size_t nqb = (size_t(a->TQ) + 63) / 64;
-  return size_t(a->B) * a->H * nqb * 2 * (64 * size_t(a->D) + 128) * sizeof(float);
+  return size_t(a->B) * a->H * nqb * 2 * (64 * size_t(padded_dim(a->D)) + 128) * sizeof(float);
 }
 
 int launch_fwd(const mote_relation_fwd_args* a, hipStream_t stream) {
@@ -1006,19 +1016,28 @@ int launch_fwd(const mote_relation_fwd_args* a, hipStream_t stream) {
     const int resident = 2 * device_cu_count();
     const int pgrid = (resident < nb ? resident : nb) / fp.jobs_nq * fp.jobs_nq;
     if (persist) hipLaunchKernelGGL(fwd_jobs_clear_kernel, dim3(1), dim3(64), 0, stream, fp.jobs);
-#define MOTE_FWD_TILE(DPV)                                                                                      \
+#define MOTE_FWD_TILE(DPV, PADV)                                                                                \
   if (persist) {                                                                                                \
-    hipLaunchKernelGGL((relation_fwd_tile_persistent_kernel<DPV>), dim3(pgrid > 0 ? pgrid : fp.jobs_nq), dim3(256), 0, \
+    hipLaunchKernelGGL((relation_fwd_tile_persistent_kernel<DPV, PADV>), dim3(pgrid > 0 ? pgrid : fp.jobs_nq), dim3(256), 0, \
                        stream, fp);                                                                             \
   } else {                                                                                                      \
-    hipLaunchKernelGGL((relation_fwd_tile_kernel<DPV>), dim3(split ? 2 * nb : nb), dim3(256), 0, stream, fp);    \
-    if (split) hipLaunchKernelGGL((relation_fwd_merge_kernel<DPV>), dim3(nb), dim3(256), 0, stream, fp);          \
+    hipLaunchKernelGGL((relation_fwd_tile_kernel<DPV, PADV>), dim3(split ? 2 * nb : nb), dim3(256), 0, stream, fp);    \
+    if (split) hipLaunchKernelGGL((relation_fwd_merge_kernel<DPV, PADV>), dim3(nb), dim3(256), 0, stream, fp);          \
   }
-    switch (DP) {
-      case 32: MOTE_FWD_TILE(32) break;
-      case 64: MOTE_FWD_TILE(64) break;
-      case 96: MOTE_FWD_TILE(96) break;
-      default: MOTE_FWD_TILE(128) break;
+    if (DP == a->D) {
+      switch (DP) {
+        case 32: MOTE_FWD_TILE(32, false) break;
+        case 64: MOTE_FWD_TILE(64, false) break;
+        case 96: MOTE_FWD_TILE(96, false) break;
+        default: MOTE_FWD_TILE(128, false) break;
+      }
+    } else {
+      switch (DP) {
+        case 32: MOTE_FWD_TILE(32, true) break;
+        case 64: MOTE_FWD_TILE(64, true) break;
+        case 96: MOTE_FWD_TILE(96, true) break;
+        default: MOTE_FWD_TILE(128, true) break;
+      }
     }
 #undef MOTE_FWD_TILE
   } else if (a->dtype == MOTE_BF16) {

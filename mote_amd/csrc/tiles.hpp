@@ -130,17 +130,32 @@ __device__ __forceinline__ typename Elem<bf16_t>::Frag tile_row_frag(const bf16_
 // scalar base with constant offset registers. `wave` must be wave-uniform (readfirstlane), which
 // keeps the LDS destinations and the per-block bases in scalar registers. Row strides must stay below
 // 2^24 elements (checked by the host launchers), so the offsets fit 32 bits.
-template <int DP, int NW, int NT>
+// PAD: rows of fewer than DP elements (dlim[t] of tile t, a multiple of 8): the columns past them get a
+// copy of the row's last chunk (no read past the row), which the kernels keep out of their results:
+// the other operand of a product over the head dim holds zeros there, and accumulator columns there are
+// not stored.
+template <int DP, int NW, int NT, bool PAD = false>
 struct TileStager {
   static constexpr int CPR = DP / 8;
   static constexpr int NINS = NT * CPR;
   static constexpr int PER = (NINS + NW - 1) / NW;
   uint32_t voff[PER];  // bytes
+  int dlim[PAD ? NT : 1];
 
   __device__ __forceinline__ static int row_of(int n, int lane) { return (64 * n + lane) / CPR; }
   __device__ __forceinline__ static int col_of(int n, int lane) {
     const int q = 64 * n + lane;
     return ((q % CPR) ^ tile_swz<DP>(q / CPR)) * 8;
+  }
+
+  __device__ __forceinline__ int col(int t, int n, int lane) const {
+    return PAD ? min(col_of(n, lane), dlim[t] - 8) : col_of(n, lane);
+  }
+
+  __device__ __forceinline__ void init(int wave, int lane, const int64_t (&stride)[NT], const int (&d)[NT]) {
+#pragma unroll
+    for (int t = 0; t < (PAD ? NT : 0); ++t) dlim[t] = d[t];
+    init(wave, lane, stride);
   }
 
   __device__ __forceinline__ void init(int wave, int lane, const int64_t (&stride)[NT]) {
@@ -149,7 +164,7 @@ struct TileStager {
     for (int i = 0; i < PER; ++i) {
       const int ins = wave + NW * i;
       const int t = ins < NINS ? ins / CPR : 0, n = ins % CPR;
-      voff[i] = uint32_t(row_of(n, lane) * int(stride[t]) + col_of(n, lane)) * 2u;
+      voff[i] = uint32_t(row_of(n, lane) * int(stride[t]) + col(t, n, lane)) * 2u;
     }
   }
 
@@ -181,7 +196,7 @@ struct TileStager {
         if (NINS % NW == 0 || ins < NINS) {
           const int t = ins / CPR, n = ins % CPR;
           const int j = min(r0 + row_of(n, lane), rlast);
-          load(src[t] + int64_t(j) * stride[t] + col_of(n, lane), dst + t * 64 * DP + n * 512);
+          load(src[t] + int64_t(j) * stride[t] + col(t, n, lane), dst + t * 64 * DP + n * 512);
         }
       }
     }

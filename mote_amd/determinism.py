@@ -1,9 +1,9 @@
 """Reproducible-backward switch for the Relation path (the interface of mote/determinism.py:41-62).
 
 What varies between two identical backward passes here:
-* the bf16 tile backward (every preset) never varies: it has no atomics, and dlam is summed in a fixed
+* the bf16 tile backward (every head dim) never varies: it has no atomics, and dlam is summed in a fixed
   order by one workgroup;
-* the fp32 and padded-head-dim backward adds dP1 with fp32 atomics unless `DETERMINISTIC` is set,
+* the fp32 backward (and bf16 rows 2^24 or more elements apart) adds dP1 with fp32 atomics unless `DETERMINISTIC` is set,
   which selects the query-stationary pass instead;
 * library GEMMs around the path (projections, `wo`) follow torch's deterministic-algorithms mode.
 
