@@ -745,8 +745,13 @@ static bool fused_bwd_wanted(const mote_relation_bwd_args* a) {
 // bf16: the atomic-free tile path, head dims off {32, 64, 96, 128} padded to the next of them (dh 48,
 // H 4, B 16, T 1241: 194 us register-staged, 109 here; dh 88, H 2, T 3000: 244 and 85; dh 104, B 2,
 // H 8, T 1000: 148 and 58; dh 48, B 2, H 4, T 256: 27 and 19).
+// The tiles' workspace grows with the pairs of blocks (8 KB each), the register-staged kernels' with the
+// rows: padded head dims whose pairs would take more than 8 GiB (H 4: 45 K rows) stay with the latter, so
+// a length that fitted the card before still does.
 static bool use_tiles(const mote_relation_bwd_args* a) {
-  return a->dtype == MOTE_BF16 && tile_strides_ok(a->p1, a->p2, a->info);
+  if (a->dtype != MOTE_BF16 || !tile_strides_ok(a->p1, a->p2, a->info)) return false;
+  if (padded_dim(a->D) == a->D) return true;
+  return int64_t(a->B) * a->H * PairTable::total(a->TQ, a->q_start) <= (int64_t(8) << 30) / 8192;
 }
 
 static WsLayout ws_layout(const mote_relation_bwd_args* a) {
