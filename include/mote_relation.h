@@ -404,6 +404,18 @@ typedef struct mote_head_norm_bwd_args {
 size_t mote_head_rms_norm_bwd_workspace(const mote_head_norm_bwd_args* args);
 int mote_head_rms_norm_bwd(const mote_head_norm_bwd_args* args, void* stream);
 
+/* Three fp32 weights of n elements each (n a multiple of 8) as one bf16 stack [w0; w1; w2] of 3 n
+ * elements, rounded to nearest even; every pointer 16-byte aligned, nothing overlapping. */
+typedef struct mote_pack_weights_args {
+  int64_t n;
+  const void* w0;
+  const void* w1;
+  const void* w2;
+  void* out;
+} mote_pack_weights_args;
+
+int mote_pack_weights(const mote_pack_weights_args* args, void* stream);
+
 /* ------------------------------------------------------------------------------------------------
  * Output gate of FullRelation._out (bf16): z = y * sigmoid(x wg^T) with the product rounded to bf16,
  * the sigmoid rounded to bf16 and z rounded again (the reference's bf16 ops, relation.py:179-181),

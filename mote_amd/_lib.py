@@ -155,6 +155,10 @@ class WgradArgs(C.Structure):
     ]
 
 
+class PackWeightsArgs(C.Structure):
+    _fields_ = [("n", C.c_int64), ("w0", C.c_void_p), ("w1", C.c_void_p), ("w2", C.c_void_p), ("out", C.c_void_p)]
+
+
 class GateBwdArgs(C.Structure):
     _fields_ = [
         ("dtype", C.c_int), ("n", C.c_int64), ("dz", C.c_void_p), ("y", C.c_void_p), ("s", C.c_void_p),
@@ -262,6 +266,7 @@ EXPORTS = {
     "mote_qkv_rope_workspace": ([C.POINTER(QkvRopeArgs)], C.c_size_t),
     "mote_qkv_rope_fwd": ([C.POINTER(QkvRopeArgs), C.c_void_p], C.c_int),
     "mote_gate_product": ([C.POINTER(GateProductArgs), C.c_void_p], C.c_int),
+    "mote_pack_weights": ([C.POINTER(PackWeightsArgs), C.c_void_p], C.c_int),
     "mote_gate_bwd": ([C.POINTER(GateBwdArgs), C.c_void_p], C.c_int),
     "mote_head_rms_norm_bwd_workspace": ([C.POINTER(HeadNormBwdArgs)], C.c_size_t),
     "mote_head_rms_norm_bwd": ([C.POINTER(HeadNormBwdArgs), C.c_void_p], C.c_int),
@@ -289,7 +294,8 @@ STRUCTS = {
     "mote_rope_givens_args": RopeArgs, "mote_rope_givens_bwd_args": RopeBwdArgs,
     "mote_relation_decode_args": DecodeArgs, "mote_add_rms_norm_args": NormArgs,
     "mote_add_rms_norm_bwd_args": NormBwdArgs, "mote_qkv_rope_args": QkvRopeArgs,
-    "mote_gate_product_args": GateProductArgs, "mote_gate_bwd_args": GateBwdArgs, "mote_head_norm_bwd_args": HeadNormBwdArgs, "mote_skinny_gemm_args": SkinnyGemmArgs,
+    "mote_gate_product_args": GateProductArgs, "mote_gate_bwd_args": GateBwdArgs,
+    "mote_pack_weights_args": PackWeightsArgs, "mote_head_norm_bwd_args": HeadNormBwdArgs, "mote_skinny_gemm_args": SkinnyGemmArgs,
     "mote_wgrad_args": WgradArgs, "mote_linear_wgrad_args": LinearWgradArgs,
     "mote_page_copy_args": PageCopyArgs, "mote_chunk_route_args": ChunkRouteArgs,
     "mote_chunk_gather_args": ChunkGatherArgs, "mote_chunk_gather_bwd_args": ChunkGatherBwdArgs,

@@ -116,6 +116,9 @@ const Entry kLayout[] = {
     F(mote_gate_product_args, x), F(mote_gate_product_args, x_sr), F(mote_gate_product_args, w),
     F(mote_gate_product_args, w_sr), F(mote_gate_product_args, y), F(mote_gate_product_args, y_sr),
     F(mote_gate_product_args, z), F(mote_gate_product_args, s), F(mote_gate_product_args, z_sr),
+    MOTE_STRUCT(mote_pack_weights_args),
+    F(mote_pack_weights_args, n), F(mote_pack_weights_args, w0), F(mote_pack_weights_args, w1),
+    F(mote_pack_weights_args, w2), F(mote_pack_weights_args, out),
     MOTE_STRUCT(mote_gate_bwd_args),
     F(mote_gate_bwd_args, dtype), F(mote_gate_bwd_args, n), F(mote_gate_bwd_args, dz), F(mote_gate_bwd_args, y),
     F(mote_gate_bwd_args, s), F(mote_gate_bwd_args, dy), F(mote_gate_bwd_args, dg),

@@ -236,14 +236,7 @@ def _rope_table_ws(a, x: torch.Tensor, inv: Optional[torch.Tensor], cacheable: b
     return ws, 0
 
 
-@torch.library.custom_op("mote::qkv_rope", mutates_args=())
-def _qkv_rope(x: torch.Tensor, w: torch.Tensor, inv_freq: Optional[torch.Tensor], theta: Optional[torch.Tensor],
-              n_heads: int, parity: int, pos0: int, keep_info: bool, norm_w1: Optional[torch.Tensor] = None,
-              norm_w2: Optional[torch.Tensor] = None, norm_eps: float = 1e-5
-              ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    """(p1, p2, I~) as [B, H, T, dh] views of x [w1; w2; wi]^T after (QK-Norm,) RoPE / Givens, and for
-    the backward (keep_info): the I~ projections before the rotation ([B, T, H dh]) and, with QK-Norm,
-    the p1 | p2 projections before the norm ([B, T, 2 H dh]); empty otherwise."""
+def _qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps):
     if not x.is_cuda:
         raise RuntimeError("mote::qkv_rope needs the HIP library and an MI355X")
     B, T, K = x.shape
@@ -279,6 +272,17 @@ def _qkv_rope(x: torch.Tensor, w: torch.Tensor, inv_freq: Optional[torch.Tensor]
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
     L.check(L.lib().mote_qkv_rope_fwd(a, L.stream_of(x)), "mote_qkv_rope_fwd")
     return p1, p2, info, iraw, qkraw
+
+
+@torch.library.custom_op("mote::qkv_rope", mutates_args=())
+def _qkv_rope(x: torch.Tensor, w: torch.Tensor, inv_freq: Optional[torch.Tensor], theta: Optional[torch.Tensor],
+              n_heads: int, parity: int, pos0: int, keep_info: bool, norm_w1: Optional[torch.Tensor] = None,
+              norm_w2: Optional[torch.Tensor] = None, norm_eps: float = 1e-5
+              ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(p1, p2, I~) as [B, H, T, dh] views of x [w1; w2; wi]^T after (QK-Norm,) RoPE / Givens, and for
+    the backward (keep_info): the I~ projections before the rotation ([B, T, H dh]) and, with QK-Norm,
+    the p1 | p2 projections before the norm ([B, T, 2 H dh]); empty otherwise."""
+    return _qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps)
 
 
 @_qkv_rope.register_fake
@@ -411,44 +415,54 @@ def _wgrad_serves(a_dtype: torch.dtype, x_dtype: torch.dtype, N: int, K: int) ->
     return USE_WGRAD and a_dtype == torch.bfloat16 and x_dtype == torch.bfloat16 and N % 64 == 0 and K % 64 == 0
 
 
-def weight_grad(a: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """a^T x over the token rows of a [..., N] and x [..., K]: the weight gradient of y = x W^T.
-    mote_linear_wgrad for bf16 on the GPU with N, K multiples of 64; the GEMM library otherwise."""
+def weight_grad(a: torch.Tensor, x: torch.Tensor, dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+    """a^T x over the token rows of a [..., N] and x [..., K]: the weight gradient of y = x W^T, in a's
+    dtype or `dtype` (fp32: the sums unrounded). mote_linear_wgrad for bf16 on the GPU with N, K
+    multiples of 64; the GEMM library otherwise."""
     N, K = a.shape[-1], x.shape[-1]
     a2, x2 = a.reshape(-1, N), x.reshape(-1, K)
-    if a2.is_cuda and _wgrad_serves(a2.dtype, x2.dtype, N, K):
-        return _linear_wgrad(a2, x2, a2.dtype)
-    return torch.matmul(a2.t(), x2)
+    dtype = a2.dtype if dtype is None else dtype
+    # under create_graph the product has to be differentiable itself
+    if a2.is_cuda and _wgrad_serves(a2.dtype, x2.dtype, N, K) and not torch.is_grad_enabled():
+        return _linear_wgrad(a2, x2, dtype)
+    return torch.matmul(a2.t(), x2).to(dtype)
 
 
 class _LinearWgrad(torch.autograd.Function):
-    """y = x W^T on the GEMM library; backward dx = dy W on the library and dW = dy^T x on
-    mote_wgrad (the library runs that product with its reduction over the token rows)."""
+    """y = x W^T on the GEMM library for bf16 x and bf16 or fp32 W (rounded to bf16 first, as autocast
+    does); backward dx = dy W on the library and dW = dy^T x on mote_linear_wgrad in W's own dtype
+    (the library runs that product with its reduction over the token rows)."""
 
     @staticmethod
     def forward(ctx, x, w):
-        ctx.save_for_backward(x, w)
-        return F.linear(x, w)
+        wb = w.to(x.dtype)
+        ctx.save_for_backward(x, w, wb)
+        return F.linear(x, wb)
 
     @staticmethod
     def backward(ctx, dy):
-        x, w = ctx.saved_tensors
-        dx = torch.matmul(dy, w) if ctx.needs_input_grad[0] else None
-        dw = weight_grad(dy, x) if ctx.needs_input_grad[1] else None
+        x, w, wb = ctx.saved_tensors
+        if torch.is_grad_enabled():  # create_graph: through the cast of W
+            wb = w.to(x.dtype)
+        dx = torch.matmul(dy, wb) if ctx.needs_input_grad[0] else None
+        dw = weight_grad(dy, x, w.dtype) if ctx.needs_input_grad[1] else None
         return dx, dw
 
 
 def linear_wgrad(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear(x, w) whose weight gradient runs on mote_linear_wgrad: bf16 x and w on the GPU (or bf16
     autocast, which casts both as F.linear would) with both widths multiples of 64; F.linear otherwise."""
-    if torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") == torch.bfloat16 and x.is_cuda:
-        x, w = x.to(torch.bfloat16), w.to(torch.bfloat16)
-    if x.is_cuda and _wgrad_serves(x.dtype, w.dtype, w.shape[0], w.shape[1]):
+    auto = torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") == torch.bfloat16 and x.is_cuda
+    if auto:
+        x = x.to(torch.bfloat16)
+    wdt = torch.bfloat16 if auto and w.dtype == torch.float32 else w.dtype  # autocast rounds fp32 weights
+    if x.is_cuda and w.is_cuda and _wgrad_serves(x.dtype, wdt, w.shape[0], w.shape[1]):
         return _LinearWgrad.apply(x, w)
     return F.linear(x, w)
 
 
-def _qr_backward(ctx, dp1, dp2, dinfo, _diraw, _dqkraw):
+def _qr_grads(ctx, dp1, dp2, dinfo, wdtype):
+    """(dx, dW of the stacked weight in wdtype, dtheta, the gains' gradients) of the fused prologue."""
     x, w, inv_freq, theta, iraw, norm_w1, norm_w2, qkraw = ctx.saved_tensors
     if (ctx.has_theta or ctx.norm) and not ctx.keep:
         raise RuntimeError("mote::qkv_rope: the backward needs keep_info=True with theta or QK-Norm")
@@ -466,11 +480,57 @@ def _qr_backward(ctx, dp1, dp2, dinfo, _diraw, _dqkraw):
         dn1, dn2 = _head_norm_bwd_(dqkv, qkraw, norm_w1, norm_w2, ctx.eps, H)
         dn1, dn2 = dn1.to(norm_w1.dtype), dn2.to(norm_w2.dtype)
     dx = torch.matmul(dqkv, w)                                        # [B, T, 3K] x [3K, K]
-    dw = weight_grad(dqkv, x)                                        # [3K, K]
-    return (dx, dw, None, (dtheta[: H // 2] if ctx.has_theta else None), None, None, None, None, dn1, dn2, None)
+    dw = weight_grad(dqkv, x, wdtype)                                # [3K, K]
+    return dx, dw, (dtheta[: H // 2] if ctx.has_theta else None), dn1, dn2
+
+
+def _qr_backward(ctx, dp1, dp2, dinfo, _diraw, _dqkraw):
+    dx, dw, dtheta, dn1, dn2 = _qr_grads(ctx, dp1, dp2, dinfo, None)
+    return dx, dw, None, dtheta, None, None, None, None, dn1, dn2, None
 
 
 _qkv_rope.register_autograd(_qr_backward, setup_context=_qr_setup)
+
+
+# ---- mote::qkv_rope_master (the prologue from fp32 master weights) --------------------------------
+@torch.library.custom_op("mote::qkv_rope_master", mutates_args=())
+def _qkv_rope_master(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, wi: torch.Tensor,
+                     inv_freq: Optional[torch.Tensor], theta: Optional[torch.Tensor], n_heads: int, parity: int,
+                     pos0: int, keep_info: bool, norm_w1: Optional[torch.Tensor] = None,
+                     norm_w2: Optional[torch.Tensor] = None, norm_eps: float = 1e-5
+                     ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    """mote::qkv_rope of the bf16 stack of three fp32 weights [H dh, H dh], made in one launch; the stack
+    is the sixth output (kept for the backward's dx)."""
+    if not x.is_cuda:
+        raise RuntimeError("mote::qkv_rope_master needs the HIP library and an MI355X")
+    ws = [t if t.data_ptr() % 16 == 0 else t.clone() for t in (w1.contiguous(), w2.contiguous(), wi.contiguous())]
+    N, K = w1.shape
+    w = torch.empty(3 * N, K, device=x.device, dtype=torch.bfloat16)
+    a = L.PackWeightsArgs()
+    a.n, a.out = N * K, w.data_ptr()
+    a.w0, a.w1, a.w2 = (t.data_ptr() for t in ws)
+    L.check(L.lib().mote_pack_weights(a, L.stream_of(x)), "mote_pack_weights")
+    return (*_qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps), w)
+
+
+@_qkv_rope_master.register_fake
+def _qkv_rope_master_fake(x, w1, w2, wi, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1=None, norm_w2=None,
+                          norm_eps=1e-5):
+    w = x.new_empty((3 * w1.shape[0], w1.shape[1]))
+    return (*_qkv_rope_fake(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps), w)
+
+
+def _qrm_setup(ctx, inputs, output):
+    x, _w1, _w2, _wi, *rest = inputs
+    _qr_setup(ctx, (x, output[5], *rest), output)
+
+
+def _qrm_backward(ctx, dp1, dp2, dinfo, _diraw, _dqkraw, _dw):
+    dx, dw, dtheta, dn1, dn2 = _qr_grads(ctx, dp1, dp2, dinfo, torch.float32)
+    return (dx, *dw.chunk(3), None, dtheta, None, None, None, None, dn1, dn2, None)
+
+
+_qkv_rope_master.register_autograd(_qrm_backward, setup_context=_qrm_setup)
 
 
 def qkv_rope(x: torch.Tensor, w: torch.Tensor, n_heads: int, inv_freq: Optional[torch.Tensor],
@@ -480,11 +540,15 @@ def qkv_rope(x: torch.Tensor, w: torch.Tensor, n_heads: int, inv_freq: Optional[
     the same as rope_givens(F.linear(x, w), ...) (relation.py:199-215); `norm` = (p1 gain, p2 gain,
     eps) applies QK-Norm to p1 / p2 first (relation.py:208-210). Differentiable in x, w, theta and
     the gains."""
+    return _qkv_rope_of(x, w, n_heads, inv_freq, theta, layer_idx, pos0, norm)
+
+
+def _qkv_rope_of(x, w, n_heads, inv_freq, theta, layer_idx, pos0, norm):
+    """qkv_rope for a stacked weight, or for a tuple of the three fp32 weights."""
     n1, n2, eps = norm if norm is not None else (None, None, 1e-5)
     keep = torch.is_grad_enabled() and (theta is not None or norm is not None)
-    p1, p2, info, _, _ = _qkv_rope(x, w, inv_freq, theta, int(n_heads), int(layer_idx) % 2, int(pos0), keep,
-                                   n1, n2, float(eps))
-    return p1, p2, info
+    args = (inv_freq, theta, int(n_heads), int(layer_idx) % 2, int(pos0), keep, n1, n2, float(eps))
+    return (_qkv_rope_master(x, *w, *args) if isinstance(w, tuple) else _qkv_rope(x, w, *args))[:3]
 
 
 # ---- mote::out_gate (the output gate of _out) ----------------------------------------------------
@@ -647,15 +711,19 @@ class FullRelation(nn.Module):
         """Projections -> (QK-Norm) -> RoPE / Givens: (p1, p2, I~) as [B, H, T, dh] views."""
         B, T, D = x.shape
         H, dh = self.n_heads, self.d_head
-        w = torch.cat([self.w1.weight, self.w2.weight, self.wi.weight], dim=0)
+        ws = (self.w1.weight, self.w2.weight, self.wi.weight)
         inv = self.inv_freq if self.use_rope else None
         theta = self.theta if self.use_givens else None
         bf16 = x.dtype == torch.bfloat16 or (torch.is_autocast_enabled() and
                                              torch.get_autocast_dtype("cuda") == torch.bfloat16)
         if USE_FUSED_PROLOGUE and bf16 and dh in (64, 96, 128) and (H * dh) % 32 == 0:
             norm = (self.p1_norm.weight, self.p2_norm.weight, self.p1_norm.eps) if self.qk_norm else None
-            return qkv_rope(x.to(torch.bfloat16), w.to(torch.bfloat16), H, inv, theta, self.layer_idx, S, norm)
-        qkv = linear_wgrad(x, w)
+            # fp32 master weights: stacked and rounded in one launch, their gradients written in fp32
+            # (three launches fewer than a concatenation, a cast and the cast of dW back)
+            master = all(w.dtype == torch.float32 and w.is_cuda and w.numel() % 8 == 0 for w in ws)
+            w = ws if master else torch.cat(ws, dim=0).to(torch.bfloat16)
+            return _qkv_rope_of(x.to(torch.bfloat16), w, H, inv, theta, self.layer_idx, S, norm)
+        qkv = linear_wgrad(x, torch.cat(ws, dim=0))
         if self.qk_norm:
             q, k, v = qkv.split(D, dim=-1)
             q = self.p1_norm(q.reshape(B, T, H, dh)).reshape(B, T, D)

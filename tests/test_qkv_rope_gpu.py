@@ -357,6 +357,40 @@ def test_out_gate_tilings_agree_bitwise(cuda):
     assert torch.equal(z, torch.cat([z0, z1], 1)) and torch.equal(s, torch.cat([s0, s1], 1))
 
 
+@pytest.mark.parametrize("H,D,T,norm", [(2, 64, 3, False), (4, 64, 130, True), (8, 96, 77, False), (2, 128, 65, True)])
+def test_prologue_from_master_weights(cuda, H, D, T, norm):
+    """mote::qkv_rope_master (three fp32 weights, one of them off a 16-byte boundary) against
+    mote::qkv_rope of their concatenation rounded to bf16: outputs, dx, dtheta and the gains' gradients
+    bit for bit, the weights' fp32 gradients the values whose bf16 rounding is the stacked dW."""
+    from mote_amd import relation as R
+
+    print(f"case master weights H={H} D={D} T={T} norm={norm}", flush=True)
+    g = torch.Generator().manual_seed(T)
+    K = H * D
+    ws = [torch.randn(K, K, generator=g).div(K ** 0.5).to(cuda) for _ in range(3)]
+    ws[1] = torch.empty(K * K + 1, device=cuda)[1:].view(K, K).copy_(ws[1])
+    x = torch.randn(2, T, K, generator=g).bfloat16().to(cuda).requires_grad_(True)
+    theta = (torch.rand(H // 2, generator=g) - 0.5).to(cuda).requires_grad_(True)
+    gains = tuple((1 + 0.1 * torch.randn(D, generator=g)).to(cuda).requires_grad_(True) for _ in range(2)) if norm else ()
+    inv = R.rope_inv_freq(D, 10000.0, cuda)
+    nrm = (*gains, 1e-5) if norm else None
+    dys = [torch.randn(2, H, T, D, generator=g).bfloat16().to(cuda) for _ in range(3)]
+    ws = [w.requires_grad_(True) for w in ws]
+    stack = torch.cat([w.detach() for w in ws]).bfloat16().requires_grad_(True)
+    got = R._qkv_rope_of(x, tuple(ws), H, inv, theta, 1, 5, nrm)
+    ref = R.qkv_rope(x, stack, H, inv, theta, 1, 5, nrm)
+    assert all(torch.equal(a, b) for a, b in zip(got, ref))
+    gg = torch.autograd.grad(got, [x, theta, *gains, *ws], dys)
+    gr = torch.autograd.grad(ref, [x, theta, *gains, stack], dys)
+    n = 2 + len(gains)
+    assert all(torch.equal(a, b) for a, b in zip(gg[:n], gr[:n]))
+    assert all(w.dtype == torch.float32 for w in gg[n:])
+    assert torch.equal(torch.cat(gg[n:]).bfloat16(), gr[n])
+    torch.library.opcheck(torch.ops.mote.qkv_rope_master.default,
+                          (x, *ws, inv, theta, H, 1, 0, True, *(gains if norm else (None, None)), 1e-5),
+                          test_utils=("test_schema", "test_faketensor", "test_autograd_registration"))
+
+
 @pytest.mark.parametrize("shape", [(1, 1, 128), (2, 3, 128), (1, 517, 256)])
 def test_gate_backward_elementwise_bits(cuda, shape):
     """mote::gate_bwd against the eager expressions it replaces, bit for bit: contiguous, transposed and

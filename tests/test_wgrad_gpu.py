@@ -149,3 +149,24 @@ def test_module_weight_gradients_on_wgrad(cuda, monkeypatch, autocast):
         assert got[n].dtype == ref[n].dtype, n
         assert rel_err(got[n], ref[n]) < 1e-2, (n, rel_err(got[n], ref[n]))
     assert rel_err(gx, rx) < 1e-2
+
+
+def test_linear_wgrad_function_under_create_graph(cuda):
+    """linear_wgrad with fp32 weights under autocast: its first gradients carry W's own dtype, and a
+    second differentiation goes through both products and the cast, as through F.linear."""
+    from mote_amd.relation import linear_wgrad
+
+    print("case linear_wgrad create_graph", flush=True)
+    torch.manual_seed(3)
+    x = torch.randn(40, 192, device=cuda, dtype=torch.bfloat16, requires_grad=True)
+    w = (torch.randn(64, 192, device=cuda) / 14).requires_grad_(True)
+
+    def second(fn):
+        with torch.autocast("cuda", torch.bfloat16):
+            y = fn(x, w)
+        gx, gw = torch.autograd.grad(y.float().square().sum(), (x, w), create_graph=True)
+        assert gx.dtype == torch.bfloat16 and gw.dtype == torch.float32
+        return torch.autograd.grad(gx.float().square().sum() + gw.square().sum(), (x, w))
+
+    for a, b in zip(second(linear_wgrad), second(torch.nn.functional.linear)):
+        assert a.dtype == b.dtype and rel_err(a, b) < 2e-2, rel_err(a, b)
