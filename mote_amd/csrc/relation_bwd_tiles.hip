@@ -45,10 +45,11 @@ __device__ __forceinline__ int lane_of(int li, int lg) { return 16 * lg + li; }
 // of one transposed read over the banks.
 __device__ __forceinline__ int dut_pos(int L) { return L ^ (((L >> 4) & 3) << 2); }
 
-__device__ __forceinline__ void store_dut(const Elem<bf16_t>::Frag (&au)[2], bf16_t* dst, int lane) {
+template <int KT>
+__device__ __forceinline__ void store_dut(const Elem<bf16_t>::Frag (&au)[KT], bf16_t* dst, int lane) {
   const int off = dut_pos(lane) * 8;
-  *reinterpret_cast<bf16x8*>(dst + off) = au[0].v;
-  *reinterpret_cast<bf16x8*>(dst + 512 + off) = au[1].v;
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) *reinterpret_cast<bf16x8*>(dst + 512 * kt + off) = au[kt].v;
 }
 
 // The dQ product's B fragment of query tile qt from the 2 KB that one key-kernel wave stored (staged
@@ -64,9 +65,10 @@ __device__ __forceinline__ Elem<bf16_t>::Frag dut_frag(const bf16_t* reg, int qt
   return f;
 }
 
+template <int KT>
 __device__ __forceinline__ void store_dut_zero(bf16_t* dst, int lane) {
 #pragma unroll
-  for (int kt = 0; kt < 2; ++kt) *reinterpret_cast<bf16x8*>(dst + kt * 512 + lane * 8) = bf16x8{};
+  for (int kt = 0; kt < KT; ++kt) *reinterpret_cast<bf16x8*>(dst + kt * 512 + lane * 8) = bf16x8{};
 }
 
 // The fused launch (bwd_kvq_kernel) stores dU write-through: buffer stores with the SC1 cache-policy
@@ -97,11 +99,21 @@ __device__ __forceinline__ void store_dut_zero_wt(__amdgpu_buffer_rsrc_t rs, uin
 // ------------------------------------------------------------------------------------------------
 // key-stationary kernel: dP2 and dI~
 // ------------------------------------------------------------------------------------------------
-template <int DP, bool MASKED, bool WT>
+// The wave's P2 / I~ fragments when they stay in registers for the whole walk (one key tile a wave).
+template <int DP, int KT>
+struct KvRegs {};
+template <int DP>
+struct KvRegs<DP, 1> {
+  Elem<bf16_t>::Frag k[DP / 32], v[DP / 32];
+};
+
+// KT: the wave's 16-key tiles, keys kc .. kc + 16 KT - 1 of the block.
+template <int DP, bool MASKED, bool WT, int KT>
 __device__ __forceinline__ void kv_block(const bf16_t* Qs, const bf16_t* Ds, const float* Ss, const bf16_t* Ks,
-                                         const bf16_t* Vs, f32x4 (&dvacc)[2][DP / 16], f32x4 (&dkacc)[2][DP / 16],
-                                         bf16_t* dut_w, __amdgpu_buffer_rsrc_t rs, uint32_t dut_b, int qh, int kh,
-                                         int li, int lg, int key0, int qa0, float nc2) {
+                                         const bf16_t* Vs, f32x4 (&dvacc)[KT][DP / 16], f32x4 (&dkacc)[KT][DP / 16],
+                                         bf16_t* dut_w, __amdgpu_buffer_rsrc_t rs, uint32_t dut_b, int qh, int kc,
+                                         int li, int lg, int key0, int qa0, float nc2,
+                                         const KvRegs<DP, KT>& kr) {
   using E = Elem<bf16_t>;
   using Frag = E::Frag;
   constexpr int KS = DP / 32, DT = DP / 16;
@@ -116,21 +128,26 @@ __device__ __forceinline__ void kv_block(const bf16_t* Qs, const bf16_t* Ds, con
     lv[4 * qt] = l4.x; lv[4 * qt + 1] = l4.y; lv[4 * qt + 2] = l4.z; lv[4 * qt + 3] = l4.w;
     c4[qt] = f32x4{cq.x, cq.y, cq.z, cq.w};
   }
-  f32x4 sacc[2][2], wacc[2][2];  // [query tile][key tile]
+  f32x4 sacc[2][KT], wacc[2][KT];  // [query tile][key tile]
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt)
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
+    for (int kt = 0; kt < KT; ++kt) {
       sacc[qt][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
       wacc[qt][kt] = c4[qt];
     }
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
-    Frag kf[2], vf[2];  // the wave's keys as B fragments (k = head dim, column = key)
+    Frag kf[KT], vf[KT];  // the wave's keys as B fragments (k = head dim, column = key)
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      kf[kt] = tile_row_frag<DP>(Ks, 32 * kh + 16 * kt + li, 4 * ks + lg);
-      vf[kt] = tile_row_frag<DP>(Vs, 32 * kh + 16 * kt + li, 4 * ks + lg);
+    for (int kt = 0; kt < KT; ++kt) {
+      if constexpr (KT == 1) {
+        kf[kt] = kr.k[ks];
+        vf[kt] = kr.v[ks];
+      } else {
+        kf[kt] = tile_row_frag<DP>(Ks, kc + 16 * kt + li, 4 * ks + lg);
+        vf[kt] = tile_row_frag<DP>(Vs, kc + 16 * kt + li, 4 * ks + lg);
+      }
     }
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
@@ -138,19 +155,19 @@ __device__ __forceinline__ void kv_block(const bf16_t* Qs, const bf16_t* Ds, con
       const Frag aq = tile_row_frag<DP>(Qs, row, 4 * ks + lg);
       const Frag ad = tile_row_frag<DP>(Ds, row, 4 * ks + lg);
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
+      for (int kt = 0; kt < KT; ++kt) {
         sacc[qt][kt] = E::mma(aq, kf[kt], sacc[qt][kt]);
         wacc[qt][kt] = E::mma(ad, vf[kt], wacc[qt][kt]);
       }
     }
   }
-  // rows 32 qh + 16 qt + 4 lg + r; key 16 kt + li of the wave's half. The elementwise chain runs
+  // rows 32 qh + 16 qt + 4 lg + r; key 16 kt + li of the wave's keys. The elementwise chain runs
   // phase by phase over the 8 elements of one key tile (two query tiles), so each transcendental's
   // result is consumed 8 instructions later instead of by the next one.
-  Frag aw[2], au[2];
-  float wv[2][8], uv[2][8];
+  Frag aw[KT], au[KT];
+  float wv[KT][8], uv[KT][8];
 #pragma unroll
-  for (int kt = 0; kt < 2; ++kt) {
+  for (int kt = 0; kt < KT; ++kt) {
     float t[8], sg[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) t[e] = sacc[e >> 2][kt][e & 3] * nc2;  // -U log2e
@@ -191,7 +208,7 @@ __device__ __forceinline__ void kv_block(const bf16_t* Qs, const bf16_t* Ds, con
     if constexpr (WT)
       store_dut_wt(au, rs, dut_b, lane_of(li, lg));
     else
-      store_dut(au, dut_w, lane_of(li, lg));
+      store_dut<KT>(au, dut_w, lane_of(li, lg));
   }
 }
 
@@ -202,14 +219,16 @@ struct KvShape {
   static constexpr int LDS = 2 * STAGE + 2 * TILE;  // two stages, then the job's 64 P2 rows and 64 I~ rows
 };
 
-// The key work of one (batch x head) bh and key block kb: 64 keys, 4 waves. FUSED (the fused launch):
+// The key work of one (batch x head) bh and key block kb: 64 keys by NW waves. Wave w takes query half
+// w / NKW and the w % NKW-th of NKW = NW / 2 parts of the keys. FUSED (the fused launch, four waves):
 // the query blocks are walked from the last down, so the pairs of the longest query blocks are stored
 // first, and the dU quadrants of each query block are counted in the kvq counts once stored.
 // PAD: head dims below DP (p.D, a multiple of 8): the key tiles' columns past D are zeroed in LDS and the
 // dI-bar rows' are zero in memory, so the staged copies in the query tile stay out of U and dW; gradient
 // columns past D are not stored.
-template <int DP, bool FUSED, bool PAD>
+template <int DP, int NW, bool FUSED, bool PAD>
 __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const int kb, bf16_t* smem) {
+  static_assert(NW == 4 || (NW == 8 && !FUSED), "the fused launch runs four-wave jobs");
   using E = Elem<bf16_t>;
   using Frag = E::Frag;
   using S = KvShape<DP>;
@@ -219,7 +238,8 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: staging in scalar registers
   const int li = lane & 15, lg = lane >> 4;
-  const int kh = wave & 1, qh = wave >> 1;
+  constexpr int NKW = NW / 2, KT = 4 / NKW;  // waves along the keys, 16-key tiles a wave
+  const int kw = wave & (NKW - 1), qh = wave >> (NW == 8 ? 2 : 1);
   const int b = bh / p.H, h = bh % p.H;
   const int k0 = kb * 64;
   const int nqb = p.TQp / 64;
@@ -229,10 +249,10 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
   const bf16_t* dbase = reinterpret_cast<const bf16_t*>(p.wdib) + int64_t(bh) * p.TQp * DP;
   const float* sbase = p.stat + int64_t(bh) * nqb * 128;
 
-  const int key0 = k0 + 32 * kh;
-  f32x4 dvacc[2][DT], dkacc[2][DT];
+  const int kc = 16 * KT * kw, key0 = k0 + kc;
+  f32x4 dvacc[KT][DT], dkacc[KT][DT];
 #pragma unroll
-  for (int kt = 0; kt < 2; ++kt)
+  for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       dvacc[kt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -241,7 +261,7 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
 
   const bf16_t* srcs[2] = {qbase, dbase};
   const int64_t strides[2] = {p.q_sr, DP};
-  TileStager<DP, 4, 2, PAD> st;
+  TileStager<DP, NW, 2, PAD> st;
   const int qdims[2] = {p.D, DP};
   st.init(wave, lane, strides, qdims);
   auto issue = [&](int qb, int stage) {
@@ -258,9 +278,9 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
   // PairTable::offset(qb) for the block in hand, moved by qb + A per block (offset(qb + 1) - offset(qb))
   const int pair_a = (p.q_start + 126) / 64;
   int64_t pair_off = PairTable::offset(qb_first, p.q_start);
-  // dU of this key block: pair (qb, kb) at PairTable::offset(qb) + kb, 8 KB per pair; wave (kh, qh)
-  // writes its 2 KB at (kh * 4 + 2 qh) * 512 elements (store_dut)
-  const int wq_off = (kh * 4 + 2 * qh) * 512;
+  // dU of this key block: pair (qb, kb) at PairTable::offset(qb) + kb, 8 KB per pair: key half kh and
+  // query half qh at (kh * 4 + 2 qh) * 512 elements, its two key tiles 512 apart (store_dut)
+  const int wq_off = KT == 2 ? (kw * 4 + 2 * qh) * 512 : ((kw >> 1) * 4 + 2 * qh + (kw & 1)) * 512;
   bf16_t* dut_bh = reinterpret_cast<bf16_t*>(p.dut) + int64_t(bh) * p.npairs * 4096 + wq_off;
   // FUSED: the (batch x head)'s pairs as one buffer (the host keeps it below 2^31 bytes)
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
@@ -270,7 +290,7 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
     // the key rows once (rows past the keys: finite copies whose results are never stored)
     const bf16_t* ksrc[2] = {kbase, vbase};
     const int64_t kstr[2] = {p.k_sr, p.v_sr};
-    TileStager<DP, 4, 2, PAD> kst;
+    TileStager<DP, NW, 2, PAD> kst;
     const int kdims[2] = {p.D, p.D};
     kst.init(wave, lane, kstr, kdims);
     kst.issue(kvs, ksrc, kstr, k0, p.TK - 1, wave, lane);
@@ -280,11 +300,19 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
   __syncthreads();
   if constexpr (PAD) {
     const int nc = CPR - p.D / 8;  // chunks past D of a row, in both tiles
-    for (int q = tid; q < 128 * nc; q += 256) {
+    for (int q = tid; q < 128 * nc; q += 64 * NW) {
       const int row = (q / nc) & 63, c = p.D / 8 + q % nc;
       *reinterpret_cast<bf16x8*>(kvs + q / nc / 64 * TILE + row * DP + (c ^ tile_swz<DP>(row)) * 8) = bf16x8{};
     }
     __syncthreads();
+  }
+  KvRegs<DP, KT> kr;
+  if constexpr (KT == 1) {
+#pragma unroll
+    for (int ks = 0; ks < DP / 32; ++ks) {
+      kr.k[ks] = tile_row_frag<DP>(kvs, kc + li, 4 * ks + lg);
+      kr.v[ks] = tile_row_frag<DP>(kvs + TILE, kc + li, 4 * ks + lg);
+    }
   }
   // FUSED: the count of a block's four dU quadrants is one atomic add by wave 0, issued right after
   // the transfers two blocks later: the waits of the next two blocks leave it in flight, so it costs
@@ -319,24 +347,24 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
     pair_off += FUSED ? -int64_t(qb - 1 + pair_a) : int64_t(qb + pair_a);  // PairTable::offset(qn)
     // quadrant visible at all (some key < some query position), and not wholly padding rows
     if (i0 < p.TQ && key0 < qa0 + 31)
-      kv_block<DP, decltype(masked)::value, FUSED>(Qs, Ds, Ss, kvs, kvs + TILE, dvacc, dkacc, dut_w, rs, dut_b, qh,
-                                                   kh, li, lg, key0, qa0, nc2);
+      kv_block<DP, decltype(masked)::value, FUSED, KT>(Qs, Ds, Ss, kvs, kvs + TILE, dvacc, dkacc, dut_w, rs, dut_b,
+                                                       qh, kc, li, lg, key0, qa0, nc2, kr);
     else if (dut_w) {
       if constexpr (FUSED)
         store_dut_zero_wt(rs, dut_b, lane);
       else
-        store_dut_zero(dut_w, lane);
+        store_dut_zero<KT>(dut_w, lane);
     }
     MOTE_STAMP(2, n);
-    // The next block's transfers were issued before this block's two dU^T stores (and the count's
+    // The next block's transfers were issued before this block's KT dU^T stores (and the count's
     // add), and vector-memory operations retire in issue order: waiting until at most those are
     // outstanding means the transfers have landed, while the stores stay in flight across the
     // barrier. Everything issued before the transfers has completed too: the previous block's stores.
     if (dut_w) {
       if (sig)
-        __builtin_amdgcn_s_waitcnt(kVmWaitStage<3>());
+        __builtin_amdgcn_s_waitcnt(kVmWaitStage<KT + 1>());
       else
-        __builtin_amdgcn_s_waitcnt(kVmWaitStage<2>());
+        __builtin_amdgcn_s_waitcnt(kVmWaitStage<KT>());
     } else {
       if (sig)
         __builtin_amdgcn_s_waitcnt(kVmWaitStage<1>());
@@ -374,12 +402,12 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
   __syncthreads();
   if (qh == 1) {
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int row = 32 * kh + 16 * kt + 4 * lg + r, col = 16 * dt + li;
+          const int row = kc + 16 * kt + 4 * lg + r, col = 16 * dt + li;
           R[row * DP + col] = dvacc[kt][dt][r];
           R[64 * DP + row * DP + col] = dkacc[kt][dt][r];
         }
@@ -387,12 +415,12 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
   __syncthreads();
   if (qh == 0) {
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int row = 32 * kh + 16 * kt + 4 * lg + r, col = 16 * dt + li;
+          const int row = kc + 16 * kt + 4 * lg + r, col = 16 * dt + li;
           R[row * DP + col] += dvacc[kt][dt][r];
           R[64 * DP + row * DP + col] += dkacc[kt][dt][r];
         }
@@ -402,7 +430,7 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
   const bf16_t* dybase = reinterpret_cast<const bf16_t*>(p.dy) + b * p.y_sb + h * p.y_sh;
   bf16_t* dkout = reinterpret_cast<bf16_t*>(p.dp2) + b * p.dk_sb + h * p.dk_sh;
   bf16_t* dvout = reinterpret_cast<bf16_t*>(p.dinfo) + b * p.dv_sb + h * p.dv_sh;
-  for (int item = tid; item < 64 * CPR; item += 256) {
+  for (int item = tid; item < 64 * CPR; item += 64 * NW) {
     const int row = item / CPR, d0 = (item % CPR) * 8;
     const int j = k0 + row;
     if (j >= p.TK || (PAD && d0 >= p.D)) continue;
@@ -434,12 +462,21 @@ __device__ __forceinline__ void kv_job(const BwdParams& p, const int bh, const i
   }
 }
 
+// Waves of a key workgroup of the two-launch form: four, two workgroups a CU; at dh 128 the tiles leave room
+// for one (99 KB of LDS) and the accumulators of 32 keys a wave took 342 registers (one wave a SIMD), so
+// eight waves of 16 keys: two waves a SIMD, one's exponentials beside the other's products, and each
+// wave's P2 / I~ fragments in registers for its whole walk. Backward at B 4, H 8, T 4096: 724 us with four
+// waves, 709 with eight, 673 with the fragments in registers too (LDS reads bound the block: 256 KB of
+// row and transposed fragments against 1031 cycles of products).
+template <int DP>
+constexpr int kKvWaves = DP <= 96 ? 4 : 8;
+
 template <int DP, bool PAD>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DP <= 96 ? 2 : 1)))
+__global__ void __launch_bounds__(64 * kKvWaves<DP>) __attribute__((amdgpu_waves_per_eu(2)))
 bwd_kv_kernel(const BwdParams p) {
   __shared__ __align__(16) bf16_t smem[KvShape<DP>::LDS];
   const int BH = p.B * p.H;
-  kv_job<DP, false, PAD>(p, blockIdx.x % BH, blockIdx.x / BH, smem);  // key block 0 sees the most queries: longest first
+  kv_job<DP, kKvWaves<DP>, false, PAD>(p, blockIdx.x % BH, blockIdx.x / BH, smem);  // key block 0 sees the most queries: longest first
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -714,7 +751,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
     const int job = __builtin_amdgcn_readfirstlane(s_job);
     if (job >= nkey + nqj) break;
     if (job < nkey) {
-      kv_job<DP, true, PAD>(q, queue + nq * (job % hq), job / hq, lds);
+      kv_job<DP, 4, true, PAD>(q, queue + nq * (job % hq), job / hq, lds);
     } else {
       const int j = job - nkey;
       dq_job<DP, 4, true, PAD>(q, queue + nq * (j % hq), nqb - 1 - j / hq, lds);
@@ -775,7 +812,7 @@ static void launch_tiles_dp(const BwdParams& p, int stages, hipStream_t stream) 
   }
   if (stages & MOTE_BWD_KEYS) {
     const int nkb = (p.TK + 63) / 64;
-    hipLaunchKernelGGL((bwd_kv_kernel<DP, PAD>), dim3(nkb * BH), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((bwd_kv_kernel<DP, PAD>), dim3(nkb * BH), dim3(64 * kKvWaves<DP>), 0, stream, p);
   }
   if (stages & MOTE_BWD_QUERIES) {
     const int npq = (p.TQp / 64 + 1) / 2;  // query-block pairs
