@@ -372,6 +372,9 @@ typedef struct mote_qkv_rope_args {
 
 size_t mote_qkv_rope_workspace(const mote_qkv_rope_args* args);
 int mote_qkv_rope_fwd(const mote_qkv_rope_args* args, void* stream);
+/* The same with the three weights apart: args->w is w1, all [H D, H D] with row stride w_sr (nothing is
+ * concatenated). D = 48 is served too, without QK-Norm. */
+int mote_qkv_rope_parts_fwd(const mote_qkv_rope_args* args, const void* w2, const void* wi, void* stream);
 
 /* ------------------------------------------------------------------------------------------------
  * Backward of QK-Norm for the fused prologue (bf16).

@@ -265,6 +265,7 @@ EXPORTS = {
     "mote_add_rms_norm_bwd": ([C.POINTER(NormBwdArgs), C.c_void_p], C.c_int),
     "mote_qkv_rope_workspace": ([C.POINTER(QkvRopeArgs)], C.c_size_t),
     "mote_qkv_rope_fwd": ([C.POINTER(QkvRopeArgs), C.c_void_p], C.c_int),
+    "mote_qkv_rope_parts_fwd": ([C.POINTER(QkvRopeArgs), C.c_void_p, C.c_void_p, C.c_void_p], C.c_int),
     "mote_gate_product": ([C.POINTER(GateProductArgs), C.c_void_p], C.c_int),
     "mote_pack_weights": ([C.POINTER(PackWeightsArgs), C.c_void_p], C.c_int),
     "mote_gate_bwd": ([C.POINTER(GateBwdArgs), C.c_void_p], C.c_int),
@@ -360,7 +361,8 @@ def view(t: torch.Tensor) -> View:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream of t's device as a raw handle (without the Stream object around it)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def ptr(t) -> int:

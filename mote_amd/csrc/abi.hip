@@ -30,6 +30,7 @@ int check_launch(const char* what) {
 size_t wgrad_workspace_bytes(const mote_wgrad_args* a);
 int launch_wgrad(const mote_wgrad_args* a, hipStream_t stream);
 size_t linear_wgrad_workspace_bytes(const mote_linear_wgrad_args* a);
+int launch_qkv_rope_parts_fwd(const mote_qkv_rope_args* a, const void* w2, const void* wi, hipStream_t stream);
 int launch_linear_wgrad(const mote_linear_wgrad_args* a, hipStream_t stream);
 
 }  // namespace mote
@@ -102,6 +103,11 @@ int mote_add_rms_norm_bwd(const mote_add_rms_norm_bwd_args* args, void* stream) 
 
 size_t mote_qkv_rope_workspace(const mote_qkv_rope_args* args) {
   return args ? mote::qkv_rope_workspace_bytes(args) : 0;
+}
+
+int mote_qkv_rope_parts_fwd(const mote_qkv_rope_args* args, const void* w2, const void* wi, void* stream) {
+  mote::g_err[0] = 0;
+  return mote::launch_qkv_rope_parts_fwd(args, w2, wi, reinterpret_cast<hipStream_t>(stream));
 }
 
 int mote_qkv_rope_fwd(const mote_qkv_rope_args* args, void* stream) {

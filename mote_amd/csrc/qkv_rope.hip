@@ -2,7 +2,7 @@
 // x [w1; w2; wi]^T with RoPE on p1 / p2 and the Givens head-pair rotation on I~ in its epilogue,
 // written straight into the [B, T, H, dh] layout the Relation kernels and the arena read.
 //
-// Product. C^T = W X^T on v_mfma_f32_16x16x32_bf16: a workgroup (4 waves at dh 64 / 96, 8 at dh 128)
+// Product. C^T = W X^T on v_mfma_f32_16x16x32_bf16: a workgroup (4 waves at dh 48 / 64 / 96, 8 at dh 128)
 // owns 32 tokens per wave and the 2 dh output features of one head pair of one projection (p1, p2:
 // heads 2k, 2k+1; I~: the Givens pair of the layer's parity, (2k, 2k+1) or (2k+1, 2k+2 mod H)). Wave
 // w holds head (w & 1) for tokens 64 (w >> 1) .. +63: dh/16 x 4 accumulator tiles, features in the
@@ -42,7 +42,7 @@ constexpr int kQkvPad = 8;       // bf16 elements of padding per output-tile row
 
 struct QkvParams {
   const bf16_t* x; int64_t x_sr;           // [M, K] token rows (M = B * T)
-  const bf16_t* w; int64_t w_sr;           // [3 H dh, K]
+  const bf16_t* w[3]; int64_t w_sr;        // the weights of p1, p2 and I~, [H dh, K] each (gate mode: the first)
   const uint32_t* tab;                     // [T][dh / 2] bf16 cos | bf16 sin << 16, or null (no RoPE)
   const float* theta;                      // [H / 2] or null (no Givens)
   bf16_t* o1; int64_t o1_sb, o1_sh, o1_sr;
@@ -111,9 +111,8 @@ qkv_rope_kernel(const QkvParams p) {
     h0 = 2 * hp + 1;
     h1 = (2 * hp + 2) % p.H;
   }
-  const int HD = p.H * DH;
-  const bf16_t* wb0 = p.w + int64_t(part * HD + h0 * DH) * p.w_sr;
-  const bf16_t* wb1 = p.w + int64_t(part * HD + h1 * DH) * p.w_sr;
+  const bf16_t* wb0 = p.w[part] + int64_t(h0 * DH) * p.w_sr;
+  const bf16_t* wb1 = p.w[part] + int64_t(h1 * DH) * p.w_sr;
   const bf16_t* xb = p.x + int64_t(r0) * p.x_sr;
   const bool full = r0 + S::TOK <= p.M;
 
@@ -406,10 +405,28 @@ static bool al16v(const void* ptr, int64_t s0, int64_t s1, int64_t s2) {
          (s2 * 2) % 16 == 0;
 }
 
+static int launch_qkv(const mote_qkv_rope_args* a, const void* w2, const void* wi, hipStream_t stream);
+
 int launch_qkv_rope_fwd(const mote_qkv_rope_args* a, hipStream_t stream) {
   if (!a) return set_error(MOTE_ERR_ARGUMENT, "qkv_rope: null args");
   if (a->D != 64 && a->D != 96 && a->D != 128)
     return set_error(MOTE_ERR_SHAPE, "qkv_rope: head dim %d (the fused prologue serves 64, 96, 128)", a->D);
+  const bf16_t* w = reinterpret_cast<const bf16_t*>(a->w);
+  const int64_t part = int64_t(a->H) * a->D * a->w_sr;  // elements of one projection's weight
+  return launch_qkv(a, w ? w + part : w, w ? w + 2 * part : w, stream);
+}
+
+int launch_qkv_rope_parts_fwd(const mote_qkv_rope_args* a, const void* w2, const void* wi, hipStream_t stream) {
+  if (!a) return set_error(MOTE_ERR_ARGUMENT, "qkv_rope_parts: null args");
+  if (a->D != 48 && a->D != 64 && a->D != 96 && a->D != 128)
+    return set_error(MOTE_ERR_SHAPE, "qkv_rope_parts: head dim %d (48, 64, 96 or 128)", a->D);
+  if (a->D == 48 && a->norm_w1)
+    return set_error(MOTE_ERR_SHAPE, "qkv_rope_parts: QK-Norm needs a head dim of 64, 96 or 128");
+  return launch_qkv(a, w2, wi, stream);
+}
+
+// a->w: the first projection's weight.
+static int launch_qkv(const mote_qkv_rope_args* a, const void* w2, const void* wi, hipStream_t stream) {
   if (a->B < 0 || a->T < 0 || a->H < 2 || a->H % 2)
     return set_error(MOTE_ERR_SHAPE, "qkv_rope: B = %d, T = %d, H = %d (H even)", a->B, a->T, a->H);
   const int K = a->H * a->D;
@@ -417,13 +434,13 @@ int launch_qkv_rope_fwd(const mote_qkv_rope_args* a, hipStream_t stream) {
   const int64_t M = int64_t(a->B) * a->T;
   if (M == 0) return MOTE_OK;
   if (M > (int64_t(1) << 30)) return set_error(MOTE_ERR_SHAPE, "qkv_rope: %lld tokens", (long long)M);
-  if (!a->x || !a->w || !a->p1.data || !a->p2.data || !a->info.data)
+  if (!a->x || !a->w || !w2 || !wi || !a->p1.data || !a->p2.data || !a->info.data)
     return set_error(MOTE_ERR_ARGUMENT, "qkv_rope: null pointer");
   if (a->B > 1 && a->x_sb != int64_t(a->T) * a->x_sr)
     return set_error(MOTE_ERR_ARGUMENT, "qkv_rope: x must hold its batches back to back (x_sb == T * x_sr)");
   if (a->x_sr >= (int64_t(1) << 23) || a->w_sr >= (int64_t(1) << 23))
     return set_error(MOTE_ERR_ARGUMENT, "qkv_rope: row strides must stay below 2^23 elements");
-  if (!al16v(a->x, a->x_sr, 0, 0) || !al16v(a->w, a->w_sr, 0, 0) ||
+  if (!al16v(a->x, a->x_sr, 0, 0) || !al16v(a->w, a->w_sr, 0, 0) || !al16v(w2, 0, 0, 0) || !al16v(wi, 0, 0, 0) ||
       !al16v(a->p1.data, a->p1.stride_b, a->p1.stride_h, a->p1.stride_r) ||
       !al16v(a->p2.data, a->p2.stride_b, a->p2.stride_h, a->p2.stride_r) ||
       !al16v(a->info.data, a->info.stride_b, a->info.stride_h, a->info.stride_r) ||
@@ -437,7 +454,9 @@ int launch_qkv_rope_fwd(const mote_qkv_rope_args* a, hipStream_t stream) {
     return set_error(MOTE_ERR_WORKSPACE, "qkv_rope: workspace too small or misaligned");
   QkvParams p;
   p.x = reinterpret_cast<const bf16_t*>(a->x); p.x_sr = a->x_sr;
-  p.w = reinterpret_cast<const bf16_t*>(a->w); p.w_sr = a->w_sr;
+  p.w[0] = reinterpret_cast<const bf16_t*>(a->w); p.w_sr = a->w_sr;
+  p.w[1] = reinterpret_cast<const bf16_t*>(w2);
+  p.w[2] = reinterpret_cast<const bf16_t*>(wi);
   p.tab = a->inv_freq ? reinterpret_cast<const uint32_t*>(a->workspace) : nullptr;
   p.theta = a->theta;
   p.o1 = reinterpret_cast<bf16_t*>(a->p1.data); p.o1_sb = a->p1.stride_b; p.o1_sh = a->p1.stride_h; p.o1_sr = a->p1.stride_r;
@@ -458,6 +477,7 @@ int launch_qkv_rope_fwd(const mote_qkv_rope_args* a, hipStream_t stream) {
     if (rc) return rc;
   }
   switch (a->D) {
+    case 48: launch_qkv_kernel<48, false>(p, M, stream); break;
     case 64: launch_qkv_kernel<64, false>(p, M, stream); break;
     case 96: launch_qkv_kernel<96, false>(p, M, stream); break;
     default: launch_qkv_kernel<128, false>(p, M, stream); break;
@@ -491,7 +511,7 @@ int launch_gate_product(const mote_gate_product_args* a, hipStream_t stream) {
     return set_error(MOTE_ERR_ARGUMENT, "gate_product: rows must start on 16-byte boundaries");
   QkvParams p = {};
   p.x = reinterpret_cast<const bf16_t*>(a->x); p.x_sr = a->x_sr;
-  p.w = reinterpret_cast<const bf16_t*>(a->w); p.w_sr = a->w_sr;
+  p.w[0] = reinterpret_cast<const bf16_t*>(a->w); p.w_sr = a->w_sr;
   p.gy = reinterpret_cast<const bf16_t*>(a->y); p.gy_sr = a->y_sr;
   p.gz = reinterpret_cast<bf16_t*>(a->z); p.gs = reinterpret_cast<bf16_t*>(a->s); p.gz_sr = a->z_sr;
   p.B = 1; p.T = int(M); p.H = a->D / DH; p.K = a->D; p.M = int(M); p.parity = 0; p.nk = a->D / kQkvK;

@@ -217,7 +217,7 @@ def _rope_table_ws(a, x: torch.Tensor, inv: Optional[torch.Tensor], cacheable: b
     n = max(int(L.lib().mote_qkv_rope_workspace(a)), 16)
     if inv is None or not cacheable:
         return torch.empty(n, device=x.device, dtype=torch.uint8), 0
-    key = (x.device, torch.cuda.current_stream(x.device).cuda_stream, inv.data_ptr(), a.T, a.pos0, a.D)
+    key = (x.device, L.stream_of(x), inv.data_ptr(), a.T, a.pos0, a.D)
     hit = _ROPE_TABLES.get(key)
     # the entry holds the frequency tensor itself: its memory cannot be recycled for another tensor
     # while the entry lives, and an in-place change of it shows in its version counter
@@ -236,7 +236,9 @@ def _rope_table_ws(a, x: torch.Tensor, inv: Optional[torch.Tensor], cacheable: b
     return ws, 0
 
 
-def _qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps):
+def _qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps, into=None):
+    """The prologue's launch for a stacked bf16 weight or a tuple of the three; `into`: (P2, I~) views
+    [B, H, T, dh] to write instead of new tensors."""
     if not x.is_cuda:
         raise RuntimeError("mote::qkv_rope needs the HIP library and an MI355X")
     B, T, K = x.shape
@@ -246,14 +248,16 @@ def _qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, no
     if norm != (norm_w2 is not None):
         raise ValueError("mote::qkv_rope: QK-Norm needs both gains")
     x = x.contiguous()
-    w = w.contiguous()
-    p1, p2, info = (_heads_out(B, T, H, D, x, x.dtype) for _ in range(3))
+    apart = isinstance(w, tuple)
+    ws = tuple(t if t.data_ptr() % 16 == 0 else t.clone() for t in (t.contiguous() for t in w)) if apart else (w.contiguous(),)
+    p1 = _heads_out(B, T, H, D, x, x.dtype)
+    p2, info = into if into is not None else (_heads_out(B, T, H, D, x, x.dtype) for _ in range(2))
     iraw = torch.empty(B, T, K, device=x.device, dtype=x.dtype) if keep_info else x.new_empty(0)
     qkraw = torch.empty(B, T, 2 * K, device=x.device, dtype=x.dtype) if (keep_info and norm) else x.new_empty(0)
     a = L.QkvRopeArgs()
     a.B, a.T, a.H, a.D, a.pos0, a.layer_parity = B, T, H, D, int(pos0), int(parity)
     a.x, a.x_sb, a.x_sr = x.data_ptr(), x.stride(0), x.stride(1)
-    a.w, a.w_sr = w.data_ptr(), w.stride(0)
+    a.w, a.w_sr = ws[0].data_ptr(), K
     inv = None if inv_freq is None else inv_freq.to(device=x.device, dtype=torch.float32).contiguous()
     th = None if theta is None else theta.detach().to(device=x.device, dtype=torch.float32).contiguous()
     a.inv_freq, a.theta = L.ptr(inv), L.ptr(th)
@@ -268,9 +272,13 @@ def _qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, no
         a.norm_w1, a.norm_w2, a.norm_eps = nw1.data_ptr(), nw2.data_ptr(), float(norm_eps)
         if keep_info:
             a.qk_raw, a.qr_sb, a.qr_sr = qkraw.data_ptr(), qkraw.stride(0), qkraw.stride(1)
-    ws, a.table_ready = _rope_table_ws(a, x, inv, inv is inv_freq)
-    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    L.check(L.lib().mote_qkv_rope_fwd(a, L.stream_of(x)), "mote_qkv_rope_fwd")
+    table, a.table_ready = _rope_table_ws(a, x, inv, inv is inv_freq)
+    a.workspace, a.workspace_bytes = table.data_ptr(), table.numel()
+    if apart:
+        L.check(L.lib().mote_qkv_rope_parts_fwd(a, ws[1].data_ptr(), ws[2].data_ptr(), L.stream_of(x)),
+                "mote_qkv_rope_parts_fwd")
+    else:
+        L.check(L.lib().mote_qkv_rope_fwd(a, L.stream_of(x)), "mote_qkv_rope_fwd")
     return p1, p2, info, iraw, qkraw
 
 
@@ -492,17 +500,11 @@ def _qr_backward(ctx, dp1, dp2, dinfo, _diraw, _dqkraw):
 _qkv_rope.register_autograd(_qr_backward, setup_context=_qr_setup)
 
 
-# ---- mote::qkv_rope_master (the prologue from fp32 master weights) --------------------------------
-@torch.library.custom_op("mote::qkv_rope_master", mutates_args=())
-def _qkv_rope_master(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, wi: torch.Tensor,
-                     inv_freq: Optional[torch.Tensor], theta: Optional[torch.Tensor], n_heads: int, parity: int,
-                     pos0: int, keep_info: bool, norm_w1: Optional[torch.Tensor] = None,
-                     norm_w2: Optional[torch.Tensor] = None, norm_eps: float = 1e-5
-                     ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    """mote::qkv_rope of the bf16 stack of three fp32 weights [H dh, H dh], made in one launch; the stack
-    is the sixth output (kept for the backward's dx)."""
-    if not x.is_cuda:
-        raise RuntimeError("mote::qkv_rope_master needs the HIP library and an MI355X")
+# ---- the prologue from the layer's own three weights -----------------------------------------------
+def _packed(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, wi: torch.Tensor) -> torch.Tensor:
+    """The bf16 stack [w1; w2; wi]: fp32 weights rounded and stacked in one launch, others by torch."""
+    if not all(t.dtype == torch.float32 for t in (w1, w2, wi)) or w1.numel() % 8:
+        return torch.cat([w1, w2, wi], dim=0).to(torch.bfloat16)
     ws = [t if t.data_ptr() % 16 == 0 else t.clone() for t in (w1.contiguous(), w2.contiguous(), wi.contiguous())]
     N, K = w1.shape
     w = torch.empty(3 * N, K, device=x.device, dtype=torch.bfloat16)
@@ -510,27 +512,78 @@ def _qkv_rope_master(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, wi: to
     a.n, a.out = N * K, w.data_ptr()
     a.w0, a.w1, a.w2 = (t.data_ptr() for t in ws)
     L.check(L.lib().mote_pack_weights(a, L.stream_of(x)), "mote_pack_weights")
-    return (*_qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps), w)
+    return w
+
+
+def _bf16_parts(x, w1, w2, wi, keep: bool):
+    """(the three bf16 weights, their stack when it was made): bf16 weights are read where they are
+    unless the backward needs the stack (its dx is one product with it)."""
+    if keep or any(t.dtype != torch.bfloat16 for t in (w1, w2, wi)):
+        w = _packed(x, w1, w2, wi)
+        return tuple(w.chunk(3)), w
+    return (w1, w2, wi), x.new_empty(0)
+
+
+@torch.library.custom_op("mote::qkv_rope_master", mutates_args=())
+def _qkv_rope_master(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, wi: torch.Tensor,
+                     inv_freq: Optional[torch.Tensor], theta: Optional[torch.Tensor], n_heads: int, parity: int,
+                     pos0: int, keep_info: bool, train: bool, norm_w1: Optional[torch.Tensor] = None,
+                     norm_w2: Optional[torch.Tensor] = None, norm_eps: float = 1e-5
+                     ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    """mote::qkv_rope from the layer's weights [H dh, H dh] (fp32 or bf16); with `train` the sixth output is
+    their bf16 stack, kept for the backward's dx (empty otherwise). dh 48 is served too (no QK-Norm)."""
+    if not x.is_cuda:
+        raise RuntimeError("mote::qkv_rope_master needs the HIP library and an MI355X")
+    ws, stack = _bf16_parts(x, w1, w2, wi, train)
+    return (*_qkv_rope_launch(x, ws, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps), stack)
 
 
 @_qkv_rope_master.register_fake
-def _qkv_rope_master_fake(x, w1, w2, wi, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1=None, norm_w2=None,
-                          norm_eps=1e-5):
+def _qkv_rope_master_fake(x, w1, w2, wi, inv_freq, theta, n_heads, parity, pos0, keep_info, train, norm_w1=None,
+                          norm_w2=None, norm_eps=1e-5):
     w = x.new_empty((3 * w1.shape[0], w1.shape[1]))
-    return (*_qkv_rope_fake(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps), w)
+    bf16 = all(t.dtype == torch.bfloat16 for t in (w1, w2, wi))
+    return (*_qkv_rope_fake(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps),
+            x.new_empty(0) if bf16 and not train else w)
 
 
 def _qrm_setup(ctx, inputs, output):
-    x, _w1, _w2, _wi, *rest = inputs
-    _qr_setup(ctx, (x, output[5], *rest), output)
+    x, w1, _w2, _wi, inv_freq, theta, n_heads, parity, pos0, keep_info, train, *norm = inputs
+    _qr_setup(ctx, (x, output[5], inv_freq, theta, n_heads, parity, pos0, keep_info, *norm), output)
+    ctx.w_dtypes = tuple(t.dtype for t in inputs[1:4])
+    ctx.train = train
 
 
 def _qrm_backward(ctx, dp1, dp2, dinfo, _diraw, _dqkraw, _dw):
-    dx, dw, dtheta, dn1, dn2 = _qr_grads(ctx, dp1, dp2, dinfo, torch.float32)
-    return (dx, *dw.chunk(3), None, dtheta, None, None, None, None, dn1, dn2, None)
+    if not ctx.train:
+        raise RuntimeError("mote::qkv_rope_master: the backward needs train=True")
+    wdtype = torch.float32 if torch.float32 in ctx.w_dtypes else None
+    dx, dw, dtheta, dn1, dn2 = _qr_grads(ctx, dp1, dp2, dinfo, wdtype)
+    dws = (d.to(t) for d, t in zip(dw.chunk(3), ctx.w_dtypes))
+    return (dx, *dws, None, dtheta, None, None, None, None, None, dn1, dn2, None)
 
 
 _qkv_rope_master.register_autograd(_qrm_backward, setup_context=_qrm_setup)
+
+
+@torch.library.custom_op("mote::qkv_rope_into", mutates_args=("p2", "info"))
+def _qkv_rope_into(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, wi: torch.Tensor, inv_freq: Optional[torch.Tensor],
+                   theta: Optional[torch.Tensor], n_heads: int, parity: int, pos0: int, p2: torch.Tensor,
+                   info: torch.Tensor, norm_w1: Optional[torch.Tensor] = None, norm_w2: Optional[torch.Tensor] = None,
+                   norm_eps: float = 1e-5) -> torch.Tensor:
+    """mote::qkv_rope_master without a backward, P2 and I~ written into the given bf16 [B, H, T, dh] views
+    (a cache's new rows); returns p1."""
+    if not x.is_cuda:
+        raise RuntimeError("mote::qkv_rope_into needs the HIP library and an MI355X")
+    ws, _ = _bf16_parts(x, w1, w2, wi, False)
+    return _qkv_rope_launch(x, ws, inv_freq, theta, n_heads, parity, pos0, False, norm_w1, norm_w2, norm_eps, (p2, info))[0]
+
+
+@_qkv_rope_into.register_fake
+def _qkv_rope_into_fake(x, w1, w2, wi, inv_freq, theta, n_heads, parity, pos0, p2, info, norm_w1=None, norm_w2=None,
+                        norm_eps=1e-5):
+    B, T, K = x.shape
+    return x.new_empty((B, T, n_heads, K // n_heads)).transpose(1, 2)
 
 
 def qkv_rope(x: torch.Tensor, w: torch.Tensor, n_heads: int, inv_freq: Optional[torch.Tensor],
@@ -539,16 +592,14 @@ def qkv_rope(x: torch.Tensor, w: torch.Tensor, n_heads: int, inv_freq: Optional[
     """The fused prologue: bf16 x [B, T, H dh] and w = [w1; w2; wi] [3 H dh, H dh] -> (p1, p2, I~),
     the same as rope_givens(F.linear(x, w), ...) (relation.py:199-215); `norm` = (p1 gain, p2 gain,
     eps) applies QK-Norm to p1 / p2 first (relation.py:208-210). Differentiable in x, w, theta and
-    the gains."""
-    return _qkv_rope_of(x, w, n_heads, inv_freq, theta, layer_idx, pos0, norm)
-
-
-def _qkv_rope_of(x, w, n_heads, inv_freq, theta, layer_idx, pos0, norm):
-    """qkv_rope for a stacked weight, or for a tuple of the three fp32 weights."""
+    the gains. w may also be the tuple of the three weights, fp32 or bf16 (mote::qkv_rope_master)."""
     n1, n2, eps = norm if norm is not None else (None, None, 1e-5)
-    keep = torch.is_grad_enabled() and (theta is not None or norm is not None)
-    args = (inv_freq, theta, int(n_heads), int(layer_idx) % 2, int(pos0), keep, n1, n2, float(eps))
-    return (_qkv_rope_master(x, *w, *args) if isinstance(w, tuple) else _qkv_rope(x, w, *args))[:3]
+    train = torch.is_grad_enabled()
+    keep = train and (theta is not None or norm is not None)
+    head = (inv_freq, theta, int(n_heads), int(layer_idx) % 2, int(pos0), keep)
+    if isinstance(w, tuple):
+        return _qkv_rope_master(x, *w, *head, train, n1, n2, float(eps))[:3]
+    return _qkv_rope(x, w, *head, n1, n2, float(eps))[:3]
 
 
 # ---- mote::out_gate (the output gate of _out) ----------------------------------------------------
@@ -707,6 +758,16 @@ class FullRelation(nn.Module):
         return out
 
     # ------------------------------------------------------------------------------------------
+    def _fused_prologue(self, bf16: bool) -> bool:
+        """Whether the one-launch prologue serves this layer: bf16 activations, a width of whole 64-column
+        stages, head dim 64 / 96 / 128, or 48 without QK-Norm (the 192-wide layer, 19,856 rows: product
+        and RoPE kernel 20.7 + 13.7 us apart, 20.0 fused)."""
+        if not USE_FUSED_PROLOGUE or not bf16:
+            return False
+        if self.d_head == 48:
+            return self.d_model % 64 == 0 and not self.qk_norm
+        return self.d_head in (64, 96, 128) and self.d_model % 32 == 0
+
     def heads(self, x: torch.Tensor, S: int):
         """Projections -> (QK-Norm) -> RoPE / Givens: (p1, p2, I~) as [B, H, T, dh] views."""
         B, T, D = x.shape
@@ -716,13 +777,12 @@ class FullRelation(nn.Module):
         theta = self.theta if self.use_givens else None
         bf16 = x.dtype == torch.bfloat16 or (torch.is_autocast_enabled() and
                                              torch.get_autocast_dtype("cuda") == torch.bfloat16)
-        if USE_FUSED_PROLOGUE and bf16 and dh in (64, 96, 128) and (H * dh) % 32 == 0:
+        if self._fused_prologue(bf16):
             norm = (self.p1_norm.weight, self.p2_norm.weight, self.p1_norm.eps) if self.qk_norm else None
             # fp32 master weights: stacked and rounded in one launch, their gradients written in fp32
-            # (three launches fewer than a concatenation, a cast and the cast of dW back)
-            master = all(w.dtype == torch.float32 and w.is_cuda and w.numel() % 8 == 0 for w in ws)
-            w = ws if master else torch.cat(ws, dim=0).to(torch.bfloat16)
-            return _qkv_rope_of(x.to(torch.bfloat16), w, H, inv, theta, self.layer_idx, S, norm)
+            # (three launches fewer than a concatenation, a cast and the cast of dW back); bf16
+            # weights: read where they are when there is no backward
+            return qkv_rope(x.to(torch.bfloat16), ws, H, inv, theta, self.layer_idx, S, norm)
         qkv = linear_wgrad(x, torch.cat(ws, dim=0))
         if self.qk_norm:
             q, k, v = qkv.split(D, dim=-1)
@@ -730,6 +790,26 @@ class FullRelation(nn.Module):
             k = self.p2_norm(k.reshape(B, T, H, dh)).reshape(B, T, D)
             qkv = torch.cat([q, k, v], dim=-1)
         return rope_givens(qkv, H, inv, theta, self.layer_idx, S)
+
+    def _heads_into(self, x: torch.Tensor, S: int, cache: ArenaLayer) -> Optional[torch.Tensor]:
+        """heads() with P2 and I~ written straight into the arena's rows [S, S + T) by the prologue's launch
+        (two copies fewer): p1, or None where that does not apply (a backward is wanted, another dtype or
+        batch, a width the fused prologue does not serve, a traced call)."""
+        B, T, _ = x.shape
+        arena = cache.arena
+        bf16 = x.dtype == torch.bfloat16 or (torch.is_autocast_enabled() and
+                                             torch.get_autocast_dtype("cuda") == torch.bfloat16)
+        if (torch.is_grad_enabled() or torch.compiler.is_compiling() or not self._fused_prologue(bf16) or T == 0
+                or arena.dtype != torch.bfloat16 or arena.batch != B or arena.n_heads != self.n_heads
+                or arena.d_head != self.d_head or arena.store.device != x.device or S + T > arena.capacity):
+            return None
+        p2, info = (t[:, :, S: S + T] for t in (arena.p2(cache.layer), arena.info(cache.layer)))
+        if any(t.data_ptr() % 16 or t.stride(3) != 1 or any(st % 8 for st in t.stride()[:3]) for t in (p2, info)):
+            return None
+        n1, n2, eps = (self.p1_norm.weight, self.p2_norm.weight, self.p1_norm.eps) if self.qk_norm else (None, None, 1e-5)
+        return _qkv_rope_into(x.to(torch.bfloat16), self.w1.weight, self.w2.weight, self.wi.weight,
+                              self.inv_freq if self.use_rope else None, self.theta if self.use_givens else None,
+                              self.n_heads, self.layer_idx % 2, S, p2, info, n1, n2, float(eps))
 
     def _out(self, y: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
         """[B, H, T, dh] -> [B, T, D] -> optional output gate -> wo (relation.py:176-182)."""
@@ -755,9 +835,12 @@ class FullRelation(nn.Module):
         B, T, D = x.shape
         arena = isinstance(cache, ArenaLayer)
         S = cache.n if arena else (0 if cache is None else cache[0].shape[2])
-        p1, p2, info = self.heads(x, S)
+        p1 = self._heads_into(x, S, cache) if arena else None
+        if p1 is None:
+            p1, p2, info = self.heads(x, S)
+            if arena:
+                cache.write(p2, info)
         if arena:
-            cache.write(p2, info)
             p2_all, info_all = cache.views(S + T)
         elif cache is not None:
             p2_all = torch.cat([cache[0], p2], dim=2)

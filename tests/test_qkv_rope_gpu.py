@@ -377,7 +377,7 @@ def test_prologue_from_master_weights(cuda, H, D, T, norm):
     dys = [torch.randn(2, H, T, D, generator=g).bfloat16().to(cuda) for _ in range(3)]
     ws = [w.requires_grad_(True) for w in ws]
     stack = torch.cat([w.detach() for w in ws]).bfloat16().requires_grad_(True)
-    got = R._qkv_rope_of(x, tuple(ws), H, inv, theta, 1, 5, nrm)
+    got = R.qkv_rope(x, tuple(ws), H, inv, theta, 1, 5, nrm)
     ref = R.qkv_rope(x, stack, H, inv, theta, 1, 5, nrm)
     assert all(torch.equal(a, b) for a, b in zip(got, ref))
     gg = torch.autograd.grad(got, [x, theta, *gains, *ws], dys)
@@ -387,8 +387,62 @@ def test_prologue_from_master_weights(cuda, H, D, T, norm):
     assert all(w.dtype == torch.float32 for w in gg[n:])
     assert torch.equal(torch.cat(gg[n:]).bfloat16(), gr[n])
     torch.library.opcheck(torch.ops.mote.qkv_rope_master.default,
-                          (x, *ws, inv, theta, H, 1, 0, True, *(gains if norm else (None, None)), 1e-5),
+                          (x, *ws, inv, theta, H, 1, 0, True, True, *(gains if norm else (None, None)), 1e-5),
                           test_utils=("test_schema", "test_faketensor", "test_autograd_registration"))
+
+
+@pytest.mark.parametrize("T,B", [(1, 1), (33, 2), (127, 1), (300, 3)])
+@pytest.mark.parametrize("layer", [0, 1])
+def test_prologue_head_dim_48(cuda, monkeypatch, T, B, layer):
+    """The 192-wide layer (4 heads of 48) under autocast on the fused prologue against the product and the
+    RoPE kernel apart: the same roundings, so outputs and gradients differ by the product's fp32 summation
+    order alone (one bf16 ulp of the projections, 2^-8, through the layer)."""
+    from mote_amd import relation as R
+
+    print(f"case prologue dh48 T={T} B={B} layer={layer}", flush=True)
+    torch.manual_seed(T)
+    m = R.FullRelation(192, 4, layer).to(cuda)
+    with torch.no_grad():
+        m.theta.uniform_(-0.5, 0.5)
+    x = torch.randn(B, T, 192, device=cuda).bfloat16().requires_grad_(True)
+    dy = torch.randn(B, T, 192, device=cuda).bfloat16()
+
+    def step():
+        with torch.autocast("cuda", torch.bfloat16):
+            y = m(x)
+        return [y, *torch.autograd.grad(y, [x, *(p for n, p in m.named_parameters() if n != "lam")], dy)]
+
+    assert m._fused_prologue(True)
+    got = step()
+    monkeypatch.setattr(R, "USE_FUSED_PROLOGUE", False)
+    for a, b in zip(got, step()):
+        assert a.dtype == b.dtype and rel_err(a, b) < 1.6e-2, rel_err(a, b)
+
+
+@pytest.mark.parametrize("S,T,B,norm,dtype", [(0, 1, 1, False, torch.bfloat16), (64, 40, 1, True, torch.bfloat16),
+                                              (100, 129, 2, False, torch.float32)])
+def test_arena_rows_written_by_the_prologue(cuda, S, T, B, norm, dtype):
+    """FullRelation.forward over an arena without gradients, whose prologue writes P2 and I~ into the
+    arena's rows, against the same call with gradients (new tensors, then copies): outputs and the whole
+    arena bit for bit, for bf16 weights read apart and fp32 ones under autocast."""
+    from mote_amd.arena import ArenaState, RelationArena
+    from mote_amd.relation import FullRelation
+
+    print(f"case arena rows S={S} T={T} B={B} norm={norm} {dtype}", flush=True)
+    torch.manual_seed(S + T)
+    m = FullRelation(256, 4, 1, qk_norm=norm).to(device=cuda, dtype=dtype)
+    x = torch.randn(B, T, 256, device=cuda).to(torch.bfloat16)
+    base = torch.randn(1, 2, B, 4, 256, 64, device=cuda).bfloat16()
+    outs = []
+    for grad in (False, True):
+        arena = RelationArena(1, 4, 256, 64, "cuda", torch.bfloat16, batch=B)
+        arena.store.copy_(base)
+        with torch.set_grad_enabled(grad), torch.autocast("cuda", torch.bfloat16, enabled=dtype == torch.float32):
+            assert (m._heads_into(x, S, ArenaState(arena, n=S)[0]) is not None) == (not grad)
+            outs.append((m(x, cache=ArenaState(arena, n=S)[0]).detach(), arena.store))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    with pytest.raises(RuntimeError, match="arena overflow"), torch.no_grad():
+        m(torch.randn(B, 200, 256, device=cuda).bfloat16(), cache=ArenaState(arena, n=100)[0])
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 128), (2, 3, 128), (1, 517, 256)])
