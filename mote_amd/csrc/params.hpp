@@ -19,8 +19,9 @@ struct FwdParams {
   float* g;
   const float* lam;
   const int32_t* cu;  // null in dense mode
-  float* part;        // split partials [nseq][H][nqb][2][64 * DP + 128] (null: no split)
-  int split_c;        // query blocks with more key blocks than this run as two halves
+  float* part;        // split partials [nseq][H][nqb][npart][64 * DP + 128] (null: no split)
+  int split_c;        // query blocks with more key blocks than this run as pieces of at most as many
+  int npart;          // the pieces of the longest query block (1: no split)
   int* jobs;          // persistent tile launch: one job counter per queue, 32 ints apart (null: one job per workgroup)
   int jobs_nq;        // its queue count (heads h go to queue h % jobs_nq)
   int64_t q_sb, q_sh, q_sr;

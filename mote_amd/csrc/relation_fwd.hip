@@ -502,9 +502,14 @@ struct FwdTileShape {
   static constexpr int LDS = NSTG * STAGE;
 };
 
-// One (query block, sequence, head) of the tile forward (or one key-range half of it when split),
-// by its block id (the launch order: head fastest, then (when split) the halves, then query blocks
+// One (query block, sequence, head) of the tile forward (or one piece of its key range when split),
+// by its block id (the launch order: head fastest, then (when split) the pieces, then query blocks
 // longest first); every wave of the workgroup calls it.
+// The pieces of a query block of nkb key blocks.
+__device__ __forceinline__ int fwd_pieces(const FwdParams& p, int nkb) {
+  return p.part != nullptr && nkb > p.split_c ? (nkb + p.split_c - 1) / p.split_c : 1;
+}
+
 // PAD: head dims below DP (p.D, a multiple of 8). The queries' columns past D are zero, which keeps the
 // staged copies there (TileStager) out of the scores; I-bar columns past D are not stored.
 template <int DP, bool PAD>
@@ -521,8 +526,8 @@ __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, 
   const int li = lane & 15, lg = lane >> 4;
   const int kh = wave & 1, qh = wave >> 1;
   const int h = bid % p.H;
-  const int half = p.part ? (bid / p.H) & 1 : 0;
-  const int rest = p.part ? bid / p.H / 2 : bid / p.H;
+  const int piece = p.part ? bid / p.H % p.npart : 0;
+  const int rest = p.part ? bid / p.H / p.npart : bid / p.H;
   const int seq = rest % p.nseq;
   const int qb = p.nqb - 1 - rest / p.nseq;
 
@@ -568,11 +573,11 @@ __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, 
   const int qlast = min(TQs, qb * 64 + 64) - 1;
   const int nkb = (qs + qlast + 63) / 64;       // keys j < qs + qlast
   const int wq_last = min(q0 + 31, TQs - 1);    // the wave's last query row
-  // long query blocks run as two workgroups over the two halves of their key blocks
-  const bool split = p.part != nullptr && nkb > p.split_c;
-  if (half == 1 && !split) return;
-  const int kb_mid = split ? (nkb + 1) / 2 : nkb;
-  const int kb_lo = half ? kb_mid : 0, kb_hi = half ? nkb : kb_mid;
+  // long query blocks run as several workgroups over even pieces of their key blocks
+  const int np = fwd_pieces(p, nkb);
+  const bool split = np > 1;
+  if (piece >= np) return;
+  const int kb_lo = nkb * piece / np, kb_hi = nkb * (piece + 1) / np;
 
   const bf16_t* srcs[2] = {kbase, vbase};
   const int64_t strides[2] = {p.k_sr, p.v_sr};
@@ -682,8 +687,8 @@ __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, 
       oacc[dt][s] = oacc[dt][s] * a0 + *reinterpret_cast<const f32x4*>(&R[row * RLD + 16 * dt + 4 * lg]) * a1;
   }
   if (split) {
-    // unnormalised state (O, m, l) of this half for the merge kernel
-    float* part = p.part + ((((int64_t)seq * p.H + h) * p.nqb + qb) * 2 + half) * (64 * DP + 128);
+    // unnormalised state (O, m, l) of this piece for the merge kernel
+    float* part = p.part + ((((int64_t)seq * p.H + h) * p.nqb + qb) * p.npart + piece) * (64 * DP + 128);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const int row = 32 * qh + 16 * s + li;
@@ -795,18 +800,18 @@ __global__ void __launch_bounds__(64) fwd_jobs_clear_kernel(int* jobs) {
   if (threadIdx.x < 8) jobs[32 * threadIdx.x] = 0;
 }
 
-// Merge of the two halves of a split query block, then the epilogue of relation_fwd_tile_kernel:
-// four threads per row, each owning DP / 4 head-dim elements.
+// Merge of the pieces of a split query block, then the epilogue of relation_fwd_tile_kernel: eight
+// threads per row, each owning DP / 8 head-dim elements; two workgroups of 32 rows a query block.
 template <int DP, bool PAD>
 __global__ void __launch_bounds__(256) relation_fwd_merge_kernel(const FwdParams p) {
-  constexpr int PER = DP / 4;  // elements per thread
+  constexpr int PER = DP / 8;  // elements per thread
+  constexpr int64_t PSTRIDE = 64 * DP + 128;
   const int tid = threadIdx.x;
-  const int row = tid >> 2, quarter = tid & 3;
-  const int bid = blockIdx.x;
-  const int h = bid % p.H;
-  const int rest = bid / p.H;
-  const int seq = rest % p.nseq;
-  const int qb = rest / p.nseq;
+  const int h = blockIdx.x % p.H;
+  const int rest = blockIdx.x / p.H;
+  const int row = 32 * (rest & 1) + (tid >> 3), lane8 = tid & 7;
+  const int seq = (rest >> 1) % p.nseq;
+  const int qb = (rest >> 1) / p.nseq;
 
   int TQs, qs;
   int64_t qoff, koff, voff, yoff, soff;
@@ -830,37 +835,45 @@ __global__ void __launch_bounds__(256) relation_fwd_merge_kernel(const FwdParams
   }
   if (qb * 64 >= TQs) return;
   const int qlast = min(TQs, qb * 64 + 64) - 1;
-  const int nkb = (qs + qlast + 63) / 64;
-  if (!(nkb > p.split_c)) return;  // this query block ran whole
-  const float* P0 = p.part + (((int64_t)seq * p.H + h) * p.nqb + qb) * 2 * (64 * DP + 128);
-  const float* P1 = P0 + (64 * DP + 128);
+  const int np = fwd_pieces(p, (qs + qlast + 63) / 64);
+  if (np == 1) return;  // this query block ran whole
+  const float* P = p.part + (((int64_t)seq * p.H + h) * p.nqb + qb) * p.npart * PSTRIDE;
   const int qi = qb * 64 + row;
   const bool qv = qi < TQs;
   const int qa = qs + qi;
-  const float m0 = P0[64 * DP + row], l0 = P0[64 * DP + 64 + row];
-  const float m1 = P1[64 * DP + row], l1 = P1[64 * DP + 64 + row];
-  const float mm = fmaxf(m0, m1);
-  const float a0 = fexp2(m0 - mm), a1 = fexp2(m1 - mm);
-  const float lt = l0 * a0 + l1 * a1;
-  const bool has = lt > 0.f;
-  const float lse = has ? (mm + __log2f(lt)) * kLn2 : kNegInf;
-  const float inv_l = has ? 1.0f / lt : 0.f;
-  const int d0 = quarter * PER;
+  const int d0 = lane8 * PER;
+  // the Self score's operands first: their loads pass under the pieces'
   const bf16_t* qrow = reinterpret_cast<const bf16_t*>(p.p1) + qoff + int64_t(h) * p.q_sh + int64_t(qv ? qi : 0) * p.q_sr;
   const bf16_t* krow = reinterpret_cast<const bf16_t*>(p.p2) + koff + int64_t(h) * p.k_sh + int64_t(qv ? qa : 0) * p.k_sr;
   float ud = 0.f;
-  if (qv) {
 #pragma unroll
-    for (int c = 0; c < PER; c += 8) {
-      if (PAD && d0 + c >= p.D) break;
-      const bf16x8 q8 = *reinterpret_cast<const bf16x8*>(qrow + d0 + c);
-      const bf16x8 k8 = *reinterpret_cast<const bf16x8*>(krow + d0 + c);
+  for (int c = 0; c < PER; c += 4) {
+    if (PAD && d0 + c >= p.D) break;
+    const bf16x4 q4 = *reinterpret_cast<const bf16x4*>(qrow + d0 + c);
+    const bf16x4 k4 = *reinterpret_cast<const bf16x4*>(krow + d0 + c);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ud = fmaf((float)q8[e], (float)k8[e], ud);
-    }
+    for (int e = 0; e < 4; ++e) ud = fmaf((float)q4[e], (float)k4[e], ud);
   }
+  float mm = 0.f;  // the pieces' references are at least 0
+  for (int i = 0; i < np; ++i) mm = fmaxf(mm, P[i * PSTRIDE + 64 * DP + row]);
+  float lt = 0.f;
+  f32x4 o[PER / 4];
+#pragma unroll
+  for (int c = 0; c < PER / 4; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+  for (int i = 0; i < np; ++i) {
+    const float* Pi = P + i * PSTRIDE;
+    const float a = fexp2(Pi[64 * DP + row] - mm);
+    lt = fmaf(Pi[64 * DP + 64 + row], a, lt);
+#pragma unroll
+    for (int c = 0; c < PER / 4; ++c) o[c] += *reinterpret_cast<const f32x4*>(Pi + row * DP + d0 + 4 * c) * a;
+  }
+  const bool has = lt > 0.f;
+  const float lse = has ? (mm + __log2f(lt)) * kLn2 : kNegInf;
+  const float inv_l = has ? 1.0f / lt : 0.f;
   ud += wave_xor(ud, 1);
   ud += wave_xor(ud, 2);
+  ud += wave_xor(ud, 4);
   const float sself = sigmoid_acc(ud * p.scale * p.tau_inv);
   const float gate = has ? sigmoid_acc(lse - *p.lam * logf((float)qa + 1.0f) - sself) : 0.f;
   if (!qv) return;
@@ -868,26 +881,17 @@ __global__ void __launch_bounds__(256) relation_fwd_merge_kernel(const FwdParams
   bf16_t* yrow = reinterpret_cast<bf16_t*>(p.y) + yoff + int64_t(h) * p.y_sh + int64_t(qi) * p.y_sr;
   float* brow = p.ibar + (soff + qi) * int64_t(PAD ? p.D : DP);
 #pragma unroll
-  for (int c = 0; c < PER; c += 8) {
-    if (PAD && d0 + c >= p.D) break;
-    const bf16x8 i8 = *reinterpret_cast<const bf16x8*>(irow + d0 + c);
-    float ib[8], yv[8];
+  for (int c = 0; c < PER / 4; ++c) {
+    if (PAD && d0 + 4 * c >= p.D) break;
+    const bf16x4 i4 = *reinterpret_cast<const bf16x4*>(irow + d0 + 4 * c);
+    bf16x4 y4;
+    const f32x4 ib = o[c] * inv_l;
 #pragma unroll
-    for (int e = 0; e < 8; e += 4) {
-      const float4 o0 = *reinterpret_cast<const float4*>(&P0[row * DP + d0 + c + e]);
-      const float4 o1 = *reinterpret_cast<const float4*>(&P1[row * DP + d0 + c + e]);
-      ib[e] = (o0.x * a0 + o1.x * a1) * inv_l;
-      ib[e + 1] = (o0.y * a0 + o1.y * a1) * inv_l;
-      ib[e + 2] = (o0.z * a0 + o1.z * a1) * inv_l;
-      ib[e + 3] = (o0.w * a0 + o1.w * a1) * inv_l;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) yv[e] = (1.0f - gate) * (float)i8[e] + gate * ib[e];
-    *reinterpret_cast<bf16x8*>(yrow + d0 + c) = Elem<bf16_t>::from_f32(yv).v;
-    *reinterpret_cast<float4*>(brow + d0 + c) = make_float4(ib[0], ib[1], ib[2], ib[3]);
-    *reinterpret_cast<float4*>(brow + d0 + c + 4) = make_float4(ib[4], ib[5], ib[6], ib[7]);
+    for (int e = 0; e < 4; ++e) y4[e] = (__bf16)((1.0f - gate) * (float)i4[e] + gate * ib[e]);
+    *reinterpret_cast<bf16x4*>(yrow + d0 + 4 * c) = y4;
+    *reinterpret_cast<f32x4*>(brow + d0 + 4 * c) = ib;
   }
-  if (quarter == 0) {
+  if (lane8 == 0) {
     p.lse[soff + qi] = lse;
     p.g[soff + qi] = gate;
   }
@@ -921,19 +925,35 @@ static bool fwd_tiles(const mote_relation_fwd_args* a) {
   return a->dtype == MOTE_BF16 && tile_strides_ok(a->p1, a->p2, a->info);
 }
 
-// Key blocks of the longest query block; query blocks with more than split_c of them run as halves.
+int device_cu_count();
+
+// Key blocks of the longest query block.
 static int fwd_max_key_blocks(const mote_relation_fwd_args* a) {
   const int qs = a->cu_seqlens ? 0 : a->q_start;
   return (qs + a->TQ - 1 + 63) / 64;
 }
-// Measured at the Mote-96M shape (78 key blocks), splitting does not pay for the merge launch; rows
-// beyond 96 key blocks (6144 positions) split.
+// Query blocks with more key blocks than this run as pieces of at most as many (1 << 30: none).
+// A launch is as long as its longest walk, or as its key blocks spread over the CUs. Where the walk is by
+// far the longer (few query blocks: new rows after a cached prefix, few sequences), pieces of the even share
+// of one workgroup a CU fill the chip; they pay the partials' round trip and a merge launch, together about
+// twelve blocks' time, so the walk has to be longer than two pieces by that. 311 rows after 4096, H 8,
+// dh 96 (40 workgroups of 65 to 69 key blocks): 57.8 -> 24.4 us; with the share of two workgroups a CU, so twice the
+// partials, 23.7, and 1500 rows (192 workgroups of up to 24) would split: 30.3 us against 26.8 whole. At the
+// Mote-96M shape (78 key blocks, an even share of 97) splitting does not pay; rows beyond 96 key blocks
+// (6144 positions) run as halves.
 static int fwd_split_c(const mote_relation_fwd_args* a) {
   const int n = fwd_max_key_blocks(a);
+  const int64_t nqb = (a->TQ + 63) / 64;
+  const int64_t blocks = int64_t(a->B) * a->H * (nqb * n - nqb * (nqb - 1) / 2);  // (varlen: an upper bound)
+  const int64_t share = (blocks + device_cu_count() - 1) / device_cu_count();
+  const int64_t c = share < 6 ? 6 : share;
+  if (n >= 2 * c + 12) return int(c);
   return n > 96 ? (n + 1) / 2 : 1 << 30;
 }
-
-int device_cu_count();
+static int fwd_pieces_max(const mote_relation_fwd_args* a) {
+  const int c = fwd_split_c(a), n = fwd_max_key_blocks(a);
+  return n > c ? (n + c - 1) / c : 1;
+}
 
 // Persistent workgroups for the tile forward (one job counter per queue in the workspace) when there
 // are at least four jobs per workgroup slot, as in the varlen prefill (C5: 4,992 jobs on 512 slots,
@@ -954,7 +974,7 @@ size_t fwd_workspace_bytes(const mote_relation_fwd_args* a) {
   if (!a || a->TQ <= 0 || a->D <= 0 || a->D > 128 || !fwd_tiles(a)) return 0;
   if (fwd_split_c(a) >= (1 << 30)) return fwd_persistent(a) ? kFwdJobBytes : 0;
   const size_t nqb = (size_t(a->TQ) + 63) / 64;
-  return size_t(a->B) * a->H * nqb * 2 * (64 * size_t(padded_dim(a->D)) + 128) * sizeof(float);
+  return size_t(a->B) * a->H * nqb * fwd_pieces_max(a) * (64 * size_t(padded_dim(a->D)) + 128) * sizeof(float);
 }
 
 int launch_fwd(const mote_relation_fwd_args* a, hipStream_t stream) {
@@ -1010,6 +1030,7 @@ int launch_fwd(const mote_relation_fwd_args* a, hipStream_t stream) {
     const bool persist = have && !split;  // (the workspace then holds the job counters)
     fp.part = split ? reinterpret_cast<float*>(a->workspace) : nullptr;
     fp.split_c = split ? fwd_split_c(a) : (1 << 30);
+    fp.npart = split ? fwd_pieces_max(a) : 1;
     fp.jobs = persist ? reinterpret_cast<int*>(a->workspace) : nullptr;
     fp.jobs_nq = a->H % 8 == 0 ? 8 : a->H % 4 == 0 ? 4 : a->H % 2 == 0 ? 2 : 1;
     const int nb = int(units * fp.nqb);
@@ -1021,8 +1042,8 @@ int launch_fwd(const mote_relation_fwd_args* a, hipStream_t stream) {
     hipLaunchKernelGGL((relation_fwd_tile_persistent_kernel<DPV, PADV>), dim3(pgrid > 0 ? pgrid : fp.jobs_nq), dim3(256), 0, \
                        stream, fp);                                                                             \
   } else {                                                                                                      \
-    hipLaunchKernelGGL((relation_fwd_tile_kernel<DPV, PADV>), dim3(split ? 2 * nb : nb), dim3(256), 0, stream, fp);    \
-    if (split) hipLaunchKernelGGL((relation_fwd_merge_kernel<DPV, PADV>), dim3(nb), dim3(256), 0, stream, fp);          \
+    hipLaunchKernelGGL((relation_fwd_tile_kernel<DPV, PADV>), dim3(nb * fp.npart), dim3(256), 0, stream, fp);          \
+    if (split) hipLaunchKernelGGL((relation_fwd_merge_kernel<DPV, PADV>), dim3(2 * nb), dim3(256), 0, stream, fp);      \
   }
     if (DP == a->D) {
       switch (DP) {

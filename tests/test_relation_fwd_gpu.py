@@ -249,3 +249,42 @@ def test_persistent_equals_one_job_per_workgroup(cuda, monkeypatch, B, H, T, S, 
         torch.cuda.synchronize()
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+# Few query blocks over many key blocks run as pieces of their key range, merged by a second launch: a
+# cached prefix with one row, one block and a ragged block after it, several heads and sequences, a padded
+# head dim, all four tile dims, and a single long sequence (whose short query blocks stay whole). Against
+# the float64 oracle of the same bf16 inputs (2e-2 of the largest element, the suite's bf16 tolerance).
+@pytest.mark.parametrize("B,H,T,S,D", [(1, 2, 1, 1500, 96), (1, 8, 65, 1999, 96), (2, 2, 300, 1000, 64), (1, 2, 130, 1100, 128),
+                                       (1, 4, 40, 1600, 32), (1, 2, 77, 1300, 48), (1, 1, 1411, 0, 64)])
+def test_key_range_pieces_match_oracle(cuda, B, H, T, S, D):
+    from mote_amd.flash_relation import _launch_fwd
+
+    print(f"case pieces B={B} H={H} T={T} S={S} D={D}", flush=True)
+    g = torch.Generator().manual_seed(T + S)
+    p1, p2, info = (torch.randn(B, H, n, D, generator=g).bfloat16() for n in (T, S + T, S + T))
+    lam = torch.tensor(0.5)
+    ref = [t.double() for t in (p1, p2, info)]
+    yr, gr = O.relation_reference(*ref, lam.double(), 2.0, S, dtype=torch.float64)
+    dev = [t.to(cuda) for t in (p1, p2, info)]
+    y, gate, ibar, lse = _launch_fwd(*dev, lam.to(cuda), 2.0, S)
+    assert rel_err(y, yr) < 2e-2 and rel_err(gate, gr) < 2e-2
+    assert bool(torch.isfinite(ibar).all()) and bool(torch.isfinite(lse[:, :, 1 if S == 0 else 0:]).all())
+    again = _launch_fwd(*dev, lam.to(cuda), 2.0, S)
+    assert all(torch.equal(a, b) for a, b in zip(again, (y, gate, ibar, lse)))
+
+
+def test_key_range_pieces_varlen(cuda):
+    """Two packed sequences, one long enough for pieces, one of a few rows: each equals its dense call to
+    the rounding of another split of the same sums."""
+    from mote_amd.flash_relation import flash_relation, flash_relation_varlen
+
+    print("case pieces varlen", flush=True)
+    g = torch.Generator().manual_seed(5)
+    p = [torch.randn(2, 1290, 96, generator=g).bfloat16().to(cuda) for _ in range(3)]
+    cu = torch.tensor([0, 10, 1290], dtype=torch.int32, device=cuda)
+    lam = torch.tensor(0.5, device=cuda)
+    y, gate = flash_relation_varlen(*p, lam, cu, 1280)
+    for a, b in ((0, 10), (10, 1290)):
+        yd, gd = flash_relation(*(t[None, :, a:b] for t in p), lam)
+        assert rel_err(y[:, a:b], yd[0]) < 1e-2 and rel_err(gate[:, a:b], gd[0]) < 1e-4
