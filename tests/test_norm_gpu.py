@@ -129,6 +129,13 @@ def test_widths_prenorm_bf16_fp32_stream(cuda, D):
     _check_f64(cuda, 37, D, torch.bfloat16, torch.float32, True, True)
 
 
+@pytest.mark.parametrize("D", [512, 764, 772])
+def test_unit_class_edges(cuda, D):
+    # the last width of the two-unit instance, the last short one of three units, the first of four
+    _check_f64(cuda, 65, D, torch.bfloat16, torch.float32, True, True)
+    _check_f64(cuda, 5, D, torch.float32, None, False, True)
+
+
 @pytest.mark.parametrize("rows", [1, 3, 4, 5, 4095, 10003])
 def test_ragged_rows_and_multipass_backward(cuda, rows):
     # 10003 rows: more than the backward's 1024 workgroups x 4 waves, so waves take several rows
