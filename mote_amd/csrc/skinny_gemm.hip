@@ -52,12 +52,21 @@ __global__ void __launch_bounds__(64 * kSkWaves) skinny_gemm_kernel(const Skinny
     }
   }
   // the decode step's exchange mass (graph.py:186) on the side: workgroup 0, wave 1, lane b < B
-  // sums g[b][0 .. heads) in head order
+  // sums g[b][0 .. heads) in head order, eight loads in flight (one after the other, the eight heads'
+  // loads were the launch's longest chain: a token of 12 layers at batch 1 255.2 -> 253.0 us)
   const int xb = int(threadIdx.x) - 64;
   const bool xm_lane = p.xm != nullptr && blockIdx.x == 0 && xb >= 0 && xb < p.B;
   float gsum = 0.f;
-  if (xm_lane)
-    for (int h = 0; h < p.heads; ++h) gsum += p.g[int64_t(xb) * p.heads + h];
+  if (xm_lane) {
+    const float* gb = p.g + int64_t(xb) * p.heads;
+    for (int h0 = 0; h0 < p.heads; h0 += 8) {
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = gb[min(h0 + j, p.heads - 1)];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) gsum = h0 + j < p.heads ? gsum + v[j] : gsum;
+    }
+  }
   // the predicate after the loads are issued (reads are harmless); uniform, so the whole
   // workgroup leaves before its barrier
   if (p.run && p.run[0] == 0) return;
