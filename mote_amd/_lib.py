@@ -8,6 +8,7 @@ HIP stream of the tensors' device.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import os
 import threading
 
@@ -335,6 +336,25 @@ def lib():
                     fn.restype = restype
                 _lib = handle
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The torch ops' native launchers (csrc/torch_launch.cpp); raises RuntimeError when not built."""
+    global _native
+    if _native is None:
+        with _lock:
+            if _native is None:
+                path = os.path.join(_HERE, "lib", "_torch_launch.so")
+                if not os.path.exists(path):
+                    raise RuntimeError(f"_torch_launch.so is not built ({path}); run `python -m mote_amd.build`")
+                spec = importlib.util.spec_from_file_location("_torch_launch", path)
+                mod = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(mod)
+                _native = mod
+    return _native
 
 
 def available() -> bool:

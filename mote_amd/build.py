@@ -1,4 +1,4 @@
-"""Build libmote_relation.so for gfx950 with hipcc, in-tree.
+"""Build libmote_relation.so for gfx950 with hipcc, and the torch ops' launchers over it, in-tree.
 
     python -m mote_amd.build          # compile every csrc/*.hip and link mote_amd/lib/libmote_relation.so
 
@@ -22,6 +22,7 @@ CSRC = os.path.join(PKG, "csrc")
 BUILD = os.path.join(PKG, "_build")
 LIBDIR = os.path.join(PKG, "lib")
 LIBNAME = "libmote_relation.so"
+TORCHNAME = "_torch_launch.so"
 ARCH = "gfx950"
 
 # -packed-fp32-ops: no v_pk_{add,mul,fma}_f32 (the host pass warns that it does not know the
@@ -53,6 +54,28 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _build_torch_launch() -> str:
+    """The torch ops' native launchers (host code over torch's headers, linked to the library beside it)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension as ce
+
+    inc = [*ce.include_paths(), sysconfig.get_paths()["include"], os.path.join(ROOT, "include")]
+    out = os.path.join(LIBDIR, TORCHNAME)
+    tmp = out + ".tmp"
+    cmd = [shutil.which("g++") or "g++", "-O2", "-fPIC", "-shared", "-std=c++17",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{p}" for p in inc),
+           os.path.join(CSRC, "torch_launch.cpp"), "-o", tmp, f"-L{LIBDIR}", f"-l:{LIBNAME}",
+           f"-L{os.path.join(os.path.dirname(torch.__file__), 'lib')}", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on torch_launch.cpp:\n{r.stderr[-6000:]}")
+    os.replace(tmp, out)
+    return out
+
+
 def build(verbose: bool = False) -> str:
     """Compile and link; returns the path of the shared library."""
     os.makedirs(BUILD, exist_ok=True)
@@ -69,6 +92,7 @@ def build(verbose: bool = False) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr[-4000:]}")
     os.replace(tmp, out)
+    _build_torch_launch()
     if verbose:
         print(f"built {out} from {len(srcs)} sources in {time.time() - t0:.1f}s")
     return out

@@ -45,19 +45,7 @@ def chunk_route(mask: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.T
     positions in order, then the others), num (int32) and cu_seqlens (int32 [B + 1])."""
     _need_gpu(mask, "mote::chunk_route")
     m = _mask_u8(mask)
-    B, Ln = m.shape
-    cum = torch.empty(B, Ln, device=m.device, dtype=torch.int32)
-    perm = torch.empty(B, Ln, device=m.device, dtype=torch.int32)
-    num = torch.empty(B, device=m.device, dtype=torch.int32)
-    cu = torch.empty(B + 1, device=m.device, dtype=torch.int32)
-    a = L.ChunkRouteArgs()
-    a.B, a.L = B, Ln
-    a.mask, a.mask_sr = m.data_ptr(), m.stride(0)
-    a.cum, a.perm, a.num, a.cu_seqlens = cum.data_ptr(), perm.data_ptr(), num.data_ptr(), cu.data_ptr()
-    if B == 0:
-        cu.zero_()
-    L.check(L.lib().mote_chunk_route(a, L.stream_of(m)), "mote_chunk_route")
-    return cum, perm, num, cu
+    return L.native().chunk_route(m, L.stream_of(m))
 
 
 @chunk_route.register_fake
@@ -165,24 +153,7 @@ def dechunk(hidden: torch.Tensor, prob: torch.Tensor, perm: torch.Tensor, num: t
     _need_gpu(prob, "mote::dechunk")
     h = _last_unit(hidden)
     pr = _last_unit(prob)
-    B, M, D = h.shape
-    L_len = mask.shape[1]
-    out = torch.empty(B, L_len, D, device=pr.device, dtype=h.dtype)
-    w = torch.empty(B, M, D, device=pr.device, dtype=torch.float32)
-    ini = init.detach().to(torch.float32).contiguous() if init is not None else None
-    a = L.DechunkArgs()
-    a.dtype, a.prob_dtype, a.out_dtype = L.dtype_code(h), L.dtype_code(pr), L.dtype_code(out)
-    a.B, a.L, a.M, a.D, a.eps = B, L_len, M, D, float(eps)
-    a.hidden, a.h_sb, a.h_sr = h.data_ptr(), h.stride(0), h.stride(1)
-    a.prob, a.p_sb, a.p_sr = pr.data_ptr(), pr.stride(0), pr.stride(1)
-    a.perm, a.num, a.cum = perm.data_ptr(), num.data_ptr(), cum.data_ptr()
-    a.init = ini.data_ptr() if ini is not None else None
-    a.out, a.o_sb, a.o_sr = out.data_ptr(), out.stride(0), out.stride(1)
-    a.w = w.data_ptr()
-    ws = torch.empty(max(int(L.lib().mote_dechunk_workspace(a)), 16), device=pr.device, dtype=torch.uint8)
-    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    L.check(L.lib().mote_dechunk_fwd(a, L.stream_of(pr)), "mote_dechunk_fwd")
-    return out, w
+    return L.native().dechunk(h, pr, perm, num, cum, mask.shape[1], eps, init, L.stream_of(pr))
 
 
 @dechunk.register_fake
@@ -198,25 +169,7 @@ def dechunk_bwd(dout: torch.Tensor, hidden: torch.Tensor, prob: torch.Tensor, pe
     h, pr = _last_unit(hidden), _last_unit(prob)
     g = _last_unit(dout.to(h.dtype))
     m = _mask_u8(mask)
-    B, M, D = h.shape
-    Ln = g.shape[1]
-    dh = torch.empty(B, M, D, device=h.device, dtype=h.dtype)
-    dp = torch.empty(B, Ln, 2, device=h.device, dtype=pr.dtype)
-    a = L.DechunkBwdArgs()
-    a.dtype, a.prob_dtype, a.dout_dtype = L.dtype_code(h), L.dtype_code(pr), L.dtype_code(g)
-    a.dx_dtype, a.dprob_dtype = L.dtype_code(dh), L.dtype_code(dp)
-    a.B, a.L, a.M, a.D, a.eps = B, Ln, M, D, float(eps)
-    a.dout, a.g_sb, a.g_sr = g.data_ptr(), g.stride(0), g.stride(1)
-    a.hidden, a.h_sb, a.h_sr = h.data_ptr(), h.stride(0), h.stride(1)
-    a.prob, a.p_sb, a.p_sr = pr.data_ptr(), pr.stride(0), pr.stride(1)
-    a.perm, a.num, a.mask, a.mask_sr, a.cum = perm.data_ptr(), num.data_ptr(), m.data_ptr(), m.stride(0), cum.data_ptr()
-    a.w = w.data_ptr()
-    a.dhidden, a.dh_sb, a.dh_sr = dh.data_ptr(), dh.stride(0), dh.stride(1)
-    a.dprob, a.dp_sb, a.dp_sr = dp.data_ptr(), dp.stride(0), dp.stride(1)
-    ws = torch.empty(max(int(L.lib().mote_dechunk_bwd_workspace(a)), 16), device=h.device, dtype=torch.uint8)
-    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    L.check(L.lib().mote_dechunk_bwd(a, L.stream_of(h)), "mote_dechunk_bwd")
-    return dh, dp
+    return L.native().dechunk_bwd(g, h, pr, perm, num, m, cum, w, eps, L.stream_of(h))
 
 
 @dechunk_bwd.register_fake

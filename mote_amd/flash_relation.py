@@ -37,15 +37,6 @@ HAS_HIP = _hip_ready()
 HAS_TRITON = HAS_HIP  # the name the reference's callers test (relation.py:29, 228); no Triton here
 
 
-def _aligned(t: torch.Tensor) -> torch.Tensor:
-    """The kernels read 16-byte chunks: unit stride on the last axis, strides a multiple of the
-    chunk and a 16-byte aligned base. Anything else is copied to a contiguous tensor."""
-    epc = 16 // t.element_size()
-    if t.stride(-1) != 1 or t.data_ptr() % 16 or any(s % epc for s in t.stride()[:-1]):
-        return t.contiguous()
-    return t
-
-
 def _check_device(*ts):
     for t in ts:
         if not t.is_cuda:
@@ -57,18 +48,6 @@ def _token_major(B, H, T, D, like: torch.Tensor, dtype) -> torch.Tensor:
     return torch.empty(B, T, H, D, device=like.device, dtype=dtype).transpose(1, 2)
 
 
-def _fwd_workspace(a, device):
-    """Scratch for the split of the longest query blocks (partial softmax states); the caller keeps
-    the returned tensor alive until the launch is queued (the caching allocator orders reuse)."""
-    n = int(L.lib().mote_relation_fwd_workspace(a))
-    if n == 0:
-        a.workspace, a.workspace_bytes = None, 0
-        return None
-    ws = torch.empty(n, device=device, dtype=torch.uint8)
-    a.workspace, a.workspace_bytes = ws.data_ptr(), n
-    return ws
-
-
 def _launch_fwd(p1, p2, info, lam, tau_s: float, q_start: int):
     B, H, TQ, D = p1.shape
     TK = p2.shape[2]
@@ -77,49 +56,13 @@ def _launch_fwd(p1, p2, info, lam, tau_s: float, q_start: int):
     if p2.dtype != p1.dtype or info.dtype != p1.dtype:
         raise TypeError("p1, p2 and info must share a dtype")
     _check_device(p1, p2, info, lam)
-    p1, p2, info = _aligned(p1), _aligned(p2), _aligned(info)
-    lam32 = lam.detach().to(torch.float32).reshape(1).contiguous()
-    y = _token_major(B, H, TQ, D, p1, info.dtype)
-    ibar = torch.empty(B, H, TQ, D, device=p1.device, dtype=torch.float32)
-    lse = torch.empty(B, H, TQ, device=p1.device, dtype=torch.float32)
-    g = torch.empty(B, H, TQ, device=p1.device, dtype=torch.float32)
-    a = L.FwdArgs()
-    a.dtype = L.dtype_code(p1)
-    a.B, a.H, a.TQ, a.TK, a.D, a.q_start = B, H, TQ, TK, D, q_start
-    a.tau_s = float(tau_s)
-    a.p1, a.p2, a.info, a.y = L.view(p1), L.view(p2), L.view(info), L.view(y)
-    a.ibar, a.lse, a.g, a.lam = ibar.data_ptr(), lse.data_ptr(), g.data_ptr(), lam32.data_ptr()
-    a.cu_seqlens, a.total_rows = None, 0
-    ws = _fwd_workspace(a, p1.device)
-    L.check(L.lib().mote_relation_fwd(a, L.stream_of(p1)), "mote_relation_fwd")
-    return y, g, ibar, lse
+    return L.native().relation_fwd(p1, p2, info, lam, float(tau_s), q_start, None, 0, L.stream_of(p1))
 
 
 def _launch_bwd(p1, p2, info, ibar, lse, g, dy, tau_s: float, q_start: int, deterministic: bool):
-    B, H, TQ, D = p1.shape
-    TK = p2.shape[2]
     _check_device(p1, p2, info, dy)
-    p1, p2, info = _aligned(p1), _aligned(p2), _aligned(info)
-    dy = _aligned(dy.to(p1.dtype))
-    ibar, lse, g = ibar.contiguous(), lse.contiguous(), g.contiguous()
-    dp1 = _token_major(B, H, TQ, D, p1, p1.dtype)
-    dp2 = _token_major(B, H, TK, D, p1, p2.dtype)
-    dinfo = _token_major(B, H, TK, D, p1, info.dtype)
-    dlam = torch.empty((), device=p1.device, dtype=torch.float32)
-    a = L.BwdArgs()
-    a.dtype = L.dtype_code(p1)
-    a.B, a.H, a.TQ, a.TK, a.D, a.q_start = B, H, TQ, TK, D, q_start
-    a.tau_s = float(tau_s)
-    a.deterministic = int(bool(deterministic))
-    a.p1, a.p2, a.info, a.dy = L.view(p1), L.view(p2), L.view(info), L.view(dy)
-    a.ibar, a.lse, a.g = ibar.data_ptr(), lse.data_ptr(), g.data_ptr()
-    a.dp1, a.dp2, a.dinfo = L.view(dp1), L.view(dp2), L.view(dinfo)
-    a.dlam = dlam.data_ptr()
-    nbytes = L.lib().mote_relation_bwd_workspace(a)
-    ws = torch.empty(max(int(nbytes), 16), device=p1.device, dtype=torch.uint8)
-    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    L.check(L.lib().mote_relation_bwd(a, L.stream_of(p1)), "mote_relation_bwd")
-    return dp1, dp2, dinfo, dlam
+    return L.native().relation_bwd(p1, p2, info, ibar, lse, g, dy, float(tau_s), q_start, bool(deterministic),
+                                   L.stream_of(p1))
 
 
 @torch.library.custom_op("mote::relation_fwd", mutates_args=())
@@ -215,27 +158,11 @@ def relation_reference(p1: torch.Tensor, p2: torch.Tensor, info: torch.Tensor, l
 def _relation_fwd_varlen(p1: torch.Tensor, p2: torch.Tensor, info: torch.Tensor, lam: torch.Tensor,
                          cu_seqlens: torch.Tensor, max_seqlen: int,
                          tau_s: float) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    H, total, D = p1.shape
     _check_device(p1, p2, info, lam, cu_seqlens)
-    p1, p2, info = (_aligned(t.unsqueeze(0)) for t in (p1, p2, info))
     cu = cu_seqlens.to(torch.int32).contiguous()
-    nseq = cu.numel() - 1
-    lam32 = lam.detach().to(torch.float32).reshape(1).contiguous()
-    y = torch.empty(total, H, D, device=p1.device, dtype=info.dtype).permute(1, 0, 2)
-    ibar = torch.empty(H, total, D, device=p1.device, dtype=torch.float32)
-    lse = torch.empty(H, total, device=p1.device, dtype=torch.float32)
-    g = torch.empty(H, total, device=p1.device, dtype=torch.float32)
-    a = L.FwdArgs()
-    a.dtype = L.dtype_code(p1)
-    a.B, a.H, a.TQ, a.TK, a.D, a.q_start = nseq, H, int(max_seqlen), int(max_seqlen), D, 0
-    a.tau_s = float(tau_s)
-    a.p1, a.p2, a.info = L.view(p1), L.view(p2), L.view(info)
-    a.y = L.view(y.unsqueeze(0))
-    a.ibar, a.lse, a.g, a.lam = ibar.data_ptr(), lse.data_ptr(), g.data_ptr(), lam32.data_ptr()
-    a.cu_seqlens, a.total_rows = cu.data_ptr(), total
-    ws = _fwd_workspace(a, p1.device)
-    L.check(L.lib().mote_relation_fwd(a, L.stream_of(p1)), "mote_relation_fwd (varlen)")
-    return y, g, ibar, lse
+    y, g, ibar, lse = L.native().relation_fwd(p1.unsqueeze(0), p2.unsqueeze(0), info.unsqueeze(0), lam, float(tau_s), 0, cu,
+                                              int(max_seqlen), L.stream_of(p1))
+    return y[0], g[0], ibar[0], lse[0]
 
 
 @_relation_fwd_varlen.register_fake

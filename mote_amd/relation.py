@@ -82,32 +82,12 @@ def _apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.
 
 
 # ---- mote::rope_givens ---------------------------------------------------------------------------
-def _heads_out(B, T, H, D, like, dtype):
-    return torch.empty(B, T, H, D, device=like.device, dtype=dtype).transpose(1, 2)
-
-
 @torch.library.custom_op("mote::rope_givens", mutates_args=())
 def _rope_givens(qkv: torch.Tensor, inv_freq: Optional[torch.Tensor], theta: Optional[torch.Tensor], n_heads: int,
                  parity: int, pos0: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    B, T, D3 = qkv.shape
-    H = n_heads
-    D = D3 // (3 * H)
     if not qkv.is_cuda:
         raise RuntimeError("mote::rope_givens needs the HIP library and an MI355X")
-    qkv = qkv if qkv.stride(-1) == 1 else qkv.contiguous()
-    p1 = _heads_out(B, T, H, D, qkv, qkv.dtype)
-    p2 = _heads_out(B, T, H, D, qkv, qkv.dtype)
-    info = _heads_out(B, T, H, D, qkv, qkv.dtype)
-    a = L.RopeArgs()
-    a.dtype = L.dtype_code(qkv)
-    a.B, a.T, a.H, a.D, a.pos0, a.layer_parity = B, T, H, D, int(pos0), int(parity)
-    inv = None if inv_freq is None else inv_freq.to(device=qkv.device, dtype=torch.float32).contiguous()
-    th = None if theta is None else theta.detach().to(device=qkv.device, dtype=torch.float32).contiguous()
-    a.inv_freq, a.theta = L.ptr(inv), L.ptr(th)
-    a.qkv, a.qkv_sb, a.qkv_sr = qkv.data_ptr(), qkv.stride(0), qkv.stride(1)
-    a.p1, a.p2, a.info = L.view(p1), L.view(p2), L.view(info)
-    L.check(L.lib().mote_rope_givens_fwd(a, L.stream_of(qkv)), "mote_rope_givens_fwd")
-    return p1, p2, info
+    return L.native().rope_givens(qkv, inv_freq, theta, n_heads, parity, pos0, L.stream_of(qkv))
 
 
 @_rope_givens.register_fake
@@ -125,31 +105,8 @@ def _rope_givens_bwd(dp1: torch.Tensor, dp2: torch.Tensor, dinfo: torch.Tensor, 
                      pos0: int, info_only: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
     """(dqkv [B, T, 3 H dh], dtheta). qkv is the projection output, or with info_only its I~ part
     alone ([B, T, H dh]): the backward reads only the I~ columns (for dtheta)."""
-    B, T, Dx = qkv.shape
-    H = n_heads
-    D = Dx // H if info_only else Dx // (3 * H)
-    D3 = 3 * H * D
-    qkv = qkv if qkv.stride(-1) == 1 else qkv.contiguous()
-    dp1, dp2, dinfo = (t.to(qkv.dtype) if t.stride(-1) == 1 else t.to(qkv.dtype).contiguous() for t in (dp1, dp2, dinfo))
-    dqkv = torch.empty(B, T, D3, device=qkv.device, dtype=qkv.dtype)
-    # written whole by the kernel when theta is given
-    dtheta = (torch.empty if theta is not None else torch.zeros)(max(H // 2, 1), device=qkv.device, dtype=torch.float32)
-    a = L.RopeBwdArgs()
-    a.dtype = L.dtype_code(qkv)
-    a.B, a.T, a.H, a.D, a.pos0, a.layer_parity = B, T, H, D, int(pos0), int(parity)
-    inv = None if inv_freq is None else inv_freq.to(device=qkv.device, dtype=torch.float32).contiguous()
-    th = None if theta is None else theta.detach().to(device=qkv.device, dtype=torch.float32).contiguous()
-    a.inv_freq, a.theta = L.ptr(inv), L.ptr(th)
-    a.qkv, a.qkv_sb, a.qkv_sr = qkv.data_ptr(), qkv.stride(0), qkv.stride(1)
-    a.qkv_info_only = int(bool(info_only))
-    a.dp1, a.dp2, a.dinfo = L.view(dp1), L.view(dp2), L.view(dinfo)
-    a.dqkv, a.dqkv_sb, a.dqkv_sr = dqkv.data_ptr(), dqkv.stride(0), dqkv.stride(1)
-    a.dtheta = dtheta.data_ptr()
-    nbytes = L.lib().mote_rope_givens_bwd_workspace(a)
-    ws = torch.empty(max(int(nbytes), 16), device=qkv.device, dtype=torch.uint8)
-    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    L.check(L.lib().mote_rope_givens_bwd(a, L.stream_of(qkv)), "mote_rope_givens_bwd")
-    return dqkv, dtheta
+    return L.native().rope_givens_bwd(dp1, dp2, dinfo, qkv, inv_freq, theta, n_heads, parity, pos0, info_only,
+                                      L.stream_of(qkv))
 
 
 @_rope_givens_bwd.register_fake
@@ -211,13 +168,15 @@ _ROPE_TABLES_PINNED: "dict" = {}   # tables a captured graph reads, kept for the
 _ROPE_TABLES_MAX = 32
 
 
-def _rope_table_ws(a, x: torch.Tensor, inv: Optional[torch.Tensor], cacheable: bool) -> Tuple[torch.Tensor, int]:
-    """Workspace for mote_qkv_rope_fwd and whether it already holds the table (table_ready).
-    `cacheable`: inv is the caller's own frequency tensor (not a converted temporary)."""
-    n = max(int(L.lib().mote_qkv_rope_workspace(a)), 16)
+def _rope_table_ws(T: int, D: int, pos0: int, x: torch.Tensor, inv: Optional[torch.Tensor],
+                   cacheable: bool) -> Tuple[torch.Tensor, int]:
+    """Workspace for mote_qkv_rope_fwd (mote_qkv_rope_workspace: a 32-bit cos / sin pair per position and
+    frequency) and whether it already holds the table (table_ready). `cacheable`: inv is the caller's own
+    frequency tensor (not a converted temporary)."""
+    n = max(T * (D // 2) * 4 if inv is not None else 0, 16)
     if inv is None or not cacheable:
         return torch.empty(n, device=x.device, dtype=torch.uint8), 0
-    key = (x.device, L.stream_of(x), inv.data_ptr(), a.T, a.pos0, a.D)
+    key = (x.device, L.stream_of(x), inv.data_ptr(), T, pos0, D)
     hit = _ROPE_TABLES.get(key)
     # the entry holds the frequency tensor itself: its memory cannot be recycled for another tensor
     # while the entry lives, and an in-place change of it shows in its version counter
@@ -241,45 +200,23 @@ def _qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, no
     [B, H, T, dh] to write instead of new tensors."""
     if not x.is_cuda:
         raise RuntimeError("mote::qkv_rope needs the HIP library and an MI355X")
-    B, T, K = x.shape
-    H = n_heads
-    D = K // H
-    norm = norm_w1 is not None
-    if norm != (norm_w2 is not None):
+    T, K = x.shape[1:]
+    D = K // n_heads
+    if (norm_w1 is None) != (norm_w2 is None):
         raise ValueError("mote::qkv_rope: QK-Norm needs both gains")
+    if norm_w1 is not None and (norm_w1.numel() != D or norm_w2.numel() != D):
+        raise ValueError("mote::qkv_rope: QK-Norm gains must have head-dim elements")
     x = x.contiguous()
-    apart = isinstance(w, tuple)
-    ws = tuple(t if t.data_ptr() % 16 == 0 else t.clone() for t in (t.contiguous() for t in w)) if apart else (w.contiguous(),)
-    p1 = _heads_out(B, T, H, D, x, x.dtype)
-    p2, info = into if into is not None else (_heads_out(B, T, H, D, x, x.dtype) for _ in range(2))
-    iraw = torch.empty(B, T, K, device=x.device, dtype=x.dtype) if keep_info else x.new_empty(0)
-    qkraw = torch.empty(B, T, 2 * K, device=x.device, dtype=x.dtype) if (keep_info and norm) else x.new_empty(0)
-    a = L.QkvRopeArgs()
-    a.B, a.T, a.H, a.D, a.pos0, a.layer_parity = B, T, H, D, int(pos0), int(parity)
-    a.x, a.x_sb, a.x_sr = x.data_ptr(), x.stride(0), x.stride(1)
-    a.w, a.w_sr = ws[0].data_ptr(), K
-    inv = None if inv_freq is None else inv_freq.to(device=x.device, dtype=torch.float32).contiguous()
-    th = None if theta is None else theta.detach().to(device=x.device, dtype=torch.float32).contiguous()
-    a.inv_freq, a.theta = L.ptr(inv), L.ptr(th)
-    a.p1, a.p2, a.info = L.view(p1), L.view(p2), L.view(info)
-    if keep_info:
-        a.info_raw, a.ir_sb, a.ir_sr = iraw.data_ptr(), iraw.stride(0), iraw.stride(1)
-    if norm:
-        nw1 = norm_w1.detach().to(device=x.device, dtype=torch.float32).contiguous()
-        nw2 = norm_w2.detach().to(device=x.device, dtype=torch.float32).contiguous()
-        if nw1.numel() != D or nw2.numel() != D:
-            raise ValueError("mote::qkv_rope: QK-Norm gains must have head-dim elements")
-        a.norm_w1, a.norm_w2, a.norm_eps = nw1.data_ptr(), nw2.data_ptr(), float(norm_eps)
-        if keep_info:
-            a.qk_raw, a.qr_sb, a.qr_sr = qkraw.data_ptr(), qkraw.stride(0), qkraw.stride(1)
-    table, a.table_ready = _rope_table_ws(a, x, inv, inv is inv_freq)
-    a.workspace, a.workspace_bytes = table.data_ptr(), table.numel()
-    if apart:
-        L.check(L.lib().mote_qkv_rope_parts_fwd(a, ws[1].data_ptr(), ws[2].data_ptr(), L.stream_of(x)),
-                "mote_qkv_rope_parts_fwd")
-    else:
-        L.check(L.lib().mote_qkv_rope_fwd(a, L.stream_of(x)), "mote_qkv_rope_fwd")
-    return p1, p2, info, iraw, qkraw
+    ws = [t.contiguous() for t in w] if isinstance(w, tuple) else [w.contiguous()]
+    if len(ws) == 3:
+        ws = [t if t.data_ptr() % 16 == 0 else t.clone() for t in ws]
+    # the caller's own frequency tensor (not a converted temporary) can key a memoised table
+    own = inv_freq is not None and inv_freq.device == x.device and inv_freq.dtype == torch.float32 and inv_freq.is_contiguous()
+    inv = inv_freq if inv_freq is None or own else inv_freq.to(device=x.device, dtype=torch.float32).contiguous()
+    table, ready = _rope_table_ws(T, D, pos0, x, inv, own)
+    p2, info = into if into is not None else (None, None)
+    return L.native().qkv_rope(x, ws, inv, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps, table,
+                               bool(ready), p2, info, L.stream_of(x))
 
 
 @torch.library.custom_op("mote::qkv_rope", mutates_args=())
@@ -393,22 +330,7 @@ def _linear_wgrad(a: torch.Tensor, x: torch.Tensor, dtype: torch.dtype) -> torch
     and K multiples of 64 (operands whose rows are not unit-stride and 16-byte aligned are copied first)."""
     if not a.is_cuda:
         raise RuntimeError("mote::linear_wgrad needs the HIP library and an MI355X")
-    ok = lambda t: t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
-    a = a if ok(a) else a.contiguous()
-    x = x if ok(x) else x.contiguous()
-    M, N = a.shape
-    K = x.shape[1]
-    dw = torch.empty(N, K, device=a.device, dtype=dtype)
-    args = L.LinearWgradArgs()
-    args.dtype, args.dw_dtype, args.M, args.N, args.K = L.dtype_code(a), L.dtype_code(dw), M, N, K
-    args.a, args.a_sr = a.data_ptr(), a.stride(0)
-    args.x, args.x_sr = x.data_ptr(), x.stride(0)
-    args.dw, args.dw_sr = dw.data_ptr(), dw.stride(0)
-    nbytes = int(L.lib().mote_linear_wgrad_workspace(args))
-    ws = torch.empty(max(nbytes, 16), device=a.device, dtype=torch.uint8)
-    args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
-    L.check(L.lib().mote_linear_wgrad(args, L.stream_of(a)), "mote_linear_wgrad")
-    return dw
+    return L.native().linear_wgrad(a, x, dtype, L.stream_of(a))
 
 
 @_linear_wgrad.register_fake
