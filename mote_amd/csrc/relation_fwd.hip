@@ -29,8 +29,10 @@
 
 namespace mote {
 
-template <typename T, int DP, int BN, int NW>
+// The register-staged form: bf16 rows 2^24 or more elements apart, past the tile kernels' 32-bit offsets.
+template <int DP, int BN, int NW>
 __global__ void __launch_bounds__(NW * 64) relation_fwd_kernel(const FwdParams p) {
+  using T = bf16_t;
   using E = Elem<T>;
   using Frag = typename E::Frag;
   constexpr int NTH = NW * 64;
@@ -40,7 +42,7 @@ __global__ void __launch_bounds__(NW * 64) relation_fwd_kernel(const FwdParams p
   constexpr int BM = NW * 32;
   constexpr int EPC = 16 / sizeof(T);         // elements per 16-byte chunk
   constexpr int KLD = DP + EPC;               // Ks row stride (elements): +16 bytes against bank conflicts
-  constexpr int VLD = BN + (sizeof(T) == 2 ? 8 : 4);
+  constexpr int VLD = BN + 8;
   constexpr int CPR = DP / EPC;               // chunks per row
   constexpr int KCH = BN * CPR;               // K chunks per block
   constexpr int KCT = (KCH + NTH - 1) / NTH;
@@ -167,30 +169,18 @@ __global__ void __launch_bounds__(NW * 64) relation_fwd_kernel(const FwdParams p
       const int it = tid + c * NTH;
       if (it < VIT) {
         const int kq = it % (BN / 4), cc = it / (BN / 4);
-        if constexpr (sizeof(T) == 2) {
-          // 8 head-dim rows x 4 keys: rows cc*8 + e, columns 4kq .. 4kq+3
+        // 8 head-dim rows x 4 keys: rows cc*8 + e, columns 4kq .. 4kq+3
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int w = e >> 1, sh = (e & 1) * 16;
-            const uint32_t a0 = (vreg[c][0].w[w] >> sh) & 0xffffu;
-            const uint32_t a1 = (vreg[c][1].w[w] >> sh) & 0xffffu;
-            const uint32_t a2 = (vreg[c][2].w[w] >> sh) & 0xffffu;
-            const uint32_t a3 = (vreg[c][3].w[w] >> sh) & 0xffffu;
-            uint2 v;
-            v.x = a0 | (a1 << 16);
-            v.y = a2 | (a3 << 16);
-            *reinterpret_cast<uint2*>(&Vt[(cc * 8 + e) * VLD + 4 * kq]) = v;
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            uint4 v;
-            v.x = vreg[c][0].w[e];
-            v.y = vreg[c][1].w[e];
-            v.z = vreg[c][2].w[e];
-            v.w = vreg[c][3].w[e];
-            *reinterpret_cast<uint4*>(&Vt[(cc * 4 + e) * VLD + 4 * kq]) = v;
-          }
+        for (int e = 0; e < 8; ++e) {
+          const int w = e >> 1, sh = (e & 1) * 16;
+          const uint32_t a0 = (vreg[c][0].w[w] >> sh) & 0xffffu;
+          const uint32_t a1 = (vreg[c][1].w[w] >> sh) & 0xffffu;
+          const uint32_t a2 = (vreg[c][2].w[w] >> sh) & 0xffffu;
+          const uint32_t a3 = (vreg[c][3].w[w] >> sh) & 0xffffu;
+          uint2 v;
+          v.x = a0 | (a1 << 16);
+          v.y = a2 | (a3 << 16);
+          *reinterpret_cast<uint2*>(&Vt[(cc * 8 + e) * VLD + 4 * kq]) = v;
         }
       }
     }
@@ -320,17 +310,7 @@ __global__ void __launch_bounds__(NW * 64) relation_fwd_kernel(const FwdParams p
         if (d0 < D) {
           const Frag kr = E::load8(kbase + int64_t(qa) * p.k_sr + d0);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            float a, b;
-            if constexpr (sizeof(T) == 2) {
-              a = (float)qf[s][ks].v[j];
-              b = (float)kr.v[j];
-            } else {
-              a = qf[s][ks].v[j];
-              b = kr.v[j];
-            }
-            ud = fmaf(a, b, ud);
-          }
+          for (int j = 0; j < 8; ++j) ud = fmaf((float)qf[s][ks].v[j], (float)kr.v[j], ud);
         }
       }
     }
@@ -352,14 +332,10 @@ __global__ void __launch_bounds__(NW * 64) relation_fwd_kernel(const FwdParams p
         ib[r] = oacc[dt][s][r] * inv_l;
         yv[r] = (1.0f - gate) * E::to_f(irow[d0 + r]) + gate * ib[r];
       }
-      if constexpr (sizeof(T) == 2) {
-        uint2 pk;
-        pk.x = uint32_t(f2bf(yv[0])) | (uint32_t(f2bf(yv[1])) << 16);
-        pk.y = uint32_t(f2bf(yv[2])) | (uint32_t(f2bf(yv[3])) << 16);
-        *reinterpret_cast<uint2*>(yrow + d0) = pk;
-      } else {
-        *reinterpret_cast<float4*>(yrow + d0) = make_float4(yv[0], yv[1], yv[2], yv[3]);
-      }
+      uint2 pk;
+      pk.x = uint32_t(f2bf(yv[0])) | (uint32_t(f2bf(yv[1])) << 16);
+      pk.y = uint32_t(f2bf(yv[2])) | (uint32_t(f2bf(yv[3])) << 16);
+      *reinterpret_cast<uint2*>(yrow + d0) = pk;
       *reinterpret_cast<float4*>(brow + d0) = make_float4(ib[0], ib[1], ib[2], ib[3]);
     }
     if (lg == 0) {
@@ -900,20 +876,22 @@ __global__ void __launch_bounds__(256) relation_fwd_merge_kernel(const FwdParams
 // ------------------------------------------------------------------------------------------------
 // host launcher
 // ------------------------------------------------------------------------------------------------
-template <typename T, int DP, int BN, int NW>
+template <int DP, int NW>
 static void launch_fwd_t(const FwdParams& fp, int nblocks, hipStream_t stream) {
-  hipLaunchKernelGGL((relation_fwd_kernel<T, DP, BN, NW>), dim3(nblocks), dim3(NW * 64), 0, stream, fp);
+  hipLaunchKernelGGL((relation_fwd_kernel<DP, 64, NW>), dim3(nblocks), dim3(NW * 64), 0, stream, fp);
 }
 
-template <typename T, int BN, int NW>
+template <int NW>
 static void launch_fwd_dp(const FwdParams& fp, int DP, int nblocks, hipStream_t stream) {
   switch (DP) {
-    case 32: launch_fwd_t<T, 32, BN, NW>(fp, nblocks, stream); break;
-    case 64: launch_fwd_t<T, 64, BN, NW>(fp, nblocks, stream); break;
-    case 96: launch_fwd_t<T, 96, BN, NW>(fp, nblocks, stream); break;
-    default: launch_fwd_t<T, 128, BN, NW>(fp, nblocks, stream); break;
+    case 32: launch_fwd_t<32, NW>(fp, nblocks, stream); break;
+    case 64: launch_fwd_t<64, NW>(fp, nblocks, stream); break;
+    case 96: launch_fwd_t<96, NW>(fp, nblocks, stream); break;
+    default: launch_fwd_t<128, NW>(fp, nblocks, stream); break;
   }
 }
+
+void launch_fwd_f32(FwdParams fp, int DP, hipStream_t stream);  // relation_fwd_f32.hip
 
 static bool view_ok(const mote_view& v) { return v.data != nullptr; }
 
@@ -1064,19 +1042,13 @@ int launch_fwd(const mote_relation_fwd_args* a, hipStream_t stream) {
   } else if (a->dtype == MOTE_BF16) {
     if (wide) {
       fp.nqb = nqb4;
-      launch_fwd_dp<bf16_t, 64, 4>(fp, DP, int(units * fp.nqb), stream);
+      launch_fwd_dp<4>(fp, DP, int(units * fp.nqb), stream);
     } else {
       fp.nqb = (a->TQ + 63) / 64;
-      launch_fwd_dp<bf16_t, 64, 2>(fp, DP, int(units * fp.nqb), stream);
+      launch_fwd_dp<2>(fp, DP, int(units * fp.nqb), stream);
     }
   } else {
-    if (wide) {
-      fp.nqb = nqb4;
-      launch_fwd_dp<float, 32, 4>(fp, DP, int(units * fp.nqb), stream);
-    } else {
-      fp.nqb = (a->TQ + 63) / 64;
-      launch_fwd_dp<float, 32, 2>(fp, DP, int(units * fp.nqb), stream);
-    }
+    launch_fwd_f32(fp, DP, stream);
   }
   return check_launch("relation_fwd");
 }

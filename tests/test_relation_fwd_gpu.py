@@ -43,6 +43,28 @@ def test_fp32_forward_matches_oracle(cuda, D, TQ, S):
     assert torch.allclose(y.cpu().double(), yr, atol=2e-4, rtol=1e-3)
 
 
+# fp32 on staged tiles: every tile dim and padded ones, lengths around the key blocks (32 keys beyond
+# dh 64, else 64) and the 64-row query blocks, cached prefixes, strided views whose other columns hold NaN
+@pytest.mark.parametrize("D", [8, 32, 40, 64, 104, 128])
+@pytest.mark.parametrize("B,H,TQ,S", [(1, 1, 31, 0), (2, 2, 33, 0), (1, 2, 64, 1), (1, 1, 65, 63), (2, 1, 129, 30)])
+def test_fp32_tile_edges(cuda, D, B, H, TQ, S):
+    from mote_amd.flash_relation import flash_relation
+
+    print(f"case fp32 tiles D={D} B={B} H={H} TQ={TQ} S={S}", flush=True)
+    g = torch.Generator().manual_seed(D + TQ)
+
+    def window(T):
+        buf = torch.full((B, T, H, D + 4), float("nan"))
+        buf[..., :D] = torch.randn(B, T, H, D, generator=g) * 0.7
+        return buf.to(cuda)[..., :D].transpose(1, 2)
+
+    p1, p2, info = window(TQ), window(S + TQ), window(S + TQ)
+    lam = torch.tensor(0.4)
+    y, gate = flash_relation(p1, p2, info, lam.to(cuda), 2.0, S)
+    yr, gr = O.relation_reference(*(t.cpu().double() for t in (p1, p2, info)), lam.double(), 2.0, S, dtype=torch.float64)
+    assert rel_err(y, yr) < 1e-5 and rel_err(gate, gr) < 1e-5
+
+
 @pytest.mark.parametrize("D", [96, 112, 24])
 def test_odd_head_dims(cuda, D):
     from mote_amd.flash_relation import flash_relation
