@@ -242,7 +242,9 @@ relation_fwd_f32_kernel(const FwdParams p) {
     const bool qv = qi < TQs;
     const int qa = qs + qi;
     const bool has = lt > 0.f;
-    const float lse = has ? (mm + __log2f(lt)) * kLn2 : kNegInf;
+    // the running bound starts at 0, so the logarithm holds most of lse: its exponent is added exactly
+    const float lse = has ? (mm + (float)__builtin_amdgcn_frexp_expf(lt) + __log2f(__builtin_amdgcn_frexp_mantf(lt))) * kLn2
+                          : kNegInf;
     const float inv_l = has ? 1.0f / lt : 0.f;
     float ud = 0.f;
     if (qv) {
