@@ -20,15 +20,16 @@ struct BwdParams {
   // workspace
   void* wq;      // [BH][TQp][DP]  P1 rows                      (register-staged kernels)
   void* wdib;    // [BH][TQp][DP]  dI-bar rows                  (both paths)
-  void* wqT;     // [BH][DP][TQp]  P1 transposed                (register-staged kernels)
-  void* wdibT;   // [BH][DP][TQp]  dI-bar transposed            (register-staged kernels)
+  void* wqT;     // [BH][DP][TQp]  P1 transposed                (register-staged bf16 kernels)
+  void* wdibT;   // [BH][DP][TQp]  dI-bar transposed            (register-staged bf16 kernels)
   float* lse2;   // [BH][TQp]                                   (register-staged kernels)
   float* cvec;   // [BH][TQp]      dA - Delta                   (register-staged kernels)
   float* stat;   // [BH][TQp / 64][128]: lse2 of the block's 64 rows, then c = dA - Delta (tile kernels)
   float* duii;   // [BH][TQp]
-  float* dp1acc; // [BH][TQ][D]                                 (register-staged kernels)
+  float* dp1acc; // [BH][TQ][D]                                 (register-staged kernels; fp32 without dut)
   float* dlam_part;  // [BH][TQp / 64]
-  void* dut;     // [BH][npairs][4 waves][2 query tiles][64 lanes][8] bf16: dU as the key kernel's waves hold it (tile kernels)
+  void* dut;     // [BH][npairs][4 waves][2 query tiles][64 lanes][8] bf16: dU as the key kernel's waves hold it (tile kernels);
+                 // fp32: [BH][npairs][4 query tiles][4 key tiles][16 keys][16 queries], or null
   int64_t npairs;    // (query block, key block) pairs per (batch, head), PairTable::total
   int* kvq;      // control words of the fused key + query launch, or null: the two launches (tile kernels)
   int kvq_nq;    // its queues: 8, 4, 2 or 1, dividing B H
@@ -88,5 +89,10 @@ __device__ __forceinline__ void dlam_sum(const float* part, int n, float* out, f
 // bf16: the atomic-free tile kernels (dP2 / dI~ key-stationary, then dP1
 // query-stationary), for the stages selected in `stages` (MOTE_BWD_KEYS, MOTE_BWD_QUERIES).
 void launch_bwd_tiles(const BwdParams& p, int stages, hipStream_t stream);
+
+// fp32 (relation_bwd_f32.hip), DP = padded_dim(D): the key blocks, storing dU where p.dut is set (else
+// adding dP1 into the accumulator if with_dq), and the dP1 and dlam stage that follows a stored dU.
+void launch_bwd_keys_f32(const BwdParams& p, int DP, bool with_dq, hipStream_t stream);
+void launch_bwd_dq_f32(const BwdParams& p, int DP, hipStream_t stream);
 
 }  // namespace mote

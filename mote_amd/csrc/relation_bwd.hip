@@ -6,7 +6,7 @@
 //      dI-bar = g dY, dg = dY.(I-bar - I~_i), dA = dg g (1-g), Delta = dI-bar.I-bar,
 //      dU_ii = -dA S (1-S) / tau, dlam partial = -sum dA ln(i+1)
 //    and the operand copies the main kernels stage from: Q and dI-bar padded to the kernel's head
-//    dim, row-major and transposed (head-dim major), c = dA - Delta, lse in log2 units (+inf for
+//    dim, row-major and (bf16) transposed (head-dim major), c = dA - Delta, lse in log2 units (+inf for
 //    padding rows and rows without a past, which zeroes their weights), and the fp32 dP1
 //    accumulator initialised with the Self part dU_ii P2_i / sqrt(D).
 // 2. key blocks (one workgroup per 64 keys of one (batch, head), 4 waves x 16 keys, longest
@@ -33,7 +33,7 @@ namespace mote {
 // 1. rows
 // ------------------------------------------------------------------------------------------------
 // LEAN (tile kernels): only dI-bar rows, the per-block stats, dU_ii and the dlam partials; the
-// register-staged kernels also need the P1 copies, both transposes and the dP1 accumulator.
+// others also need the P1 copies and the dP1 accumulator, bf16 both transposes.
 template <typename T, int DP, bool LEAN>
 __global__ void __launch_bounds__(256) bwd_rows_kernel(const BwdParams p) {
   using E = Elem<T>;
@@ -42,8 +42,9 @@ __global__ void __launch_bounds__(256) bwd_rows_kernel(const BwdParams p) {
   constexpr int NCH = kRowBlock * CPR;      // chunks per block
   constexpr int CT = (NCH + 255) / 256;     // chunks per thread
   constexpr int LD = DP + EPC;              // LDS row stride (elements)
-  __shared__ __align__(16) T sq[LEAN ? 1 : kRowBlock * LD];
-  __shared__ __align__(16) T sd[LEAN ? 1 : kRowBlock * LD];
+  constexpr bool TR = !LEAN && sizeof(T) == 2;  // with the transposed copies
+  __shared__ __align__(16) T sq[TR ? kRowBlock * LD : 1];
+  __shared__ __align__(16) T sd[TR ? kRowBlock * LD : 1];
   __shared__ float part[3][kRowBlock][CPR + 1];
   __shared__ float sdu[kRowBlock];
   __shared__ float sred[kRowBlock];
@@ -121,11 +122,11 @@ __global__ void __launch_bounds__(256) bwd_rows_kernel(const BwdParams p) {
     part[0][r][cc] = dgate;
     part[1][r][cc] = delta;
     part[2][r][cc] = uii;
-    if constexpr (!LEAN) {
+    if constexpr (TR) {
       store_chunk(&sq[r * LD + d0], cq);
       store_chunk(&sd[r * LD + d0], cd);
-      store_chunk(wq + r * DP + d0, cq);
     }
+    if constexpr (!LEAN) store_chunk(wq + r * DP + d0, cq);
     store_chunk(wd + r * DP + d0, cd);
   }
   __syncthreads();
@@ -168,6 +169,7 @@ __global__ void __launch_bounds__(256) bwd_rows_kernel(const BwdParams p) {
   // pass 2: dP1 accumulator initialised with the Self part dU_ii P2_i / sqrt(D)
 #pragma unroll
   for (int c = 0; c < (LEAN ? 0 : CT); ++c) {
+    if (!p.dp1acc) break;  // fp32 with a stored dU: its dP1 stage adds the Self part
     const int idx = tid + 256 * c;
     if (idx >= NCH) break;
     const int r = idx / CPR, cc = idx % CPR;
@@ -183,7 +185,7 @@ __global__ void __launch_bounds__(256) bwd_rows_kernel(const BwdParams p) {
           make_float4(f * E::to_f(ek[e]), f * E::to_f(ek[e + 1]), f * E::to_f(ek[e + 2]), f * E::to_f(ek[e + 3]));
   }
   // transposed copies: row d holds the 64 rows of this block
-  if constexpr (!LEAN) {
+  if constexpr (TR) {
     T* wqT = reinterpret_cast<T*>(p.wqT) + int64_t(bh) * DP * p.TQp + i0;
     T* wdT = reinterpret_cast<T*>(p.wdibT) + int64_t(bh) * DP * p.TQp + i0;
     constexpr int CH = DP * kRowBlock / EPC;
@@ -192,15 +194,9 @@ __global__ void __launch_bounds__(256) bwd_rows_kernel(const BwdParams p) {
       Chunk vq, vd;
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
-        if constexpr (sizeof(T) == 2) {
-          const int r0 = (cc * 8 + 2 * w) * LD + d;
-          vq.w[w] = uint32_t(sq[r0]) | (uint32_t(sq[r0 + LD]) << 16);
-          vd.w[w] = uint32_t(sd[r0]) | (uint32_t(sd[r0 + LD]) << 16);
-        } else {
-          const int r0 = (cc * 4 + w) * LD + d;
-          vq.w[w] = __float_as_uint(sq[r0]);
-          vd.w[w] = __float_as_uint(sd[r0]);
-        }
+        const int r0 = (cc * 8 + 2 * w) * LD + d;
+        vq.w[w] = uint32_t(sq[r0]) | (uint32_t(sq[r0 + LD]) << 16);
+        vd.w[w] = uint32_t(sd[r0]) | (uint32_t(sd[r0 + LD]) << 16);
       }
       store_chunk(wqT + int64_t(d) * p.TQp + cc * EPC, vq);
       store_chunk(wdT + int64_t(d) * p.TQp + cc * EPC, vd);
@@ -220,10 +216,10 @@ __global__ void __launch_bounds__(256) bwd_rows_kernel(const BwdParams p) {
 // ------------------------------------------------------------------------------------------------
 // Transposed staging of a [64 keys x DP] block into LDS as [DP][LDT] (head-dim major):
 // item = 4 consecutive keys x one 16-byte chunk of the head dim.
-template <typename T, int DP, int NTH>
-__device__ __forceinline__ void stage_transposed(T* dst, int LDT, const T* base, int64_t row_stride, int j0, int nrows,
-                                                 int D, int tid) {
-  constexpr int EPC = 16 / sizeof(T);
+template <int DP, int NTH>
+__device__ __forceinline__ void stage_transposed(bf16_t* dst, int LDT, const bf16_t* base, int64_t row_stride, int j0,
+                                                 int nrows, int D, int tid) {
+  constexpr int EPC = 8;
   constexpr int ITEMS = (64 / 4) * (DP / EPC);
   for (int it = tid; it < ITEMS; it += NTH) {
     const int kq = it % 16, cc = it / 16;
@@ -233,41 +229,31 @@ __device__ __forceinline__ void stage_transposed(T* dst, int LDT, const T* base,
       const int j = j0 + 4 * kq + r;
       v[r] = (j < nrows && cc * EPC < D) ? load_chunk(base + int64_t(j) * row_stride + cc * EPC) : zero_chunk();
     }
-    if constexpr (sizeof(T) == 2) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int w = e >> 1, sh = (e & 1) * 16;
-        uint2 o;
-        o.x = ((v[0].w[w] >> sh) & 0xffffu) | (((v[1].w[w] >> sh) & 0xffffu) << 16);
-        o.y = ((v[2].w[w] >> sh) & 0xffffu) | (((v[3].w[w] >> sh) & 0xffffu) << 16);
-        *reinterpret_cast<uint2*>(&dst[(cc * 8 + e) * LDT + 4 * kq]) = o;
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        uint4 o;
-        o.x = v[0].w[e];
-        o.y = v[1].w[e];
-        o.z = v[2].w[e];
-        o.w = v[3].w[e];
-        *reinterpret_cast<uint4*>(&dst[(cc * 4 + e) * LDT + 4 * kq]) = o;
-      }
+    for (int e = 0; e < 8; ++e) {
+      const int w = e >> 1, sh = (e & 1) * 16;
+      uint2 o;
+      o.x = ((v[0].w[w] >> sh) & 0xffffu) | (((v[1].w[w] >> sh) & 0xffffu) << 16);
+      o.y = ((v[2].w[w] >> sh) & 0xffffu) | (((v[3].w[w] >> sh) & 0xffffu) << 16);
+      *reinterpret_cast<uint2*>(&dst[(cc * 8 + e) * LDT + 4 * kq]) = o;
     }
   }
 }
 
-template <typename T, int DP, int BM, bool WITH_DQ>
+// bf16 rows too far apart for the tile kernels (fp32: relation_bwd_f32.hip).
+template <int DP, bool WITH_DQ>
 __global__ void __launch_bounds__(256) bwd_keys_kernel(const BwdParams p) {
+  using T = bf16_t;
   using E = Elem<T>;
   using Frag = typename E::Frag;
-  constexpr int BN = 64;
+  constexpr int BM = 64, BN = 64;
   constexpr int KS = DP / 32;
   constexpr int DT = DP / 16;
   constexpr int QT = BM / 16;           // query tiles per block
   constexpr int EPC = 16 / sizeof(T);
   constexpr int PADE = 16 / sizeof(T);  // 16-byte row padding
   constexpr int QLD = DP + PADE;        // Qs / Ds row stride
-  constexpr int TLD = BM + (sizeof(T) == 2 ? 8 : 4);   // QTs / DTs row stride
+  constexpr int TLD = BM + 8;           // QTs / DTs row stride
   constexpr int ULD = BN + PADE;        // dUs row stride
   constexpr int KLD = BN + PADE;        // KTs row stride
   __shared__ __align__(16) T Qs[BM * QLD];
@@ -304,7 +290,7 @@ __global__ void __launch_bounds__(256) bwd_keys_kernel(const BwdParams p) {
       vf[ks] = E::zero();
     }
   }
-  if constexpr (WITH_DQ) stage_transposed<T, DP, 256>(KTs, KLD, kbase, p.k_sr, k0, p.TK, D, tid);
+  if constexpr (WITH_DQ) stage_transposed<DP, 256>(KTs, KLD, kbase, p.k_sr, k0, p.TK, D, tid);
 
   const int nqb = p.TQp / BM;
   const int qb_lo = max(0, k0 + 1 - p.q_start) / BM;
@@ -596,7 +582,7 @@ __global__ void __launch_bounds__(128) bwd_queries_kernel(const BwdParams p) {
       store_chunk(&Vs[row * KLD + cc * EPC], ok ? load_chunk(vbase + int64_t(j) * p.v_sr + cc * EPC) : zero_chunk());
     }
     if constexpr (BN == 64) {
-      stage_transposed<T, DP, NTH>(KTs, TLD, kbase, p.k_sr, j0, p.TK, D, tid);
+      stage_transposed<DP, NTH>(KTs, TLD, kbase, p.k_sr, j0, p.TK, D, tid);
     } else {
       // 32-key blocks (fp32): the same transposed staging over 32 rows
       constexpr int ITEMS = (BN / 4) * (DP / EPC);
@@ -610,17 +596,9 @@ __global__ void __launch_bounds__(128) bwd_queries_kernel(const BwdParams p) {
         }
 #pragma unroll
         for (int e = 0; e < EPC; ++e) {
-          if constexpr (sizeof(T) == 4) {
-            uint4 o;
-            o.x = v[0].w[e]; o.y = v[1].w[e]; o.z = v[2].w[e]; o.w = v[3].w[e];
-            *reinterpret_cast<uint4*>(&KTs[(cc * 4 + e) * TLD + 4 * kq]) = o;
-          } else {
-            const int w = e >> 1, sh = (e & 1) * 16;
-            uint2 o;
-            o.x = ((v[0].w[w] >> sh) & 0xffffu) | (((v[1].w[w] >> sh) & 0xffffu) << 16);
-            o.y = ((v[2].w[w] >> sh) & 0xffffu) | (((v[3].w[w] >> sh) & 0xffffu) << 16);
-            *reinterpret_cast<uint2*>(&KTs[(cc * 8 + e) * TLD + 4 * kq]) = o;
-          }
+          uint4 o;
+          o.x = v[0].w[e]; o.y = v[1].w[e]; o.z = v[2].w[e]; o.w = v[3].w[e];
+          *reinterpret_cast<uint4*>(&KTs[(cc * 4 + e) * TLD + 4 * kq]) = o;
         }
       }
     }
@@ -754,6 +732,13 @@ static bool use_tiles(const mote_relation_bwd_args* a) {
   return int64_t(a->B) * a->H * PairTable::total(a->TQ, a->q_start) <= (int64_t(8) << 30) / 8192;
 }
 
+// fp32: whether the key blocks store dU (16 KB per 64 x 64 pair) for the dP1 stage instead of adding dP1
+// with atomics or recomputing it; both modes, the results are reproducible either way. Up to 2 GiB of it
+// (H 8: 11 K rows), so that a length that fitted the card before still does.
+static bool f32_stores_du(const mote_relation_bwd_args* a) {
+  return a->dtype == MOTE_F32 && int64_t(a->B) * a->H * PairTable::total(a->TQ, a->q_start) <= (int64_t(2) << 30) / 16384;
+}
+
 static WsLayout ws_layout(const mote_relation_bwd_args* a) {
   const size_t es = a->dtype == MOTE_BF16 ? 2 : 4;
   const size_t BH = size_t(a->B) * a->H;
@@ -770,11 +755,17 @@ static WsLayout ws_layout(const mote_relation_bwd_args* a) {
     w.kvq = o; o = align256(o + (kKvqCounts + BH * (TQp / kRowBlock)) * 4);
   } else {
     w.wq = o; o = align256(o + BH * TQp * DP * es);
-    w.wqT = o; o = align256(o + BH * TQp * DP * es);
-    w.wdibT = o; o = align256(o + BH * TQp * DP * es);
+    if (a->dtype == MOTE_BF16) {
+      w.wqT = o; o = align256(o + BH * TQp * DP * es);
+      w.wdibT = o; o = align256(o + BH * TQp * DP * es);
+    }
     w.lse2 = o; o = align256(o + BH * TQp * 4);
     w.cvec = o; o = align256(o + BH * TQp * 4);
-    w.dp1acc = o; o = align256(o + BH * size_t(a->TQ) * a->D * 4);
+    if (f32_stores_du(a)) {
+      w.dut = o; o = align256(o + BH * size_t(PairTable::total(a->TQ, a->q_start)) * 16384);
+    } else {
+      w.dp1acc = o; o = align256(o + BH * size_t(a->TQ) * a->D * 4);
+    }
   }
   w.duii = o; o = align256(o + BH * TQp * 4);
   w.dlam_part = o; o = align256(o + BH * (TQp / kRowBlock) * 4);
@@ -784,19 +775,28 @@ static WsLayout ws_layout(const mote_relation_bwd_args* a) {
 
 size_t bwd_workspace_bytes(const mote_relation_bwd_args* a) { return ws_layout(a).total; }
 
-// Register-staged kernels (fp32, and bf16 rows too far apart for the tile kernels).
+// fp32, and bf16 off the tile kernels (register-staged).
 template <typename T, int DP>
 static void launch_bwd_t(const BwdParams& p, bool deterministic, int stages, hipStream_t stream) {
   const int BH = p.B * p.H;
   if (stages & MOTE_BWD_ROWS)
     hipLaunchKernelGGL((bwd_rows_kernel<T, DP, false>), dim3(p.TQp / kRowBlock, BH), dim3(256), 0, stream, p);
-  const int nkb = (p.TK + 63) / 64;
-  constexpr int BM = sizeof(T) == 2 ? 64 : 32;
   if (stages & MOTE_BWD_KEYS) {
-    if (!deterministic)
-      hipLaunchKernelGGL((bwd_keys_kernel<T, DP, BM, true>), dim3(nkb * BH), dim3(256), 0, stream, p);
-    else
-      hipLaunchKernelGGL((bwd_keys_kernel<T, DP, BM, false>), dim3(nkb * BH), dim3(256), 0, stream, p);
+    if constexpr (sizeof(T) == 4) {
+      launch_bwd_keys_f32(p, DP, !deterministic, stream);
+    } else {
+      const int nkb = (p.TK + 63) / 64;
+      if (!deterministic)
+        hipLaunchKernelGGL((bwd_keys_kernel<DP, true>), dim3(nkb * BH), dim3(256), 0, stream, p);
+      else
+        hipLaunchKernelGGL((bwd_keys_kernel<DP, false>), dim3(nkb * BH), dim3(256), 0, stream, p);
+    }
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (p.dut) {  // dP1 and dlam; nothing left to finish
+      if (stages & MOTE_BWD_QUERIES) launch_bwd_dq_f32(p, DP, stream);
+      return;
+    }
   }
   if ((stages & MOTE_BWD_QUERIES) && deterministic) {
     constexpr int BNQ = sizeof(T) == 2 ? 64 : 32;
@@ -885,7 +885,12 @@ int launch_bwd(const mote_relation_bwd_args* a, hipStream_t stream) {
     p.wq = ws + w.wq; p.wqT = ws + w.wqT; p.wdibT = ws + w.wdibT;
     p.lse2 = reinterpret_cast<float*>(ws + w.lse2);
     p.cvec = reinterpret_cast<float*>(ws + w.cvec);
-    p.dp1acc = reinterpret_cast<float*>(ws + w.dp1acc);
+    if (f32_stores_du(a)) {
+      p.dut = ws + w.dut;
+      p.npairs = PairTable::total(a->TQ, a->q_start);
+    } else {
+      p.dp1acc = reinterpret_cast<float*>(ws + w.dp1acc);
+    }
   }
   p.B = a->B; p.H = a->H; p.TQ = a->TQ; p.TK = a->TK; p.D = a->D; p.q_start = a->q_start;
   p.TQp = (a->TQ + kRowBlock - 1) / kRowBlock * kRowBlock;

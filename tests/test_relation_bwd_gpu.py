@@ -73,6 +73,34 @@ def test_fp32_grads_match_oracle(cuda, D, TQ, S, det):
         assert torch.allclose(a.cpu().double(), b, atol=3e-4, rtol=2e-3), n
 
 
+@pytest.mark.parametrize("det", [False, True])
+@pytest.mark.parametrize("D,TQ,S", [(64, 1, 0), (64, 31, 1), (64, 33, 31), (96, 32, 32), (128, 65, 15), (32, 95, 64), (40, 64, 7),
+                                    (104, 129, 0), (64, 1, 63)])
+def test_fp32_key_block_edges(cuda, D, TQ, S, det):
+    """The fp32 kernels' 32-key, 64-query and 32-query blocks of 16-row wave parts at their edges, both modes."""
+    t = _inputs(2, 3, TQ, S, D, torch.float32, seed=D + TQ + S)
+    _check(_grads(*t, S, deterministic=det), _oracle_grads(*t, S), 1e-5, *t, S)
+
+
+@pytest.mark.parametrize("det", [False, True])
+@pytest.mark.parametrize("D", [32, 40])
+def test_fp32_beyond_the_stored_du(cuda, D, det):
+    """22400 heads of 130 queries: more dU than is stored (2 GiB), so dP1 by atomics or recomputed; a few
+    heads against the same heads by themselves, whose dU is stored (the bound of the one-pass / two-pass
+    agreement: both sum the same fp32 terms in another order)."""
+    S, T, H = 5, 130, 22400
+    mk = lambda n: torch.randn(1, H, n, D, device="cuda").requires_grad_(True)
+    torch.manual_seed(D)
+    p1, p2, info, dy = mk(T), mk(S + T), mk(S + T), mk(T).detach()
+    lam = torch.tensor(0.5, device="cuda", requires_grad=True)
+    big = _grads(p1, p2, info, lam, dy, S, det)
+    for h in (0, 11111, H - 3):
+        few = [t.detach()[:, h:h + 3].clone().requires_grad_(True) for t in (p1, p2, info)]
+        got = _grads(*few, lam, dy[:, h:h + 3], S, det)
+        for a, b, n in zip(big, got, NAMES[:3]):
+            assert torch.allclose(a[:, h:h + 3], b, atol=3e-5, rtol=1e-5), n
+
+
 @pytest.mark.parametrize("D", [96, 112, 24])
 def test_odd_head_dim_grads(cuda, D):
     p1, p2, info, lam, dy = _inputs(1, 2, 90, 0, D, torch.float32)
