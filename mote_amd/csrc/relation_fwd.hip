@@ -478,14 +478,14 @@ struct FwdTileShape {
   static constexpr int LDS = NSTG * STAGE;
 };
 
-// One (query block, sequence, head) of the tile forward (or one piece of its key range when split),
-// by its block id (the launch order: head fastest, then (when split) the pieces, then query blocks
-// longest first); every wave of the workgroup calls it.
 // The pieces of a query block of nkb key blocks.
 __device__ __forceinline__ int fwd_pieces(const FwdParams& p, int nkb) {
   return p.part != nullptr && nkb > p.split_c ? (nkb + p.split_c - 1) / p.split_c : 1;
 }
 
+// One (query block, sequence, head) of the tile forward (or one piece of its key range when split),
+// by its block id (the launch order: head fastest, then (when split) the pieces, then query blocks
+// longest first); every wave of the workgroup calls it.
 // PAD: head dims below DP (p.D, a multiple of 8). The queries' columns past D are zero, which keeps the
 // staged copies there (TileStager) out of the scores; I-bar columns past D are not stored.
 template <int DP, bool PAD>
