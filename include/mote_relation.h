@@ -110,15 +110,16 @@ int mote_relation_fwd(const mote_relation_fwd_args* args, void* stream);
  * dp2 and dinfo [B,H,TK,D] in `dtype` (any strides) and dlam (one fp32, overwritten).
  * bf16 (row strides below 2^24 elements) runs atomic-free kernels (key-stationary dp2/dinfo, then
  * query-stationary dp1): every result is bitwise reproducible whatever `deterministic` says.
- * Other shapes (fp32, longer row strides): `deterministic` != 0 selects the atomic-free pair of
- * kernels (the reference's MOTE_DETERMINISTIC_RELATION, flash_relation.py:51), 0 the one-pass
- * kernel with fp32 atomics for dp1.
+ * So does fp32 while its stored dU takes at most 2 GiB (16 KB per visible 64 x 64 pair).
+ * Other shapes (longer fp32, padded bf16 head dims beyond 8 GiB of dU, longer row strides):
+ * `deterministic` != 0 selects the atomic-free pair of kernels (the reference's
+ * MOTE_DETERMINISTIC_RELATION, flash_relation.py:51), 0 the one-pass kernel with fp32 atomics for dp1.
  * The workspace is caller-allocated device memory of at least mote_relation_bwd_workspace()
  * bytes; its contents on entry do not matter.
  * `stages` selects which launches run (MOTE_BWD_ROWS: per-row terms and operand copies;
  * MOTE_BWD_KEYS: the key-stationary kernel; MOTE_BWD_QUERIES: the query-stationary dp1 kernel,
- * where the path has one; MOTE_BWD_FINISH: dp1 cast and dlam, which the bf16 tile path computes in
- * its MOTE_BWD_QUERIES launch instead); 0 runs all of them. A caller that
+ * where the path has one; MOTE_BWD_FINISH: dp1 cast and dlam, which the atomic-free paths that store dU
+ * compute in their MOTE_BWD_QUERIES launch instead); 0 runs all of them. A caller that
  * splits them (to time or overlap them) issues them in that order on one stream with one workspace.
  * On the bf16 tile path with D <= 96, MOTE_BWD_KEYS and MOTE_BWD_QUERIES in one call run as one
  * launch (dp1 bit-identical to the separate launches, dp2 / dinfo the same terms added in another
