@@ -22,7 +22,7 @@
 // What bounds it: the two transposed fragment reads per pair of products (LDS), and for the narrow
 // widths the bytes of the two operands. 576 x 192 over 19,856 rows (the 192-wide layer's stacked
 // projections, 30 MB of operands): 18.0 us with the sum, against 110 us for the GEMM library's product;
-// 2304 x 768 over 4964 rows 34.2 us (514 TFLOP/s), library 49.
+// 2304 x 768 over 4964 rows 35.3 us (498 TFLOP/s), library 50; over 79,424 rows 351 us, library 524.
 #include "common.hpp"
 #include "params.hpp"
 #include "tiles.hpp"
