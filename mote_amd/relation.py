@@ -169,13 +169,14 @@ _ROPE_TABLES_MAX = 32
 
 
 def _rope_table_ws(T: int, D: int, pos0: int, x: torch.Tensor, inv: Optional[torch.Tensor],
-                   cacheable: bool) -> Tuple[torch.Tensor, int]:
+                   cacheable: bool) -> Tuple[torch.Tensor, int, Optional[tuple]]:
     """Workspace for mote_qkv_rope_fwd (mote_qkv_rope_workspace: a 32-bit cos / sin pair per position and
-    frequency) and whether it already holds the table (table_ready). `cacheable`: inv is the caller's own
-    frequency tensor (not a converted temporary)."""
+    frequency), whether it already holds the table (table_ready), and what _rope_table_keep takes once a
+    launch has filled it (None: not to be kept). `cacheable`: inv is the caller's own frequency tensor
+    (not a converted temporary)."""
     n = max(T * (D // 2) * 4 if inv is not None else 0, 16)
     if inv is None or not cacheable:
-        return torch.empty(n, device=x.device, dtype=torch.uint8), 0
+        return torch.empty(n, device=x.device, dtype=torch.uint8), 0, None
     key = (x.device, L.stream_of(x), inv.data_ptr(), T, pos0, D)
     hit = _ROPE_TABLES.get(key)
     # the entry holds the frequency tensor itself: its memory cannot be recycled for another tensor
@@ -184,15 +185,20 @@ def _rope_table_ws(T: int, D: int, pos0: int, x: torch.Tensor, inv: Optional[tor
     if torch.cuda.is_current_stream_capturing():
         if valid:
             _ROPE_TABLES_PINNED[hit[2].data_ptr()] = hit[2]
-            return hit[2], 1
-        return torch.empty(n, device=x.device, dtype=torch.uint8), 0
+            return hit[2], 1, None
+        return torch.empty(n, device=x.device, dtype=torch.uint8), 0, None
     if valid:
-        return hit[2], 1
-    if hit is None and len(_ROPE_TABLES) >= _ROPE_TABLES_MAX:
-        _ROPE_TABLES.pop(next(iter(_ROPE_TABLES)))  # a pinned table stays alive through the pin
+        return hit[2], 1, None
     ws = torch.empty(n, device=x.device, dtype=torch.uint8)
-    _ROPE_TABLES[key] = (inv, inv._version, ws)
-    return ws, 0
+    # a call without rows launches nothing, so it leaves the table unwritten
+    return ws, 0, (key, inv, inv._version, ws) if x.numel() else None
+
+
+def _rope_table_keep(key, inv, version, ws):
+    """Memoise a table whose launch was accepted: a refused call must not leave an unwritten one behind."""
+    if key not in _ROPE_TABLES and len(_ROPE_TABLES) >= _ROPE_TABLES_MAX:
+        _ROPE_TABLES.pop(next(iter(_ROPE_TABLES)), None)  # a pinned table stays alive through the pin
+    _ROPE_TABLES[key] = (inv, version, ws)
 
 
 def _qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps, into=None):
@@ -213,10 +219,13 @@ def _qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, no
     # the caller's own frequency tensor (not a converted temporary) can key a memoised table
     own = inv_freq is not None and inv_freq.device == x.device and inv_freq.dtype == torch.float32 and inv_freq.is_contiguous()
     inv = inv_freq if inv_freq is None or own else inv_freq.to(device=x.device, dtype=torch.float32).contiguous()
-    table, ready = _rope_table_ws(T, D, pos0, x, inv, own)
+    table, ready, fresh = _rope_table_ws(T, D, pos0, x, inv, own)
     p2, info = into if into is not None else (None, None)
-    return L.native().qkv_rope(x, ws, inv, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps, table,
-                               bool(ready), p2, info, L.stream_of(x))
+    out = L.native().qkv_rope(x, ws, inv, theta, n_heads, parity, pos0, keep_info, norm_w1, norm_w2, norm_eps, table,
+                              bool(ready), p2, info, L.stream_of(x))
+    if fresh is not None:
+        _rope_table_keep(*fresh)
+    return out
 
 
 @torch.library.custom_op("mote::qkv_rope", mutates_args=())
