@@ -405,6 +405,11 @@ static bool al16v(const void* ptr, int64_t s0, int64_t s1, int64_t s2) {
          (s2 * 2) % 16 == 0;
 }
 
+// Whether a view's rows of D elements lie apart (a row stride below D would write into the next row).
+static bool rows_apart(const mote_view& v, const mote_qkv_rope_args* a) {
+  return (a->T < 2 || v.stride_r >= a->D) && (a->H < 2 || v.stride_h >= a->D) && (a->B < 2 || v.stride_b >= a->D);
+}
+
 static int launch_qkv(const mote_qkv_rope_args* a, const void* w2, const void* wi, hipStream_t stream);
 
 int launch_qkv_rope_fwd(const mote_qkv_rope_args* a, hipStream_t stream) {
@@ -436,6 +441,8 @@ static int launch_qkv(const mote_qkv_rope_args* a, const void* w2, const void* w
   if (M > (int64_t(1) << 30)) return set_error(MOTE_ERR_SHAPE, "qkv_rope: %lld tokens", (long long)M);
   if (!a->x || !a->w || !w2 || !wi || !a->p1.data || !a->p2.data || !a->info.data)
     return set_error(MOTE_ERR_ARGUMENT, "qkv_rope: null pointer");
+  if (!rows_apart(a->p1, a) || !rows_apart(a->p2, a) || !rows_apart(a->info, a))
+    return set_error(MOTE_ERR_ARGUMENT, "qkv_rope: p1, p2 and info need strides of at least %d elements", a->D);
   if (a->B > 1 && a->x_sb != int64_t(a->T) * a->x_sr)
     return set_error(MOTE_ERR_ARGUMENT, "qkv_rope: x must hold its batches back to back (x_sb == T * x_sr)");
   if (a->x_sr >= (int64_t(1) << 23) || a->w_sr >= (int64_t(1) << 23))

@@ -267,6 +267,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> qkv_rope(const Tensor& x, con
                                                             const OptTensor& info_, int64_t stream) {
   const int64_t B = x.size(0), T = x.size(1), K = x.size(2), D = K / H;
   const at::ScalarType dt = x.scalar_type();
+  for (const OptTensor* t : {&p2_, &info_})  // the caller's memory: the kernel writes all of [B, H, T, D]
+    TORCH_CHECK(!t->has_value() || ((*t)->sizes() == at::IntArrayRef({B, H, T, D}) && (*t)->scalar_type() == dt &&
+                                    (*t)->device() == x.device()),
+                "qkv_rope: P2 and I~ must be [", B, ", ", H, ", ", T, ", ", D, "] in x's dtype on x's device");
   Tensor p1 = heads(B, T, H, D, x, dt);
   Tensor p2 = p2_ ? *p2_ : heads(B, T, H, D, x, dt), info = info_ ? *info_ : heads(B, T, H, D, x, dt);
   const bool norm = norm_w1.has_value();

@@ -689,6 +689,11 @@ class FullRelation(nn.Module):
         return out
 
     # ------------------------------------------------------------------------------------------
+    def _check_width(self, x: torch.Tensor) -> None:
+        """The prologue's kernels take the head dim from x, so its width has to be the layer's."""
+        if x.dim() != 3 or x.shape[-1] != self.d_model:
+            raise RuntimeError(f"FullRelation takes x [B, T, {self.d_model}], got {list(x.shape)}")
+
     def _fused_prologue(self, bf16: bool) -> bool:
         """Whether the one-launch prologue serves this layer: bf16 activations, a width of whole 64-column
         stages, head dim 64 / 96 / 128, or 48 without QK-Norm (the 192-wide layer, 19,856 rows: product
@@ -701,6 +706,7 @@ class FullRelation(nn.Module):
 
     def heads(self, x: torch.Tensor, S: int):
         """Projections -> (QK-Norm) -> RoPE / Givens: (p1, p2, I~) as [B, H, T, dh] views."""
+        self._check_width(x)
         B, T, D = x.shape
         H, dh = self.n_heads, self.d_head
         ws = (self.w1.weight, self.w2.weight, self.wi.weight)
@@ -726,6 +732,7 @@ class FullRelation(nn.Module):
         """heads() with P2 and I~ written straight into the arena's rows [S, S + T) by the prologue's launch
         (two copies fewer): p1, or None where that does not apply (a backward is wanted, another dtype or
         batch, a width the fused prologue does not serve, a traced call)."""
+        self._check_width(x)
         B, T, _ = x.shape
         arena = cache.arena
         bf16 = x.dtype == torch.bfloat16 or (torch.is_autocast_enabled() and
@@ -761,6 +768,7 @@ class FullRelation(nn.Module):
         mass g [B, H, T] (relation.py:184-268)."""
         if not USE_FLASH:
             raise RuntimeError("mote_amd.relation has only the HIP path (USE_FLASH = False is not supported)")
+        self._check_width(x)
         if not x.is_cuda:
             raise RuntimeError("FullRelation needs the HIP library and an MI355X (x is on the CPU)")
         B, T, D = x.shape
