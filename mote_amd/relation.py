@@ -434,6 +434,8 @@ _qkv_rope.register_autograd(_qr_backward, setup_context=_qr_setup)
 # ---- the prologue from the layer's own three weights -----------------------------------------------
 def _packed(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, wi: torch.Tensor) -> torch.Tensor:
     """The bf16 stack [w1; w2; wi]: fp32 weights rounded and stacked in one launch, others by torch."""
+    if not w1.shape == w2.shape == wi.shape or any(t.device != x.device for t in (w1, w2, wi)):
+        raise RuntimeError("mote::qkv_rope_master: the three weights must be of one shape, on x's device")
     if not all(t.dtype == torch.float32 for t in (w1, w2, wi)) or w1.numel() % 8:
         return torch.cat([w1, w2, wi], dim=0).to(torch.bfloat16)
     ws = [t if t.data_ptr() % 16 == 0 else t.clone() for t in (w1.contiguous(), w2.contiguous(), wi.contiguous())]

@@ -58,3 +58,28 @@ def test_prologue_entry_refuses_overlapping_rows(view, stride):
     setattr(getattr(a, view), stride, 96)
     rc = L.lib().mote_qkv_rope_parts_fwd(a, C.c_void_p(1 << 21), C.c_void_p(1 << 21), None)
     assert rc != 0 and b"strides of at least 128" in L.lib().mote_last_error()
+
+
+@pytest.mark.parametrize("what,match", [
+    ("x dtype", "x must be bf16"), ("heads", "x must be bf16"), ("one weight", "weights must be"), ("stack", "weights must be"),
+    ("weight dtype", "weights must be"), ("weight device", "weights must be"), ("inv_freq", "inv_freq needs"), ("theta", "theta needs"),
+])
+def test_prologue_refuses_operands_of_other_sizes(what, match):
+    """256-wide rows over the weights and frequencies of another layer would be read past their ends."""
+    x, w = torch.zeros(2, 5, 256, dtype=BF16), torch.zeros(256, 256, dtype=BF16)
+    args = {"x dtype": (x.float(), [w] * 3), "heads": (x, [w] * 3, None, None, None, None, 3), "one weight": (x, [w, w[:192], w]),
+            "stack": (x, [torch.zeros(768, 192, dtype=BF16)]), "weight dtype": (x, [w, w.float(), w]),
+            "weight device": (x, [w, w, w.to("meta")]), "inv_freq": (x, [w] * 3, None, None, torch.zeros(24)),
+            "theta": (x, [w] * 3, None, None, torch.zeros(32), torch.zeros(1))}[what]
+    with pytest.raises(RuntimeError, match=match):
+        _prologue(*args)
+
+
+@pytest.mark.parametrize("shapes", [((64, 64), (64, 32), (64, 64)), ((64, 64), (64, 64), (32, 64))])
+def test_weight_stack_refuses_unequal_weights(shapes):
+    x, ws = torch.zeros(1, 1, 64, dtype=BF16), [torch.zeros(s) for s in shapes]
+    with pytest.raises(RuntimeError, match="of one shape"):
+        R._packed(x, *ws)
+    ws = [torch.zeros(64, 64), torch.zeros(64, 64, device="meta"), torch.zeros(64, 64)]
+    with pytest.raises(RuntimeError, match="on x's device"):
+        R._packed(x, *ws)
