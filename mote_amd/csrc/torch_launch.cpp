@@ -168,6 +168,10 @@ std::tuple<Tensor, Tensor> rope_givens_bwd(const Tensor& dp1_, const Tensor& dp2
 }
 
 Tensor linear_wgrad(Tensor a_, Tensor x, at::ScalarType dtype, int64_t stream) {
+  TORCH_CHECK(a_.dim() == 2 && x.dim() == 2 && a_.size(0) == x.size(0) && a_.scalar_type() == x.scalar_type() &&
+                  a_.device() == x.device(),
+              "linear_wgrad: a [M, N] and x [M, K] of one dtype and device, got ", a_.sizes(), " ", a_.scalar_type(), " and ",
+              x.sizes(), " ", x.scalar_type());
   auto rows = [](const Tensor& t) {
     return t.stride(1) == 1 && t.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.contiguous();
   };

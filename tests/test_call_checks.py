@@ -83,3 +83,11 @@ def test_weight_stack_refuses_unequal_weights(shapes):
     ws = [torch.zeros(64, 64), torch.zeros(64, 64, device="meta"), torch.zeros(64, 64)]
     with pytest.raises(RuntimeError, match="on x's device"):
         R._packed(x, *ws)
+
+
+@pytest.mark.parametrize("x", [torch.zeros(6, 64, dtype=BF16), torch.zeros(7, 64), torch.zeros(7, 64, dtype=BF16, device="meta"),
+                               torch.zeros(1, 7, 64, dtype=BF16)], ids=["rows", "dtype", "device", "dims"])
+def test_weight_gradient_refuses_unlike_operands(x):
+    """A shorter x would be read past its end, an fp32 one as bf16."""
+    with pytest.raises(RuntimeError, match=r"linear_wgrad: a \[M, N\] and x"):
+        L.native().linear_wgrad(torch.zeros(7, 128, dtype=BF16), x, torch.float32, 0)
