@@ -572,6 +572,8 @@ def _og_setup(ctx, inputs, output):
 def _gate_bwd(dz: torch.Tensor, y: torch.Tensor, s: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """bf16 (dy, dg) = (dz s, dz y s (1 - s)) of equally shaped bf16 tensors whose last axis is a multiple
     of 8, contiguous results."""
+    if not dz.shape == y.shape == s.shape or any(t.dtype != torch.bfloat16 or t.device != dz.device for t in (dz, y, s)):
+        raise RuntimeError("mote::gate_bwd takes bf16 dz, y and s of one shape on one device")
     if not dz.is_cuda:
         raise RuntimeError("mote::gate_bwd needs the HIP library and an MI355X")
     # the kernel walks flat memory in 16-byte chunks: copies of views in another order or off a chunk

@@ -91,3 +91,13 @@ def test_weight_gradient_refuses_unlike_operands(x):
     """A shorter x would be read past its end, an fp32 one as bf16."""
     with pytest.raises(RuntimeError, match=r"linear_wgrad: a \[M, N\] and x"):
         L.native().linear_wgrad(torch.zeros(7, 128, dtype=BF16), x, torch.float32, 0)
+
+
+@pytest.mark.parametrize("bad", [torch.zeros(1, 4, 64, dtype=BF16), torch.zeros(1, 5, 64), torch.zeros(1, 5, 64, dtype=BF16, device="meta")],
+                         ids=["shape", "dtype", "device"])
+def test_gate_backward_refuses_unlike_operands(bad):
+    """The launch is sized by dz: a smaller y or s would be read, a smaller dy written, past the end."""
+    good = torch.zeros(1, 5, 64, dtype=BF16)
+    for args in ((good, bad, good), (good, good, bad)):
+        with pytest.raises(RuntimeError, match="of one shape on one device"):
+            R._gate_bwd._init_fn(*args)
