@@ -172,8 +172,12 @@ Tensor linear_wgrad(Tensor a_, Tensor x, at::ScalarType dtype, int64_t stream) {
                   a_.device() == x.device(),
               "linear_wgrad: a [M, N] and x [M, K] of one dtype and device, got ", a_.sizes(), " ", a_.scalar_type(), " and ",
               x.sizes(), " ", x.scalar_type());
+  // rows the kernel can walk: apart (an expanded gradient has stride 0), within its 32-bit offsets, aligned
   auto rows = [](const Tensor& t) {
-    return t.stride(1) == 1 && t.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.contiguous();
+    const int64_t sr = t.stride(0);
+    const bool ok = t.stride(1) == 1 && sr >= t.size(1) && sr < (int64_t(1) << 24) && sr % 8 == 0 &&
+                    reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+    return ok ? t : t.contiguous();
   };
   a_ = rows(a_);
   x = rows(x);

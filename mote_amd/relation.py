@@ -306,26 +306,13 @@ USE_WGRAD = True  # bf16 rows, both widths multiples of 64: mote_linear_wgrad; e
 
 @torch.library.custom_op("mote::wgrad", mutates_args=())
 def _wgrad(a: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """bf16 dW [N, K] = a^T x for a [M, N], x [M, K], fp32 sums (operands whose rows are not unit-stride
-    and 16-byte aligned are copied first)."""
+    """bf16 dW [N, K] = a^T x for a [M, N], x [M, K], fp32 sums, N and K multiples of 128: mote::linear_wgrad
+    under its earlier name."""
     if not a.is_cuda:
         raise RuntimeError("mote::wgrad needs the HIP library and an MI355X")
-    ok = lambda t: t.stride(1) == 1 and (t.stride(0) * 2) % 16 == 0 and t.data_ptr() % 16 == 0
-    a = a if ok(a) else a.contiguous()
-    x = x if ok(x) else x.contiguous()
-    M, N = a.shape
-    K = x.shape[1]
-    dw = torch.empty(N, K, device=a.device, dtype=a.dtype)
-    args = L.WgradArgs()
-    args.dtype, args.M, args.N, args.K = L.dtype_code(a), M, N, K
-    args.a, args.a_sr = a.data_ptr(), a.stride(0)
-    args.x, args.x_sr = x.data_ptr(), x.stride(0)
-    args.dw, args.dw_sr = dw.data_ptr(), dw.stride(0)
-    nbytes = int(L.lib().mote_wgrad_workspace(args))
-    ws = torch.empty(max(nbytes, 16), device=a.device, dtype=torch.uint8)
-    args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
-    L.check(L.lib().mote_wgrad(args, L.stream_of(a)), "mote_wgrad")
-    return dw
+    if a.dtype != torch.bfloat16 or a.shape[1] % 128 or x.shape[1] % 128:
+        raise RuntimeError(f"mote::wgrad: {a.dtype} [M, {a.shape[1]}] and [M, {x.shape[1]}] (bf16, widths multiples of 128)")
+    return L.native().linear_wgrad(a, x, a.dtype, L.stream_of(a))
 
 
 @_wgrad.register_fake
@@ -336,7 +323,7 @@ def _wgrad_fake(a, x):
 @torch.library.custom_op("mote::linear_wgrad", mutates_args=())
 def _linear_wgrad(a: torch.Tensor, x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """dW [N, K] = a^T x in `dtype` (bf16, or the fp32 sums unrounded) for bf16 a [M, N], x [M, K] with N
-    and K multiples of 64 (operands whose rows are not unit-stride and 16-byte aligned are copied first)."""
+    and K multiples of 64 (operands whose rows are not apart, unit-stride and 16-byte aligned are copied first)."""
     if not a.is_cuda:
         raise RuntimeError("mote::linear_wgrad needs the HIP library and an MI355X")
     return L.native().linear_wgrad(a, x, dtype, L.stream_of(a))

@@ -170,3 +170,54 @@ def test_linear_wgrad_function_under_create_graph(cuda):
 
     for a, b in zip(second(linear_wgrad), second(torch.nn.functional.linear)):
         assert a.dtype == b.dtype and rel_err(a, b) < 2e-2, rel_err(a, b)
+
+
+def _rows(form, M, N, dev):
+    """bf16 [M, N] operands whose rows the kernel cannot walk where they are."""
+    t = torch.randn(M, N, device=dev).bfloat16()
+    if form == "expanded":
+        return t[:1].expand(M, N)
+    if form == "far apart":  # a row stride past the kernel's 32-bit offsets
+        return torch.empty((M - 1) * (1 << 24) + N, device=dev, dtype=torch.bfloat16).as_strided((M, N), (1 << 24, 1)).copy_(t)
+    if form == "overlapping":
+        return torch.randn((M - 1) * 8 + N, device=dev).bfloat16().as_strided((M, N), (8, 1))
+    return t
+
+
+@pytest.mark.parametrize("N,K", [(192, 64), (128, 256)])
+@pytest.mark.parametrize("form", ["expanded", "far apart", "overlapping"])
+def test_rows_the_kernel_cannot_walk_are_copied(cuda, N, K, form):
+    """Either operand, through mote::linear_wgrad and (multiples of 128) mote::wgrad; bounds as above."""
+    from mote_amd.relation import _linear_wgrad, _wgrad
+
+    print(f"case wgrad rows {form} N={N} K={K}", flush=True)
+    torch.manual_seed(N)
+    for fa, fx in ((form, "plain"), ("plain", form)):
+        a, x = _rows(fa, 5, N, cuda), _rows(fx, 5, K, cuda)
+        ref = a.double().t().contiguous() @ x.double().contiguous()
+        assert rel_err(_linear_wgrad(a, x, torch.float32), ref) < 1e-5
+        if N % 128 == 0:
+            assert rel_err(_wgrad(a, x), ref) < 4e-3
+
+
+@pytest.mark.parametrize("reduce", [lambda y: y.sum((0, 1)), lambda y: y.sum(1)], ids=["sum over rows", "sum over time"])
+@pytest.mark.parametrize("d,H", [(192, 4), (256, 4)])
+def test_output_reduced_over_its_rows(cuda, monkeypatch, d, H, reduce):
+    """A layer's output summed over its rows hands wo's backward a gradient of row stride 0: weight
+    gradients as with the products on the GEMM library (bf16 there: 2^-9 an element, and a change of order)."""
+    from mote_amd import relation as R
+
+    print(f"case reduced output d={d}", flush=True)
+    torch.manual_seed(2)
+    m = R.FullRelation(d, H, 0, device=cuda)
+    x = torch.randn(1, 77, d, device=cuda)
+    dy = torch.randn(d, device=cuda)
+
+    def grads(use):
+        monkeypatch.setattr(R, "USE_WGRAD", use)
+        with torch.autocast("cuda", torch.bfloat16):
+            out = reduce(m(x))
+        return torch.autograd.grad(out, list(m.parameters()), dy.to(out.dtype).expand_as(out))
+
+    for a, b in zip(grads(True), grads(False)):
+        assert rel_err(a, b) < 1e-2, rel_err(a, b)
