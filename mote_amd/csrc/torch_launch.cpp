@@ -177,7 +177,7 @@ Tensor linear_wgrad(Tensor a_, Tensor x, at::ScalarType dtype, int64_t stream) {
     const int64_t sr = t.stride(0);
     const bool ok = t.stride(1) == 1 && sr >= t.size(1) && sr < (int64_t(1) << 24) && sr % 8 == 0 &&
                     reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
-    return ok ? t : t.contiguous();
+    return ok ? t : t.clone(at::MemoryFormat::Contiguous);  // (contiguous() keeps a contiguous tensor off a boundary)
   };
   a_ = rows(a_);
   x = rows(x);
@@ -276,7 +276,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> qkv_rope(const Tensor& x, con
                                                             const OptTensor& info_, int64_t stream) {
   const int64_t B = x.size(0), T = x.size(1), K = x.size(2), D = K / H;
   const at::ScalarType dt = x.scalar_type();
-  TORCH_CHECK(dt == at::kBFloat16 && K == H * D, "qkv_rope: x must be bf16 of ", H, " heads, got ", dt, " rows of ", K);
+  TORCH_CHECK(dt == at::kBFloat16 && K == H * D && x.is_contiguous(), "qkv_rope: x must be bf16 of ", H, " heads, got ", dt, " rows of ", K);
   for (const Tensor& w : ws)
     TORCH_CHECK(w.sizes() == at::IntArrayRef({ws.size() == 3 ? K : 3 * K, K}) && w.scalar_type() == dt &&
                     w.device() == x.device() && w.is_contiguous(),
@@ -294,7 +294,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> qkv_rope(const Tensor& x, con
   Tensor qkraw = keep_info && norm ? empty({B, T, 2 * K}, x, dt) : empty({0}, x, dt);
   mote_qkv_rope_args a{};
   a.B = int(B); a.T = int(T); a.H = int(H); a.D = int(D); a.pos0 = int(pos0); a.layer_parity = int(parity);
-  a.x = x.data_ptr(); a.x_sb = x.stride(0); a.x_sr = x.stride(1);
+  a.x = x.data_ptr(); a.x_sb = T * K; a.x_sr = K;  // contiguous (the strides of axes of one element may be any)
   a.w = ws[0].data_ptr(); a.w_sr = K;
   Tensor inv, th, n1, n2;
   if (inv_freq) {

@@ -212,10 +212,9 @@ def _qkv_rope_launch(x, w, inv_freq, theta, n_heads, parity, pos0, keep_info, no
         raise ValueError("mote::qkv_rope: QK-Norm needs both gains")
     if norm_w1 is not None and (norm_w1.numel() != D or norm_w2.numel() != D):
         raise ValueError("mote::qkv_rope: QK-Norm gains must have head-dim elements")
-    x = x.contiguous()
-    ws = [t.contiguous() for t in w] if isinstance(w, tuple) else [w.contiguous()]
-    if len(ws) == 3:
-        ws = [t if t.data_ptr() % 16 == 0 else t.clone() for t in ws]
+    # the kernel reads 16-byte chunks: contiguous copies of operands that are not, or start off a chunk
+    x, *ws = (t if t.data_ptr() % 16 == 0 else t.clone()
+              for t in (t.contiguous() for t in (x, *(w if isinstance(w, tuple) else (w,)))))
     # the caller's own frequency tensor (not a converted temporary) can key a memoised table
     own = inv_freq is not None and inv_freq.device == x.device and inv_freq.dtype == torch.float32 and inv_freq.is_contiguous()
     inv = inv_freq if inv_freq is None or own else inv_freq.to(device=x.device, dtype=torch.float32).contiguous()

@@ -419,6 +419,24 @@ def test_prologue_head_dim_48(cuda, monkeypatch, T, B, layer):
         assert a.dtype == b.dtype and rel_err(a, b) < 1.6e-2, rel_err(a, b)
 
 
+@pytest.mark.parametrize("d,H", [(192, 4), (256, 4)])
+@pytest.mark.parametrize("T", [1, 33])
+def test_prologue_takes_x_off_a_boundary(cuda, d, H, T):
+    """x one element past a 16-byte boundary, or (T = 1) with a row stride of one: contiguous either way, the
+    results those of an aligned copy bit for bit."""
+    from mote_amd.relation import FullRelation
+
+    print(f"case misaligned x d={d} T={T}", flush=True)
+    torch.manual_seed(d)
+    m = FullRelation(d, H, 0, device=cuda, dtype=torch.bfloat16)
+    x = torch.randn(2, T, d, device=cuda).bfloat16()
+    forms = [torch.empty(2 * T * d + 1, device=cuda, dtype=torch.bfloat16)[1:].view(2, T, d).copy_(x)]
+    if T == 1:
+        forms.append(x.clone().as_strided((2, 1, d), (d, 1, 1)))
+    for f in forms:
+        assert all(torch.equal(a, b) for a, b in zip(m.heads(f, 3), m.heads(x, 3)))
+
+
 @pytest.mark.parametrize("S,T,B,norm,dtype", [(0, 1, 1, False, torch.bfloat16), (64, 40, 1, True, torch.bfloat16),
                                               (100, 129, 2, False, torch.float32)])
 def test_arena_rows_written_by_the_prologue(cuda, S, T, B, norm, dtype):

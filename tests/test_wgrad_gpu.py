@@ -181,11 +181,15 @@ def _rows(form, M, N, dev):
         return torch.empty((M - 1) * (1 << 24) + N, device=dev, dtype=torch.bfloat16).as_strided((M, N), (1 << 24, 1)).copy_(t)
     if form == "overlapping":
         return torch.randn((M - 1) * 8 + N, device=dev).bfloat16().as_strided((M, N), (8, 1))
+    if form == "off a boundary":  # contiguous, so contiguous() would keep it
+        return torch.empty(M * N + 1, device=dev, dtype=torch.bfloat16)[1:].view(M, N).copy_(t)
+    if form == "one row":  # contiguous whatever its row stride says
+        return t[0].clone().as_strided((1, N), (1, 1))
     return t
 
 
 @pytest.mark.parametrize("N,K", [(192, 64), (128, 256)])
-@pytest.mark.parametrize("form", ["expanded", "far apart", "overlapping"])
+@pytest.mark.parametrize("form", ["expanded", "far apart", "overlapping", "off a boundary", "one row"])
 def test_rows_the_kernel_cannot_walk_are_copied(cuda, N, K, form):
     """Either operand, through mote::linear_wgrad and (multiples of 128) mote::wgrad; bounds as above."""
     from mote_amd.relation import _linear_wgrad, _wgrad
@@ -193,7 +197,8 @@ def test_rows_the_kernel_cannot_walk_are_copied(cuda, N, K, form):
     print(f"case wgrad rows {form} N={N} K={K}", flush=True)
     torch.manual_seed(N)
     for fa, fx in ((form, "plain"), ("plain", form)):
-        a, x = _rows(fa, 5, N, cuda), _rows(fx, 5, K, cuda)
+        M = 1 if form == "one row" else 5
+        a, x = _rows(fa, M, N, cuda), _rows(fx, M, K, cuda)
         ref = a.double().t().contiguous() @ x.double().contiguous()
         assert rel_err(_linear_wgrad(a, x, torch.float32), ref) < 1e-5
         if N % 128 == 0:
