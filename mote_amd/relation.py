@@ -354,24 +354,25 @@ def weight_grad(a: torch.Tensor, x: torch.Tensor, dtype: Optional[torch.dtype] =
 
 
 class _LinearWgrad(torch.autograd.Function):
-    """y = x W^T on the GEMM library for bf16 x and bf16 or fp32 W (rounded to bf16 first, as autocast
-    does); backward dx = dy W on the library and dW = dy^T x on mote_linear_wgrad in W's own dtype
-    (the library runs that product with its reduction over the token rows)."""
+    """y = x W^T on the GEMM library for bf16 x and wb, W in bf16 (W itself, or its cast by the caller);
+    backward dx = dy W on the library and dW = dy^T x on mote_linear_wgrad, in W's own dtype straight to W
+    (the library runs that product with its reduction over the token rows). Only wb is saved: a later
+    in-place update of fp32 W leaves the graph usable, as with F.linear of the cast. Under create_graph the
+    gradient goes to wb, through the cast."""
 
     @staticmethod
-    def forward(ctx, x, w):
-        wb = w.to(x.dtype)
-        ctx.save_for_backward(x, w, wb)
+    def forward(ctx, x, w, wb):
+        ctx.save_for_backward(x, wb)
+        ctx.w_dtype = w.dtype
         return F.linear(x, wb)
 
     @staticmethod
     def backward(ctx, dy):
-        x, w, wb = ctx.saved_tensors
-        if torch.is_grad_enabled():  # create_graph: through the cast of W
-            wb = w.to(x.dtype)
+        x, wb = ctx.saved_tensors
         dx = torch.matmul(dy, wb) if ctx.needs_input_grad[0] else None
-        dw = weight_grad(dy, x, w.dtype) if ctx.needs_input_grad[1] else None
-        return dx, dw
+        if torch.is_grad_enabled():
+            return dx, None, (weight_grad(dy, x) if ctx.needs_input_grad[2] else None)
+        return dx, (weight_grad(dy, x, ctx.w_dtype) if ctx.needs_input_grad[1] else None), None
 
 
 def linear_wgrad(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -382,7 +383,7 @@ def linear_wgrad(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         x = x.to(torch.bfloat16)
     wdt = torch.bfloat16 if auto and w.dtype == torch.float32 else w.dtype  # autocast rounds fp32 weights
     if x.is_cuda and w.is_cuda and _wgrad_serves(x.dtype, wdt, w.shape[0], w.shape[1]):
-        return _LinearWgrad.apply(x, w)
+        return _LinearWgrad.apply(x, w, w.to(x.dtype))
     return F.linear(x, w)
 
 

@@ -226,3 +226,25 @@ def test_output_reduced_over_its_rows(cuda, monkeypatch, d, H, reduce):
 
     for a, b in zip(grads(True), grads(False)):
         assert rel_err(a, b) < 1e-2, rel_err(a, b)
+
+
+@pytest.mark.parametrize("d,H", [(192, 4), (256, 4)])
+def test_backward_after_an_in_place_weight_update(cuda, d, H):
+    """Under autocast a graph keeps the weights' bf16 copies, so a backward after an optimizer's in-place step
+    on the fp32 masters gives the gradients it would have given before (Givens off: theta itself is saved)."""
+    from mote_amd.relation import FullRelation
+
+    print(f"case backward after update d={d}", flush=True)
+    torch.manual_seed(4)
+    m = FullRelation(d, H, 0, givens=False, device=cuda)
+    x = torch.randn(2, 50, d, device=cuda, requires_grad=True)
+    leaves = [x, *m.parameters()]
+    with torch.autocast("cuda", torch.bfloat16):
+        out = m(x)
+    dy = torch.randn_like(out)
+    before = torch.autograd.grad(out, leaves, dy, retain_graph=True)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.mul_(0.5)
+    for a, b in zip(torch.autograd.grad(out, leaves, dy), before):
+        assert a.dtype == torch.float32 and torch.equal(a, b)
