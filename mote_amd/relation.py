@@ -340,6 +340,13 @@ def _wgrad_serves(a_dtype: torch.dtype, x_dtype: torch.dtype, N: int, K: int) ->
     return USE_WGRAD and a_dtype == torch.bfloat16 and x_dtype == torch.bfloat16 and N % 64 == 0 and K % 64 == 0
 
 
+def _transformed() -> bool:
+    """Whether a functional transform (vmap, grad, jvp; batched gradients too) or a forward-mode level is
+    active: products then stay with torch, since mote_linear_wgrad's function and op have neither rule."""
+    return not torch.compiler.is_compiling() and (torch._C._are_functorch_transforms_active()
+                                                  or torch.autograd.forward_ad._current_level >= 0)
+
+
 def weight_grad(a: torch.Tensor, x: torch.Tensor, dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     """a^T x over the token rows of a [..., N] and x [..., K]: the weight gradient of y = x W^T, in a's
     dtype or `dtype` (fp32: the sums unrounded). mote_linear_wgrad for bf16 on the GPU with N, K
@@ -348,7 +355,7 @@ def weight_grad(a: torch.Tensor, x: torch.Tensor, dtype: Optional[torch.dtype] =
     a2, x2 = a.reshape(-1, N), x.reshape(-1, K)
     dtype = a2.dtype if dtype is None else dtype
     # under create_graph the product has to be differentiable itself
-    if a2.is_cuda and _wgrad_serves(a2.dtype, x2.dtype, N, K) and not torch.is_grad_enabled():
+    if a2.is_cuda and _wgrad_serves(a2.dtype, x2.dtype, N, K) and not torch.is_grad_enabled() and not _transformed():
         return _linear_wgrad(a2, x2, dtype)
     return torch.matmul(a2.t(), x2).to(dtype)
 
@@ -382,7 +389,7 @@ def linear_wgrad(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if auto:
         x = x.to(torch.bfloat16)
     wdt = torch.bfloat16 if auto and w.dtype == torch.float32 else w.dtype  # autocast rounds fp32 weights
-    if x.is_cuda and w.is_cuda and _wgrad_serves(x.dtype, wdt, w.shape[0], w.shape[1]):
+    if x.is_cuda and w.is_cuda and _wgrad_serves(x.dtype, wdt, w.shape[0], w.shape[1]) and not _transformed():
         return _LinearWgrad.apply(x, w, w.to(x.dtype))
     return F.linear(x, w)
 

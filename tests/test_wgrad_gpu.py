@@ -248,3 +248,31 @@ def test_backward_after_an_in_place_weight_update(cuda, d, H):
             p.mul_(0.5)
     for a, b in zip(torch.autograd.grad(out, leaves, dy), before):
         assert a.dtype == torch.float32 and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("N,K", [(64, 192), (128, 128)])
+def test_linear_wgrad_under_transforms(cuda, N, K):
+    """grad, vmap, jvp, forward-mode levels and batched gradients over linear_wgrad, as over F.linear: every
+    product the library's, so the bits are its own (batched ones within a bf16 rounding, 2^-8)."""
+    from mote_amd.relation import linear_wgrad
+
+    print(f"case linear_wgrad transforms N={N}", flush=True)
+    torch.manual_seed(6)
+    x, t = (torch.randn(3, 20, K, device=cuda).bfloat16() for _ in range(2))
+    w = (torch.randn(N, K, device=cuda) / K ** 0.5).bfloat16()
+    F = torch.nn.functional
+
+    def forward_mode(fn):
+        with torch.autograd.forward_ad.dual_level():
+            return torch.autograd.forward_ad.unpack_dual(fn(torch.autograd.forward_ad.make_dual(x, t), w)).tangent
+
+    def batched(fn):
+        wr = w.clone().requires_grad_(True)
+        y = fn(x, wr)
+        return torch.autograd.grad(y, wr, torch.stack([y.detach(), 2 * y.detach()]), is_grads_batched=True)[0]
+
+    for run in (lambda fn: torch.func.grad(lambda v: fn(x, v).float().square().sum())(w),
+                lambda fn: torch.func.vmap(fn, (0, None))(x, w),
+                lambda fn: torch.func.jvp(lambda v: fn(v, w), (x,), (t,))[1], forward_mode, batched):
+        got, want = run(linear_wgrad), run(F.linear)
+        assert got.shape == want.shape and rel_err(got, want) < 2.0 ** -7, rel_err(got, want)
