@@ -385,13 +385,13 @@ class _LinearWgrad(torch.autograd.Function):
 def linear_wgrad(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear(x, w) whose weight gradient runs on mote_linear_wgrad: bf16 x and w on the GPU (or bf16
     autocast, which casts both as F.linear would) with both widths multiples of 64; F.linear otherwise."""
-    auto = torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") == torch.bfloat16 and x.is_cuda
-    if auto:
-        x = x.to(torch.bfloat16)
-    wdt = torch.bfloat16 if auto and w.dtype == torch.float32 else w.dtype  # autocast rounds fp32 weights
-    if x.is_cuda and w.is_cuda and _wgrad_serves(x.dtype, wdt, w.shape[0], w.shape[1]) and not _transformed():
-        return _LinearWgrad.apply(x, w, w.to(x.dtype))
-    return F.linear(x, w)
+    wb = w
+    if torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") == torch.bfloat16 and x.is_cuda:
+        x, wb = x.to(torch.bfloat16), w.to(torch.bfloat16)  # (F.linear itself would not cast fp64)
+    if x.is_cuda and w.is_cuda and _wgrad_serves(x.dtype, wb.dtype, *w.shape) and not _transformed():
+        # fp32 weights take dW from the function itself, others through their cast
+        return _LinearWgrad.apply(x, w if w.dtype == torch.float32 else wb, wb)
+    return F.linear(x, wb)
 
 
 def _qr_grads(ctx, dp1, dp2, dinfo, wdtype):

@@ -253,7 +253,8 @@ def test_backward_after_an_in_place_weight_update(cuda, d, H):
 @pytest.mark.parametrize("N,K", [(64, 192), (128, 128)])
 def test_linear_wgrad_under_transforms(cuda, N, K):
     """grad, vmap, jvp, forward-mode levels and batched gradients over linear_wgrad, as over F.linear: every
-    product the library's, so the bits are its own (batched ones within a bf16 rounding, 2^-8)."""
+    product the library's, so they differ by the order of a batched one alone: one bf16 rounding, 2^-7 of the
+    largest element."""
     from mote_amd.relation import linear_wgrad
 
     print(f"case linear_wgrad transforms N={N}", flush=True)
@@ -276,3 +277,23 @@ def test_linear_wgrad_under_transforms(cuda, N, K):
                 lambda fn: torch.func.jvp(lambda v: fn(v, w), (x,), (t,))[1], forward_mode, batched):
         got, want = run(linear_wgrad), run(F.linear)
         assert got.shape == want.shape and rel_err(got, want) < 2.0 ** -7, rel_err(got, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float16])
+@pytest.mark.parametrize("N", [64, 72])
+def test_linear_wgrad_casts_other_weights_under_autocast(cuda, N, dtype):
+    """Weights that autocast's own F.linear refuses (fp64) or casts (fp16), at a served width and beside it:
+    the product of the bf16 casts, gradients in the weights' dtype (bf16 roundings, 2^-9 each)."""
+    from mote_amd.relation import linear_wgrad
+
+    print(f"case linear_wgrad weights {dtype} N={N}", flush=True)
+    torch.manual_seed(7)
+    x = torch.randn(30, 128, device=cuda, requires_grad=True)
+    w = (torch.randn(N, 128, device=cuda) / 12).to(dtype).requires_grad_(True)
+    with torch.autocast("cuda", torch.bfloat16):
+        y = linear_wgrad(x, w)
+    xb, wb = x.detach().bfloat16().double(), w.detach().bfloat16().double()
+    assert y.dtype == torch.bfloat16 and rel_err(y, xb @ wb.t()) < 1e-2
+    dx, dw = torch.autograd.grad(y, (x, w), torch.ones_like(y))
+    assert dx.dtype == torch.float32 and dw.dtype == dtype
+    assert rel_err(dx, wb.sum(0).expand_as(dx)) < 1e-2 and rel_err(dw, xb.sum(0).expand_as(dw)) < 1e-2
