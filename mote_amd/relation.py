@@ -589,7 +589,11 @@ def _og_backward(ctx, dz, _ds):
     """z = y s, s = sigmoid(g), g = x wg^T: dy = dz s, dg = dz y s (1 - s), dx = dg wg, dwg = dg^T x."""
     x, wg, y, s = ctx.saved_tensors
     dz = torch.zeros_like(y) if dz is None else dz
-    dy, dg = _gate_bwd(dz, y, s)
+    if torch.is_grad_enabled():  # create_graph: as torch ops, which can be differentiated again
+        dzf, sf = dz.float(), s.float()
+        dy, dg = (dzf * sf).to(y.dtype), (dzf * y.float() * sf * (1.0 - sf)).to(x.dtype)
+    else:
+        dy, dg = _gate_bwd(dz, y, s)
     dx = torch.matmul(dg, wg)
     dwg = weight_grad(dg, x)
     return dx, dwg, dy

@@ -484,6 +484,22 @@ def test_gate_backward_elementwise_bits(cuda, shape):
         assert torch.equal(dg, (dzf * b.float() * sf * (1.0 - sf)).bfloat16())
 
 
+def test_out_gate_gradient_can_be_differentiated_again(cuda):
+    """z = y s is linear in y, dy = dz s in dz: under create_graph the gradient of dy with respect to dz is s
+    itself, and the first gradients are the bits of a plain backward."""
+    from mote_amd.relation import _out_gate, out_gate
+
+    print("case out_gate create_graph", flush=True)
+    g = torch.Generator().manual_seed(91)
+    x, y, dz = (torch.randn(1, 33, 128, generator=g).bfloat16().to(cuda).requires_grad_(True) for _ in range(3))
+    wg = (torch.randn(128, 128, generator=g) / 11).bfloat16().to(cuda).requires_grad_(True)
+    z = out_gate(x, wg, y)
+    plain = torch.autograd.grad(z, (x, y), dz, retain_graph=True)
+    first = torch.autograd.grad(z, (x, y), dz, create_graph=True)
+    assert all(torch.equal(a, b) for a, b in zip(first, plain))
+    assert torch.equal(torch.autograd.grad(first[1], dz, torch.ones_like(y))[0], _out_gate(x, wg, y)[1])
+
+
 def test_out_gate_and_qk_norm_ops_pass_opcheck(cuda):
     from mote_amd.relation import rope_inv_freq
 
