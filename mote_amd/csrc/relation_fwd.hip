@@ -360,13 +360,6 @@ __global__ void __launch_bounds__(NW * 64) relation_fwd_kernel(const FwdParams p
 //                     (a lane holds one query and keys 4g + r of each 16-key tile: the permuted k
 //                     order both fragments share)
 // ------------------------------------------------------------------------------------------------
-// The running reference m of a query's online softmax is an upper bound of its exponents rather
-// than their maximum: with u2 = U log2e, the exponent SiLU(U) log2e = u2 sigmoid(U) never exceeds
-// max(u2, 0), so the block's bound comes from the raw dot products (one max per element, no SiLU
-// needed first) and m starts at 0. Exponents then stay in [-0.4, 0] below the bound for u2 >= 0
-// and the row sum l is exact up to rounding whatever m is; LSE = (m + log2 l) ln2.
-// The row sums come from the P^T fragments too: one more product with a fragment whose row 0 is
-// all ones adds sum_k P[k][q] into row 0 of `lacc`.
 // S^T = K Q^T for the wave's quadrant: keys 32 kh + 16 kt + 4 lg + r (rows), query 16 s + li.
 template <int DP>
 __device__ __forceinline__ void fwd_scores(const bf16_t* Ks, const typename Elem<bf16_t>::Frag (&qf)[2][DP / 32],
@@ -397,7 +390,11 @@ __device__ __forceinline__ void fwd_scores(const bf16_t* Ks, const typename Elem
 // the row sum l is exact up to rounding whatever m is; LSE = (m + log2 l) ln2.
 // The row sums come from the P^T fragments too: one more product with a fragment whose row 0 is
 // all ones adds sum_k P[k][q] into row 0 of `lacc`.
-template <int DP, bool MASKED>
+// PAD takes neither shortcut: the reference is the block's largest exponent (so the largest weight is 1, which
+// bf16 holds exactly) and the row sums are the lane's own weights in fp32 before their rounding (element 0
+// of `lacc`; the lane groups' sums are added at the end). Against 64 bits at dh 48, T 1241: lse 1.3e-6 (1.9e-3
+// with rounded weights summed), g 5e-8 (2e-5).
+template <int DP, bool MASKED, bool PAD>
 __device__ __forceinline__ void fwd_softmax_pv(const bf16_t* Vs, const f32x4 (&sacc)[2][2], f32x4 (&oacc)[DP / 16][2],
                                                f32x4 (&lacc)[2], float (&m_run)[2], const typename Elem<bf16_t>::Frag& ones,
                                                int key0, const int (&qabs)[2], float c2, int kh, int li, int lg) {
@@ -415,50 +412,90 @@ __device__ __forceinline__ void fwd_softmax_pv(const bf16_t* Vs, const f32x4 (&s
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int r = 0; r < 4; ++r) keep[s][kt][r] = !MASKED || key0 + 16 * kt + 4 * lg + r < qabs[s];
-  float bnd[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    float mx = kNegInf;
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, keep[s][kt][r] ? sacc[kt][s][r] : kNegInf);
-    bnd[s] = mx;
-  }
-  // Whether any query's bound exceeds its reference by the slack needs no reduction over the lane
-  // groups: some lane's own maximum exceeds it exactly when the query's maximum does (c2 > 0 and the
-  // reference is at least 0). The query's maximum is formed only in the rare rescale branch.
-  const bool need = (bnd[0] * c2 > m_run[0] + kRescale) || (bnd[1] * c2 > m_run[1] + kRescale);
-  if (__ballot(need) != 0ull) {
-    asm volatile("" ::: "memory");  // a real branch: the rescale is rare
-    lanegroup_max2(bnd[0], bnd[1]);
-#pragma unroll
-    for (int s = 0; s < 2; ++s) bnd[s] = fmaxf(bnd[s] * c2, 0.f);
+  Frag pf[2];
+  if constexpr (PAD) {
+    float ev[2][8], mx[2];  // exponents in log2 units
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const float mn = bnd[s] > m_run[s] + kRescale ? bnd[s] : m_run[s];
-      const float alpha = fexp2(m_run[s] - mn);
-      lacc[s] *= alpha;
+      mx[s] = kNegInf;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) oacc[dt][s] *= alpha;
-      m_run[s] = mn;
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float u2 = sacc[kt][s][r] * c2;
+          const float e = u2 * frcp(1.0f + fexp2(-u2));
+          ev[s][4 * kt + r] = keep[s][kt][r] ? e : kNegInf;
+          mx[s] = fmaxf(mx[s], ev[s][4 * kt + r]);
+        }
     }
-  }
-  Frag pf[2];
+    if (__ballot(mx[0] > m_run[0] + kRescale || mx[1] > m_run[1] + kRescale) != 0ull) {
+      asm volatile("" ::: "memory");  // a real branch: the rescale is rare
+      lanegroup_max2(mx[0], mx[1]);
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    float pv[8];
+      for (int s = 0; s < 2; ++s) {
+        const float mn = mx[s] > m_run[s] + kRescale ? mx[s] : m_run[s];
+        const float alpha = fexp2(m_run[s] - mn);
+        lacc[s][0] *= alpha;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float u2 = sacc[kt][s][r] * c2;
-        const float sg = frcp(1.0f + fexp2(-u2));
-        const float pr = fexp2(fmaf(u2, sg, -m_run[s]));
-        pv[4 * kt + r] = keep[s][kt][r] ? pr : 0.f;
+        for (int dt = 0; dt < DT; ++dt) oacc[dt][s] *= alpha;
+        m_run[s] = mn;
       }
-    pf[s] = E::from_f32(pv);
-    lacc[s] = E::mma(ones, pf[s], lacc[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      float pv[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        pv[e] = fexp2(ev[s][e] - m_run[s]);
+        lacc[s][0] += pv[e];
+      }
+      pf[s] = E::from_f32(pv);
+    }
+  } else {
+    float bnd[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      float mx = kNegInf;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, keep[s][kt][r] ? sacc[kt][s][r] : kNegInf);
+      bnd[s] = mx;
+    }
+    // Whether any query's bound exceeds its reference by the slack needs no reduction over the lane
+    // groups: some lane's own maximum exceeds it exactly when the query's maximum does (c2 > 0 and the
+    // reference is at least 0). The query's maximum is formed only in the rare rescale branch.
+    const bool need = (bnd[0] * c2 > m_run[0] + kRescale) || (bnd[1] * c2 > m_run[1] + kRescale);
+    if (__ballot(need) != 0ull) {
+      asm volatile("" ::: "memory");  // a real branch: the rescale is rare
+      lanegroup_max2(bnd[0], bnd[1]);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) bnd[s] = fmaxf(bnd[s] * c2, 0.f);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const float mn = bnd[s] > m_run[s] + kRescale ? bnd[s] : m_run[s];
+        const float alpha = fexp2(m_run[s] - mn);
+        lacc[s] *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) oacc[dt][s] *= alpha;
+        m_run[s] = mn;
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      float pv[8];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float u2 = sacc[kt][s][r] * c2;
+          const float sg = frcp(1.0f + fexp2(-u2));
+          const float pr = fexp2(fmaf(u2, sg, -m_run[s]));
+          pv[4 * kt + r] = keep[s][kt][r] ? pr : 0.f;
+        }
+      pf[s] = E::from_f32(pv);
+      lacc[s] = E::mma(ones, pf[s], lacc[s]);
+    }
   }
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) {
@@ -561,7 +598,9 @@ __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, 
   const int dims[2] = {p.D, p.D};
   st.init(wave, lane, strides, dims);
   const float c2 = p.scale * kLog2e;
-  float m_run[2] = {0.f, 0.f};
+  // PAD: below every exponent (SiLU log2e is at least -0.41), so the first visible block sets it; finite, so
+  // that a merge of two parts without keys is one of zeros
+  float m_run[2] = {PAD ? -1e4f : 0.f, PAD ? -1e4f : 0.f};
   f32x4 lacc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
   f32x4 oacc[DT][2];
 #pragma unroll
@@ -608,7 +647,7 @@ __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, 
     if (q0 < TQs && key0 < qs + wq_last) {
       f32x4 sacc[2][2];
       fwd_scores<DP>(Ks, qf, sacc, kh, li, lg);
-      fwd_softmax_pv<DP, decltype(masked)::value>(Ks + TILE, sacc, oacc, lacc, m_run, ones, key0, qabs, c2, kh, li,
+      fwd_softmax_pv<DP, decltype(masked)::value, PAD>(Ks + TILE, sacc, oacc, lacc, m_run, ones, key0, qabs, c2, kh, li,
                                                   lg);
     }
     MOTE_STAMP(2, kb);
@@ -627,10 +666,11 @@ __device__ __forceinline__ void fwd_tile_job(const FwdParams& p, const int bid, 
     slot = slot + 1 == NSTG ? 0 : slot + 1;
   }
 
-  // row sums: row 0 of lacc, held by lanes 0..15 (query li); broadcast to the other lane groups
+  // row sums: row 0 of lacc, held by lanes 0..15 (query li), broadcast to the other lane groups; PAD: every
+  // lane group's part
   float l_run[2];
 #pragma unroll
-  for (int s = 0; s < 2; ++s) l_run[s] = __shfl(lacc[s][0], li, 64);
+  for (int s = 0; s < 2; ++s) l_run[s] = PAD ? lanegroup_sum(lacc[s][0]) : __shfl(lacc[s][0], li, 64);
   // merge the key halves: kh = 1 hands (m, l, O) to kh = 0 through LDS
   float* R = reinterpret_cast<float*>(smem);     // [64 queries][RLD]
   float* RM = R + 64 * RLD;                      // [64] m, then [64] l
@@ -830,7 +870,7 @@ __global__ void __launch_bounds__(256) relation_fwd_merge_kernel(const FwdParams
 #pragma unroll
     for (int e = 0; e < 4; ++e) ud = fmaf((float)q4[e], (float)k4[e], ud);
   }
-  float mm = 0.f;  // the pieces' references are at least 0
+  float mm = 0.f;  // the pieces' references are at least 0 (PAD: -0.41, or no reference at all)
   for (int i = 0; i < np; ++i) mm = fmaxf(mm, P[i * PSTRIDE + 64 * DP + row]);
   float lt = 0.f;
   f32x4 o[PER / 4];
@@ -897,8 +937,9 @@ static bool view_ok(const mote_view& v) { return v.data != nullptr; }
 
 // The tile kernel serves bf16 with row strides below 2^24: D in {32, 64, 96, 128} as they are, other head
 // dims padded to the next of these. Padded it beats the register-staged kernel, which pays a transpose
-// and two barriers a block, at every size tried (dh 48, H 4, B 16, T 1241: 59.3 -> 42.8 us; dh 88, H 2,
-// T 3000: 146 -> 42; dh 104, B 2, H 8, T 1000: 63 -> 26; dh 48, B 2, H 4, T 256: 14.5 -> 9.2).
+// and two barriers a block, at every size tried (dh 48, H 4, B 16, T 1241: 54.6 -> 38.3 us, of which the
+// fp32 row sums and references take 1.6; dh 88, H 2, T 3000: 146 -> 24.0; dh 104, B 2, H 8, T 1000: 62.6 ->
+// 25.8; dh 48, B 2, H 4, T 256: 14.3 -> 8.9).
 static bool fwd_tiles(const mote_relation_fwd_args* a) {
   return a->dtype == MOTE_BF16 && tile_strides_ok(a->p1, a->p2, a->info);
 }

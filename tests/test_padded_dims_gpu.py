@@ -82,3 +82,31 @@ def test_padded_varlen_equals_dense(cuda, D):
     finally:
         for k, v in zip(("MOTE_FWD_PERSIST", "MOTE_BWD_FUSED"), old):
             os.environ.pop(k, None) if v is None else os.environ.__setitem__(k, v)
+
+
+@pytest.mark.parametrize("D", [8, 24, 48, 88, 120])
+@pytest.mark.parametrize("T,S", [(1, 40), (64, 0), (300, 37)])
+def test_padded_row_sums_are_fp32(cuda, D, T, S):
+    """lse and g come from weights added in fp32 before their rounding to bf16, so they are off the float64
+    values of the same inputs by fp32 arithmetic alone: the scores' sums and the exponentials, a few 2^-24 of
+    exponents up to about 10, under 1e-5 (weights summed after the rounding: 1e-3). I-bar keeps one bf16 rounding
+    a weight, 2^-9 at most."""
+    from mote_amd.flash_relation import _launch_fwd
+
+    print(f"case padded sums D={D} T={T} S={S}", flush=True)
+    g = torch.Generator().manual_seed(D + T)
+    p1, p2, info = _window(g, 1, T, 2, D, cuda), _window(g, 1, S + T, 2, D, cuda), _window(g, 1, S + T, 2, D, cuda)
+    _, gate, ibar, lse = _launch_fwd(p1, p2, info, torch.tensor(0.4, device=cuda), 2.0, S)
+    u = torch.matmul(p1.double(), p2.double().transpose(2, 3).contiguous()) / D ** 0.5
+    at = torch.arange(S, S + T, device=cuda)
+    past = torch.arange(S + T, device=cuda)[None] < at[:, None]
+    e = torch.nn.functional.silu(u).masked_fill(~past, float("-inf"))
+    ref = torch.logsumexp(e, -1)
+    self_ = torch.sigmoid(torch.diagonal(u, S, 2, 3) / 2.0)
+    has = past.any(-1)
+    gref = torch.sigmoid(ref - 0.4 * torch.log(at.double() + 1) - self_)
+    assert float((lse.double() - ref)[..., has].abs().max()) < 1e-5
+    assert bool((lse[..., ~has] == float("-inf")).all()) and bool((gate[..., ~has] == 0).all())
+    assert float((gate.double() - gref)[..., has].abs().max()) < 1e-5
+    bref = torch.matmul(torch.softmax(e, -1).nan_to_num(), info.double().contiguous())
+    assert float((ibar.double() - bref).norm() / bref.norm()) < 2.0 ** -9
