@@ -114,8 +114,10 @@ int mote_relation_fwd(const mote_relation_fwd_args* args, void* stream);
  * Other shapes (longer fp32, padded bf16 head dims beyond 8 GiB of dU, longer row strides):
  * `deterministic` != 0 selects the atomic-free pair of kernels (the reference's
  * MOTE_DETERMINISTIC_RELATION, flash_relation.py:51), 0 the one-pass kernel with fp32 atomics for dp1.
- * The workspace is caller-allocated device memory of at least mote_relation_bwd_workspace()
- * bytes; its contents on entry do not matter.
+ * The workspace is caller-allocated device memory of mote_relation_bwd_workspace() bytes or more; its
+ * contents on entry do not matter. A caller short of memory may pass fewer, down to
+ * mote_relation_bwd_workspace_min() (of the order of the operands): padded bf16 head dims and fp32 then store
+ * no dU and run as the other shapes do. The two are equal where there is no such choice.
  * `stages` selects which launches run (MOTE_BWD_ROWS: per-row terms and operand copies;
  * MOTE_BWD_KEYS: the key-stationary kernel; MOTE_BWD_QUERIES: the query-stationary dp1 kernel,
  * where the path has one; MOTE_BWD_FINISH: dp1 cast and dlam, which the atomic-free paths that store dU
@@ -147,6 +149,7 @@ typedef struct mote_relation_bwd_args {
 } mote_relation_bwd_args;
 
 size_t mote_relation_bwd_workspace(const mote_relation_bwd_args* args);
+size_t mote_relation_bwd_workspace_min(const mote_relation_bwd_args* args);
 int mote_relation_bwd(const mote_relation_bwd_args* args, void* stream);
 
 /* ------------------------------------------------------------------------------------------------

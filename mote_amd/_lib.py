@@ -254,6 +254,7 @@ EXPORTS = {
     "mote_relation_fwd_workspace": ([C.POINTER(FwdArgs)], C.c_size_t),
     "mote_relation_fwd": ([C.POINTER(FwdArgs), C.c_void_p], C.c_int),
     "mote_relation_bwd_workspace": ([C.POINTER(BwdArgs)], C.c_size_t),
+    "mote_relation_bwd_workspace_min": ([C.POINTER(BwdArgs)], C.c_size_t),
     "mote_relation_bwd": ([C.POINTER(BwdArgs), C.c_void_p], C.c_int),
     "mote_rope_givens_fwd": ([C.POINTER(RopeArgs), C.c_void_p], C.c_int),
     "mote_rope_givens_bwd_workspace": ([C.POINTER(RopeBwdArgs)], C.c_size_t),

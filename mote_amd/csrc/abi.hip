@@ -26,6 +26,7 @@ int check_launch(const char* what) {
   return MOTE_OK;
 }
 
+size_t bwd_workspace_min_bytes(const mote_relation_bwd_args* a);  // relation_bwd.hip (out of params.hpp as below)
 // wgrad.hip (kept out of params.hpp, whose text every recorded kernel profile is tied to)
 size_t wgrad_workspace_bytes(const mote_wgrad_args* a);
 int launch_wgrad(const mote_wgrad_args* a, hipStream_t stream);
@@ -52,6 +53,10 @@ int mote_relation_fwd(const mote_relation_fwd_args* args, void* stream) {
 
 size_t mote_relation_bwd_workspace(const mote_relation_bwd_args* args) {
   return args ? mote::bwd_workspace_bytes(args) : 0;
+}
+
+size_t mote_relation_bwd_workspace_min(const mote_relation_bwd_args* args) {
+  return args ? mote::bwd_workspace_min_bytes(args) : 0;
 }
 
 int mote_relation_bwd(const mote_relation_bwd_args* args, void* stream) {

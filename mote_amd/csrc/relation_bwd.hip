@@ -720,35 +720,39 @@ static bool fused_bwd_wanted(const mote_relation_bwd_args* a) {
   return !(e && e[0] == '0');
 }
 
-// bf16: the atomic-free tile path, head dims off {32, 64, 96, 128} padded to the next of them (dh 48,
-// H 4, B 16, T 1241: 194 us register-staged, 109 here; dh 88, H 2, T 3000: 244 and 85; dh 104, B 2,
-// H 8, T 1000: 148 and 58; dh 48, B 2, H 4, T 256: 27 and 19).
-// The tiles' workspace grows with the pairs of blocks (8 KB each), the register-staged kernels' with the
-// rows: padded head dims whose pairs would take more than 8 GiB (H 4: 45 K rows) stay with the latter, so
-// a length that fitted the card before still does.
-static bool use_tiles(const mote_relation_bwd_args* a) {
-  if (a->dtype != MOTE_BF16 || !tile_strides_ok(a->p1, a->p2, a->info)) return false;
-  if (padded_dim(a->D) == a->D) return true;
-  return int64_t(a->B) * a->H * PairTable::total(a->TQ, a->q_start) <= (int64_t(8) << 30) / 8192;
+// Which kernels serve a call; both stored-dU paths have a smaller-scratch alternative (lean).
+// tiles: bf16 on the atomic-free tile path, head dims off {32, 64, 96, 128} padded to the next of them (dh 48,
+//   H 4, B 16, T 1241: 194 us register-staged, 109 here; dh 88, H 2, T 3000: 244 and 85; dh 104, B 2,
+//   H 8, T 1000: 148 and 58; dh 48, B 2, H 4, T 256: 27 and 19). Its scratch grows with the pairs of blocks
+//   (8 KB each), the register-staged kernels' with the rows, so a padded head dim takes at most 8 GiB of it
+//   (H 4: 45 K rows) and runs register-staged beyond.
+// f32_du: fp32 key blocks store dU (16 KB a pair) for the dP1 stage instead of adding dP1 with atomics or
+//   recomputing it; both modes, the results are reproducible either way. At most 2 GiB (H 8: 11 K rows).
+// lean: neither where the other kernels serve too. A caller that cannot spare the scratch passes
+//   mote_relation_bwd_workspace_min() bytes and gets these.
+struct BwdPlan {
+  bool tiles, f32_du;
+};
+static BwdPlan bwd_plan(const mote_relation_bwd_args* a, bool lean) {
+  const int64_t pairs = int64_t(a->B) * a->H * PairTable::total(a->TQ, a->q_start);
+  BwdPlan p{};
+  if (a->dtype == MOTE_F32)
+    p.f32_du = !lean && pairs <= (int64_t(2) << 30) / 16384;
+  else
+    p.tiles = tile_strides_ok(a->p1, a->p2, a->info) &&
+              (padded_dim(a->D) == a->D || (!lean && pairs <= (int64_t(8) << 30) / 8192));
+  return p;
 }
 
-// fp32: whether the key blocks store dU (16 KB per 64 x 64 pair) for the dP1 stage instead of adding dP1
-// with atomics or recomputing it; both modes, the results are reproducible either way. Up to 2 GiB of it
-// (H 8: 11 K rows), so that a length that fitted the card before still does.
-static bool f32_stores_du(const mote_relation_bwd_args* a) {
-  return a->dtype == MOTE_F32 && int64_t(a->B) * a->H * PairTable::total(a->TQ, a->q_start) <= (int64_t(2) << 30) / 16384;
-}
-
-static WsLayout ws_layout(const mote_relation_bwd_args* a) {
+static WsLayout ws_layout(const mote_relation_bwd_args* a, const BwdPlan& plan) {
   const size_t es = a->dtype == MOTE_BF16 ? 2 : 4;
   const size_t BH = size_t(a->B) * a->H;
   const size_t TQp = size_t((a->TQ + kRowBlock - 1) / kRowBlock) * kRowBlock;
   const size_t DP = padded_dim(a->D);
-  const bool tiles = use_tiles(a);
   WsLayout w{};
   size_t o = 0;
   w.wdib = o; o = align256(o + BH * TQp * DP * es);
-  if (tiles) {
+  if (plan.tiles) {
     w.stat = o; o = align256(o + BH * (TQp / kRowBlock) * 128 * 4);
     // dU fragments: 8 KB per visible (query block, key block) pair
     w.dut = o; o = align256(o + BH * size_t(PairTable::total(a->TQ, a->q_start)) * 8192);
@@ -761,7 +765,7 @@ static WsLayout ws_layout(const mote_relation_bwd_args* a) {
     }
     w.lse2 = o; o = align256(o + BH * TQp * 4);
     w.cvec = o; o = align256(o + BH * TQp * 4);
-    if (f32_stores_du(a)) {
+    if (plan.f32_du) {
       w.dut = o; o = align256(o + BH * size_t(PairTable::total(a->TQ, a->q_start)) * 16384);
     } else {
       w.dp1acc = o; o = align256(o + BH * size_t(a->TQ) * a->D * 4);
@@ -773,7 +777,11 @@ static WsLayout ws_layout(const mote_relation_bwd_args* a) {
   return w;
 }
 
-size_t bwd_workspace_bytes(const mote_relation_bwd_args* a) { return ws_layout(a).total; }
+size_t bwd_workspace_bytes(const mote_relation_bwd_args* a) { return ws_layout(a, bwd_plan(a, false)).total; }
+size_t bwd_workspace_min_bytes(const mote_relation_bwd_args* a) {  // (at a few rows the copies outweigh dU)
+  const size_t full = bwd_workspace_bytes(a), lean = ws_layout(a, bwd_plan(a, true)).total;
+  return lean < full ? lean : full;
+}
 
 // fp32, and bf16 off the tile kernels (register-staged).
 template <typename T, int DP>
@@ -831,7 +839,6 @@ int launch_bwd(const mote_relation_bwd_args* a, hipStream_t stream) {
   if (a->B <= 0 || a->H <= 0 || a->TQ < 0 || a->TK != a->q_start + a->TQ)
     return set_error(MOTE_ERR_SHAPE, "relation_bwd: bad sizes (TK=%d, q_start=%d, TQ=%d)", a->TK, a->q_start, a->TQ);
   if (!a->dlam) return set_error(MOTE_ERR_ARGUMENT, "relation_bwd: null dlam");
-  const WsLayout w = ws_layout(a);
   if (a->TQ == 0) {
     // no query rows: dP2 / dI~ of the prefix and dlam are zero (fill kernels, no memset nodes)
     const int es = a->dtype == MOTE_BF16 ? 2 : 4;
@@ -846,6 +853,12 @@ int launch_bwd(const mote_relation_bwd_args* a, hipStream_t stream) {
   if (!a->p1.data || !a->p2.data || !a->info.data || !a->dy.data || !a->ibar || !a->lse || !a->g || !a->dp1.data ||
       !a->dp2.data || !a->dinfo.data)
     return set_error(MOTE_ERR_ARGUMENT, "relation_bwd: null tensor pointer");
+  BwdPlan plan = bwd_plan(a, false);
+  WsLayout w = ws_layout(a, plan);
+  if (a->workspace_bytes < w.total) {
+    plan = bwd_plan(a, true);
+    w = ws_layout(a, plan);
+  }
   if (!a->workspace || a->workspace_bytes < w.total)
     return set_error(MOTE_ERR_WORKSPACE, "relation_bwd: workspace of %zu bytes, %zu needed", a->workspace_bytes, w.total);
   BwdParams p{};
@@ -858,12 +871,11 @@ int launch_bwd(const mote_relation_bwd_args* a, hipStream_t stream) {
   p.dp2 = a->dp2.data; p.dk_sb = a->dp2.stride_b; p.dk_sh = a->dp2.stride_h; p.dk_sr = a->dp2.stride_r;
   p.dinfo = a->dinfo.data; p.dv_sb = a->dinfo.stride_b; p.dv_sh = a->dinfo.stride_h; p.dv_sr = a->dinfo.stride_r;
   p.dlam = a->dlam;
-  const bool tiles = use_tiles(a);
   char* ws = reinterpret_cast<char*>(a->workspace);
   p.wdib = ws + w.wdib;
   p.duii = reinterpret_cast<float*>(ws + w.duii);
   p.dlam_part = reinterpret_cast<float*>(ws + w.dlam_part);
-  if (tiles) {
+  if (plan.tiles) {
     p.stat = reinterpret_cast<float*>(ws + w.stat);
     p.dut = ws + w.dut;
     p.npairs = PairTable::total(a->TQ, a->q_start);
@@ -885,7 +897,7 @@ int launch_bwd(const mote_relation_bwd_args* a, hipStream_t stream) {
     p.wq = ws + w.wq; p.wqT = ws + w.wqT; p.wdibT = ws + w.wdibT;
     p.lse2 = reinterpret_cast<float*>(ws + w.lse2);
     p.cvec = reinterpret_cast<float*>(ws + w.cvec);
-    if (f32_stores_du(a)) {
+    if (plan.f32_du) {
       p.dut = ws + w.dut;
       p.npairs = PairTable::total(a->TQ, a->q_start);
     } else {
@@ -899,7 +911,7 @@ int launch_bwd(const mote_relation_bwd_args* a, hipStream_t stream) {
   const int DP = padded_dim(a->D);
   const bool det = a->deterministic != 0;
   const int st = a->stages ? a->stages : (MOTE_BWD_ROWS | MOTE_BWD_KEYS | MOTE_BWD_QUERIES | MOTE_BWD_FINISH);
-  if (tiles) {
+  if (plan.tiles) {
     switch (DP) {
       case 32: launch_bwd_tile_path<32>(p, st, stream); break;
       case 64: launch_bwd_tile_path<64>(p, st, stream); break;

@@ -108,7 +108,15 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> relation_bwd(Tensor p1, Tensor p2, Te
   a.ibar = fptr(ibar); a.lse = fptr(lse); a.g = fptr(g);
   a.dp1 = view(dp1); a.dp2 = view(dp2); a.dinfo = view(dinfo);
   a.dlam = fptr(dlam);
-  const Tensor ws = bytes(mote_relation_bwd_workspace(&a), p1);
+  // a step that leaves too little memory for the stored dU runs without it
+  const size_t full = mote_relation_bwd_workspace(&a), least = mote_relation_bwd_workspace_min(&a);
+  Tensor ws;
+  try {
+    ws = bytes(full, p1);
+  } catch (const c10::OutOfMemoryError&) {
+    if (least == full) throw;
+    ws = bytes(least, p1);
+  }
   a.workspace = ws.data_ptr();
   a.workspace_bytes = size_t(ws.numel());
   check(mote_relation_bwd(&a, reinterpret_cast<void*>(stream)), "mote_relation_bwd");
