@@ -21,8 +21,9 @@
 //
 // What bounds it: the two transposed fragment reads per pair of products (LDS), and for the narrow
 // widths the bytes of the two operands. 576 x 192 over 19,856 rows (the 192-wide layer's stacked
-// projections, 30 MB of operands): 18.0 us with the sum, against 110 us for the GEMM library's product;
-// 2304 x 768 over 4964 rows 35.3 us (498 TFLOP/s), library 50; over 79,424 rows 351 us, library 524.
+// projections, 30 MB of operands): 17.8 us with the sum, against 110 us for the GEMM library's product;
+// 2304 x 768 over 4964 rows 32.3 us (544 TFLOP/s), library 50; over 79,424 rows 336 us (837 TFLOP/s), library
+// 524 (as graphs of ten calls).
 #include "common.hpp"
 #include "params.hpp"
 #include "tiles.hpp"
@@ -102,14 +103,17 @@ wgrad_kernel(const WgradParams p) {
     __builtin_amdgcn_s_waitcnt(0);  // this wave's transfers of stage b
     lds_barrier();
     const int r0 = m0 + b * kWgTok;
-    if (r0 + kWgTok > p.M) {
+    if (__builtin_expect(r0 + kWgTok > p.M, 0)) {
       // the last stage of the reduction: its rows past M hold copies of row M - 1; zero them in both
       // tiles (whole rows, so the chunk swizzle does not matter)
-      const int z0 = p.M - r0;  // first row past M
-      for (int q = threadIdx.x; q < (kWgTok - z0) * (TK / 8); q += 64 * kWgWaves)
-        *reinterpret_cast<bf16x8*>(cur + z0 * TK + q * 8) = bf16x8{};
-      for (int q = threadIdx.x; q < (kWgTok - z0) * (TN / 8); q += 64 * kWgWaves)
-        *reinterpret_cast<bf16x8*>(cur + XT + z0 * TN + q * 8) = bf16x8{};
+      // (one loop over both tiles, off the hot path, its bounds opaque: as two loops the compiler kept their
+      // addresses in registers that every stage advanced between the products, 351 us at 79,424 rows)
+      int z0 = p.M - r0;
+      asm volatile("" : "+s"(z0));
+      for (int q = threadIdx.x; q < (kWgTok - z0) * (TK + TN) / 8; q += 64 * kWgWaves) {
+        const int row = z0 + q / ((TK + TN) / 8), c = q % ((TK + TN) / 8) * 8;
+        *reinterpret_cast<bf16x8*>(cur + (c < TK ? row * TK + c : XT + row * TN + c - TK)) = bf16x8{};
+      }
       lds_barrier();
     }
     // every fragment of the stage, then the next stage's transfers into the other slot, then the
