@@ -195,13 +195,15 @@ bwd_keys_f32_kernel(const BwdParams p) {
           acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ua[r], Kt[off], acc, 0, 0, 0);
           acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ub[r], Kt[off + 16 * DP], acc, 0, 0, 0);
         }
+        // every block issues its AFTER adds: columns past D add zero to the row's own columns, each lane to
+        // another one; rows past TQ are in the last block alone, whose adds nothing counts, and add nothing
+        // (as zeros to one element, 4096 cached keys after one another took 170 us at T = 1)
         const int d = 16 * dt + li;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          // rows past TQ and columns past D add zero to a valid element: the count of adds stays fixed
           const int qi = qb * 32 + 16 * dqt + 4 * lg + r;
-          const bool ok = qi < p.TQ && d < D;
-          unsafeAtomicAdd(&p.dp1acc[(int64_t(bh) * p.TQ + min(qi, p.TQ - 1)) * D + min(d, D - 1)], ok ? acc[r] * p.scale : 0.f);
+          if (qi < p.TQ)
+            unsafeAtomicAdd(&p.dp1acc[(int64_t(bh) * p.TQ + qi) * D + d % D], d < D ? acc[r] * p.scale : 0.f);
         }
       }
     }
