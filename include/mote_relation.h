@@ -108,10 +108,11 @@ int mote_relation_fwd(const mote_relation_fwd_args* args, void* stream);
  * Inputs are the forward's inputs and saved statistics (ibar, lse, g as produced by
  * mote_relation_fwd, dense layout) and dy ([B, H, TQ, D], any strides). Outputs dp1 [B,H,TQ,D],
  * dp2 and dinfo [B,H,TK,D] in `dtype` (any strides) and dlam (one fp32, overwritten).
- * bf16 (row strides below 2^24 elements) runs atomic-free kernels (key-stationary dp2/dinfo, then
- * query-stationary dp1): every result is bitwise reproducible whatever `deterministic` says.
- * So does fp32 while its stored dU takes at most 2 GiB (16 KB per visible 64 x 64 pair).
- * Other shapes (longer fp32, padded bf16 head dims beyond 8 GiB of dU, longer row strides):
+ * bf16 with D in {32, 64, 96, 128} (row strides below 2^24 elements) runs atomic-free kernels (key-stationary
+ * dp2/dinfo, then query-stationary dp1): every result is bitwise reproducible whatever `deterministic` says.
+ * So do other bf16 head dims (padded) while their stored dU takes at most 8 GiB (8 KB per visible 64 x 64
+ * pair), and fp32 while it takes at most 2 GiB (16 KB a pair; 256 MB at D <= 32), except few queries after a
+ * longer cached prefix. Those and other shapes (longer row strides, a workspace below the full size):
  * `deterministic` != 0 selects the atomic-free pair of kernels (the reference's
  * MOTE_DETERMINISTIC_RELATION, flash_relation.py:51), 0 the one-pass kernel with fp32 atomics for dp1.
  * The workspace is caller-allocated device memory of mote_relation_bwd_workspace() bytes or more; its

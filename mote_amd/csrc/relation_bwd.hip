@@ -730,17 +730,34 @@ static bool fused_bwd_wanted(const mote_relation_bwd_args* a) {
 //   recomputing it; both modes, the results are reproducible either way. At most 2 GiB (H 8: 11 K rows).
 // lean: neither where the other kernels serve too. A caller that cannot spare the scratch passes
 //   mote_relation_bwd_workspace_min() bytes and gets these.
+// Few queries after a long cached prefix (a turn that is trained on) run lean as well unless `deterministic`: dP1's
+// own stage is then a handful of workgroups that each walk every key block, while atomics or register-staged
+// blocks spread over the keys. fp32, full and lean: dh 64, B H 8, 311 queries after 4096: 160 and 125 us; B H 16,
+// 1 after 4096: 104 and 41; B H 4, 620 after 1024: 77 and 70. Atomics cost by the head dim (dh 128, B H 16, 100
+// after 1024: 98 and 109; dh 96, B H 64, 100 after 4096: 450 and 479), so the line is a count of dP1's
+// workgroups that falls with its square; with as many queries as prefix they no longer win (dh 64, B H 1, 1300
+// after 1024: 114 and 117; without a prefix 94 and 115). dh 32 runs lean too where dU would pass the 256 MB of
+// the Infinity Cache (B H 64, T 2000: 523 and 482 us; 242 MB, T 1300: 229 and 233).
+// bf16, tiles and register-staged: dh 48, B H 8, 16 after 4096: 35 and 27 us; B H 4, 311: 50 and 41; B H 16, 100:
+// 50 and 53; B H 1, 620: 41 and 46; one query after 1024: 16 and 14, B H 64: 26 and 32.
 struct BwdPlan {
   bool tiles, f32_du;
 };
 static BwdPlan bwd_plan(const mote_relation_bwd_args* a, bool lean) {
-  const int64_t pairs = int64_t(a->B) * a->H * PairTable::total(a->TQ, a->q_start);
+  const int64_t BH = int64_t(a->B) * a->H, DP = padded_dim(a->D), w = DP * DP;
+  const int64_t pairs = BH * PairTable::total(a->TQ, a->q_start);
   BwdPlan p{};
-  if (a->dtype == MOTE_F32)
+  if (a->dtype == MOTE_F32) {
+    const bool few = a->TQ < a->q_start && BH * ((a->TQ + 31) / 32) * w < int64_t(device_cu_count()) * 64 * 64;
+    lean = lean || (!a->deterministic && (few || (DP == 32 && pairs > (int64_t(256) << 20) / 16384)));
     p.f32_du = !lean && pairs <= (int64_t(2) << 30) / 16384;
-  else
+  } else {
+    const bool few = a->q_start >= 1536 && 13 * int64_t(a->TQ) <= a->q_start && BH * a->TQ * w <= 1500 * 64 * 64 &&
+                     BH * w <= 32 * 64 * 64;
+    lean = lean || (!a->deterministic && few);
     p.tiles = tile_strides_ok(a->p1, a->p2, a->info) &&
               (padded_dim(a->D) == a->D || (!lean && pairs <= (int64_t(8) << 30) / 8192));
+  }
   return p;
 }
 

@@ -41,6 +41,23 @@ def test_sizes_agree_where_nothing_is_chosen(a):
     assert full == least > 0
 
 
+@pytest.mark.parametrize("dtype,B,H,T,S,D,stored", [
+    (L.MOTE_F32, 1, 8, 311, 4096, 64, False), (L.MOTE_F32, 1, 8, 311, 300, 64, True),     # fewer queries than prefix
+    (L.MOTE_F32, 1, 8, 1000, 1500, 64, True),                                             # as many workgroups as CUs
+    (L.MOTE_F32, 1, 16, 100, 1024, 128, True), (L.MOTE_F32, 1, 4, 311, 1024, 128, False),
+    (L.MOTE_F32, 8, 8, 1300, 0, 32, True), (L.MOTE_F32, 8, 8, 2000, 0, 32, False), (L.MOTE_F32, 8, 8, 2000, 0, 64, True),
+    (L.MOTE_BF16, 1, 4, 311, 4096, 48, False), (L.MOTE_BF16, 1, 4, 400, 4096, 48, True), (L.MOTE_BF16, 1, 2, 300, 1024, 48, True),
+    (L.MOTE_BF16, 1, 1, 311, 4096, 120, False), (L.MOTE_BF16, 1, 8, 1, 8192, 64, True),
+])
+def test_few_queries_after_a_prefix_store_no_du(dtype, B, H, T, S, D, stored):
+    """The rule's two sides: dU (8 or 16 KB a pair) is in the workspace or is not; a deterministic call stores it."""
+    a = _args(dtype, B, H, T, D, S)
+    a.deterministic = 1
+    det = L.lib().mote_relation_bwd_workspace(a)
+    a.deterministic = 0
+    assert (L.lib().mote_relation_bwd_workspace(a) == det) == stored
+
+
 @pytest.mark.parametrize("T", [1, 64, 65, 200])
 def test_least_workspace_is_never_the_larger(T):
     for dtype, D in ((L.MOTE_BF16, 40), (L.MOTE_BF16, 120), (L.MOTE_F32, 8), (L.MOTE_F32, 128)):
@@ -96,6 +113,27 @@ def test_backward_on_the_least_workspace(cuda, dtype, D, B, H, T, S, det):
         assert rel_err(x, y) < tol, (name, rel_err(x, y))
     terms = O.relation_dlam_terms(*ref, lr, dy.cpu().double(), 2.0, S)
     assert abs(float(dlam) - float(dr[3])) < tol * max(float(terms.abs().sum()), 1e-3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,D,T,S", [(torch.float32, 24, 1, 70), (torch.float32, 48, 33, 300), (torch.float32, 96, 100, 101),
+                                         (torch.bfloat16, 48, 1, 1536), (torch.bfloat16, 88, 65, 2000), (torch.bfloat16, 120, 7, 1600)])
+def test_few_queries_after_a_prefix_match_oracle(cuda, dtype, D, T, S):
+    """The route of few queries through the op, tolerances as above."""
+    from mote_amd.flash_relation import flash_relation
+
+    print(f"case few queries {dtype} D={D} T={T} S={S}", flush=True)
+    p1, p2, info, lam, dy = _case(dtype, 1, 2, T, D, S, cuda)
+    xs = [t.requires_grad_(True) for t in (p1, p2, info, lam)]
+    got = torch.autograd.grad(flash_relation(*xs, 2.0, S)[0], xs, dy)
+    tol = 2e-2 if dtype == torch.bfloat16 else 1e-5
+    ref = [t.detach().cpu().double() for t in (p1, p2, info)]
+    lr = torch.tensor(0.4, dtype=torch.float64)
+    dr = O.relation_backward(*ref, lr, dy.cpu().double(), 2.0, S)
+    for name, x, y in zip(("dp1", "dp2", "dinfo"), got, dr):
+        assert rel_err(x, y) < tol, (name, rel_err(x, y))
+    terms = O.relation_dlam_terms(*ref, lr, dy.cpu().double(), 2.0, S)
+    assert abs(float(got[3]) - float(dr[3])) < tol * max(float(terms.abs().sum()), 1e-3)
 
 
 @pytest.mark.gpu
