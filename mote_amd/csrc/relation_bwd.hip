@@ -23,6 +23,12 @@
 //    recomputes w and dU per (query block, key block) and accumulates dQ in registers instead of
 //    atomics (the reference's two-pass `_bwd_q_kernel`, flash_relation.py:419-460), so every
 //    result is bitwise reproducible. dlam: a fixed-order sum of the row partials.
+//
+// This is the register-staged bf16 form (bwd_keys_kernel, bwd_queries_kernel). Most calls take another form of
+// stages 2 and 3 (bwd_plan): bf16 the tile kernels (relation_bwd_tiles.hip) and fp32 the staged key kernel
+// (relation_bwd_f32.hip), both with dU stored by the key blocks and read by dP1's own stage, without atomics
+// in either mode. fp32 without a stored dU keeps the staged key kernel with the atomics of stage 2, or
+// the query-stationary kernel in deterministic mode.
 #include "common.hpp"
 #include "bwd.hpp"
 

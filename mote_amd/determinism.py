@@ -1,10 +1,16 @@
 """Reproducible-backward switch for the Relation path (the interface of mote/determinism.py:41-62).
 
 What varies between two identical backward passes here:
-* the bf16 tile backward (every head dim) never varies: it has no atomics, and dlam is summed in a fixed
-  order by one workgroup;
-* the fp32 backward (and bf16 rows 2^24 or more elements apart) adds dP1 with fp32 atomics unless `DETERMINISTIC` is set,
-  which selects the query-stationary pass instead;
+* the bf16 tile backward never varies: it has no atomics, and dlam is summed in a fixed order by one
+  workgroup. It serves head dims 32 / 64 / 96 / 128, and others while their stored dU takes at most 8 GiB
+  (8 KB per visible 64 x 64 block pair);
+* nor does the fp32 backward while its stored dU takes at most 2 GiB (16 KB a pair; 256 MB at head dims
+  up to 32);
+* everything else adds dP1 with fp32 atomics unless `DETERMINISTIC` is set: longer fp32 and padded bf16
+  shapes, few queries after a much longer cached prefix (fp32, padded bf16), rows 2^24 or more elements
+  apart (bf16), and a call that is given less workspace than the stored dU needs, as the package's own
+  launcher does where the card has no room for it. `DETERMINISTIC` stores dU for few queries after a
+  prefix too and selects the query-stationary pass where dU is not stored;
 * library GEMMs around the path (projections, `wo`) follow torch's deterministic-algorithms mode.
 
 `apply(reproducible)` sets all three the way the reference's switch does: the environment variable
