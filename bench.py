@@ -1002,17 +1002,17 @@ def bench_qkv(rows: int, dev, copies: int, launches: int = 20):
 
 
 def bench_wgrad(rows: int, dev, copies: int, launches: int = 20):
-    """mote::wgrad, the prologue's weight gradient dW = dqkv^T x at the Mote-96M shape (dqkv bf16
+    """mote::linear_wgrad, the prologue's weight gradient dW = dqkv^T x (bf16 out) at the Mote-96M shape (dqkv bf16
     [rows, 2304], x bf16 [rows, 768]), against the GEMM library's dqkv^T x (torch.matmul of the
     transposed view, what the unfused backward runs); each a HIP graph of `launches` launches over
     `copies` input sets. Work: 2 rows 3D D FLOP."""
-    from mote_amd.relation import _wgrad
+    from mote_amd.relation import _linear_wgrad
 
     D = D_MODEL
     g = torch.Generator(device="cpu").manual_seed(9)
     sets = [(torch.randn(rows, 3 * D, generator=g).to(torch.bfloat16).to(dev),
              torch.randn(rows, D, generator=g).to(torch.bfloat16).to(dev)) for _ in range(copies)]
-    fns = {"mote_wgrad": lambda i: _wgrad(*sets[i % copies]),
+    fns = {"mote_wgrad": lambda i: _linear_wgrad(*sets[i % copies], torch.bfloat16),
            "library": lambda i: torch.matmul(sets[i % copies][0].t(), sets[i % copies][1])}
     a, b = fns["mote_wgrad"](0), fns["library"](0)
     diff = float((a.float() - b.float()).abs().max()) / max(float(b.float().abs().max()), 1e-3)
