@@ -1,4 +1,6 @@
-// Fused Relation forward for gfx950.
+// Fused Relation forward for gfx950: the register-staged kernel described here (bf16 rows too far apart for
+// the tiles), then the bf16 tile kernel, which serves every other bf16 call, and the merge of its key-range
+// pieces. fp32 is relation_fwd_f32.hip.
 //
 // One workgroup owns BM = 32 * NW query rows of one (sequence, head); wave w owns rows
 // [32w, 32w + 32) as two 16-row tiles. The strictly-past keys are streamed in blocks of BN rows:
@@ -346,7 +348,7 @@ __global__ void __launch_bounds__(NW * 64) relation_fwd_kernel(const FwdParams p
 }
 
 // ------------------------------------------------------------------------------------------------
-// bf16 tile kernel for D in {32, 64, 96, 128}
+// bf16 tile kernel: D in {32, 64, 96, 128} as they are, other head dims padded to the next of these (PAD)
 //
 // One workgroup of four waves per 64 query rows of one (sequence, head). P2 and I~ blocks of 64 rows
 // are staged global -> LDS (tiles.hpp), double-buffered. Wave w owns the 32 x 32 quadrant (query

@@ -1,8 +1,9 @@
 // Native launchers of the torch ops: output allocation, argument blocks and the C-ABI calls of the ops whose
-// Python bodies did the same through ctypes. A body's allocations, views and argument fields took 19 to
-// 25 us of interpreter time a call (the forward 18.0, the backward 25.1), 7.9 and 10.8 here, and a small layer's step is paced by them. Dispatch,
-// autograd, fake implementations and every check of what a call may pass stay with the Python ops;
-// these functions take tensors those have accepted and raise RuntimeError with the library's message
+// Python bodies did the same through ctypes. A body's allocations, views and argument fields took 18 to
+// 25 us of interpreter time a call (the forward 18.0, the backward 25.1), 7.9 and 10.8 here, and a small
+// layer's step is paced by them. Dispatch, autograd and fake implementations stay with the Python ops, and
+// so do checks of what a call may pass, except the sizes, types and devices of operands whose extent the
+// kernel takes from another one: those are compared here. RuntimeError with the library's message
 // when a call fails. Host code only; streams come as raw handles.
 #include <torch/extension.h>
 

@@ -219,7 +219,7 @@ class ChunkLayer(nn.Module):
             M = min(Ln, -(-M // self.bucket) * self.bucket)
         out = chunk_gather(hidden, perm, num, boundary_mask, cum, M)
         # in num's own type: against int64 positions the comparison converted every element (11 us for
-        # 8 x 5056 flags, 4 so)
+        # 8 x 5056 flags, 6 so)
         next_mask = torch.arange(M, device=hidden.device, dtype=num.dtype)[None, :] < num[:, None]
         return out, next_mask
 

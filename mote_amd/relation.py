@@ -3,10 +3,10 @@
 Same constructor, parameter names and construction order (relation.py:97-157), same forward
 signature and return convention (relation.py:184-268). What runs underneath:
 
-    p1, p2, I~ = mote::qkv_rope(x, [w1; w2; wi])  HIP: one launch for the projections with RoPE on
-                                                 p1/p2 and Givens on I~ in the epilogue (bf16,
-                                                 dh 64 / 96 / 128, no QK-Norm); otherwise one
-                                                 hipBLASLt GEMM and mote::rope_givens
+    p1, p2, I~ = mote::qkv_rope(x, [w1; w2; wi])  HIP: one launch for the projections with QK-Norm and
+                                                 RoPE on p1/p2 and Givens on I~ in the epilogue
+                                                 (bf16, dh 64 / 96 / 128, and 48 without QK-Norm);
+                                                 otherwise one hipBLASLt GEMM and mote::rope_givens
     Y, g = mote::relation_fwd(p1, P2, I~)        HIP: the fused Relation core (any T, decode too)
     out = wo(Y [* sigmoid(wg x)])                 Y is token-major already, so no transpose copy
 
