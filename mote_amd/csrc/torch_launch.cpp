@@ -277,7 +277,7 @@ std::tuple<Tensor, Tensor, Tensor> add_rms_norm_bwd(const Tensor& dy, const OptT
 
 // The fused prologue; ws: the stacked weight, or the three (p1, p2, I~ projections); p2 / info: views to
 // write instead of new tensors. The kernel reads its operands at the sizes that x and H give: they are checked
-// against those here. The cos / sin table (memoised by the caller) comes as `table`.
+// against those here (a longer stack, frequency or angle tensor is read at its start). The cos / sin table (memoised by the caller) comes as `table`.
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> qkv_rope(const Tensor& x, const std::vector<Tensor>& ws, const OptTensor& inv_freq,
                                                             const OptTensor& theta, int64_t H, int64_t parity, int64_t pos0,
                                                             bool keep_info, const OptTensor& norm_w1, const OptTensor& norm_w2,
@@ -287,11 +287,11 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> qkv_rope(const Tensor& x, con
   const at::ScalarType dt = x.scalar_type();
   TORCH_CHECK(dt == at::kBFloat16 && K == H * D && x.is_contiguous(), "qkv_rope: x must be bf16 of ", H, " heads, got ", dt, " rows of ", K);
   for (const Tensor& w : ws)
-    TORCH_CHECK(w.sizes() == at::IntArrayRef({ws.size() == 3 ? K : 3 * K, K}) && w.scalar_type() == dt &&
-                    w.device() == x.device() && w.is_contiguous(),
+    TORCH_CHECK(w.dim() == 2 && (ws.size() == 3 ? w.size(0) == K : w.size(0) >= 3 * K) && w.size(1) == K &&
+                    w.scalar_type() == dt && w.device() == x.device() && w.is_contiguous(),
                 "qkv_rope: weights must be contiguous bf16 [", K, ", ", K, "] each or [", 3 * K, ", ", K, "] stacked, on x's device");
-  TORCH_CHECK(!inv_freq || inv_freq->numel() == D / 2, "qkv_rope: inv_freq needs ", D / 2, " values");
-  TORCH_CHECK(!theta || theta->numel() == H / 2, "qkv_rope: theta needs ", H / 2, " values");
+  TORCH_CHECK(!inv_freq || inv_freq->numel() >= D / 2, "qkv_rope: inv_freq needs ", D / 2, " values");
+  TORCH_CHECK(!theta || theta->numel() >= H / 2, "qkv_rope: theta needs ", H / 2, " values");
   for (const OptTensor* t : {&p2_, &info_})  // the caller's memory: the kernel writes all of [B, H, T, D]
     TORCH_CHECK(!t->has_value() || ((*t)->sizes() == at::IntArrayRef({B, H, T, D}) && (*t)->scalar_type() == dt &&
                                     (*t)->device() == x.device()),
