@@ -388,14 +388,16 @@ def linear_wgrad(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     wb = w
     if torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") == torch.bfloat16 and x.is_cuda:
         x, wb = x.to(torch.bfloat16), w.to(torch.bfloat16)  # (F.linear itself would not cast fp64)
-    if x.is_cuda and w.is_cuda and _wgrad_serves(x.dtype, wb.dtype, *w.shape) and not _transformed():
+    # (without a backward the function would only cost 2 us of host time)
+    if torch.is_grad_enabled() and x.is_cuda and w.is_cuda and _wgrad_serves(x.dtype, wb.dtype, *w.shape) and not _transformed():
         # fp32 weights take dW from the function itself, others through their cast
         return _LinearWgrad.apply(x, w if w.dtype == torch.float32 else wb, wb)
     return F.linear(x, wb)
 
 
-def _qr_grads(ctx, dp1, dp2, dinfo, wdtype):
-    """(dx, dW of the stacked weight in wdtype, dtheta, the gains' gradients) of the fused prologue."""
+def _qr_grads(ctx, dp1, dp2, dinfo, wdtype, need_w):
+    """(dx, dW of the stacked weight in wdtype, dtheta, the gains' gradients) of the fused prologue; dx and,
+    without need_w, dW are None where nothing takes them (the products are most of this backward)."""
     x, w, inv_freq, theta, iraw, norm_w1, norm_w2, qkraw = ctx.saved_tensors
     if (ctx.has_theta or ctx.norm) and not ctx.keep:
         raise RuntimeError("mote::qkv_rope: the backward needs keep_info=True with theta or QK-Norm")
@@ -412,13 +414,13 @@ def _qr_grads(ctx, dp1, dp2, dinfo, wdtype):
     if ctx.norm:  # gradients of the normalised p1 / p2 back through QK-Norm, in place in dqkv
         dn1, dn2 = _head_norm_bwd_(dqkv, qkraw, norm_w1, norm_w2, ctx.eps, H)
         dn1, dn2 = dn1.to(norm_w1.dtype), dn2.to(norm_w2.dtype)
-    dx = torch.matmul(dqkv, w)                                        # [B, T, 3K] x [3K, K]
-    dw = weight_grad(dqkv, x, wdtype)                                # [3K, K]
+    dx = torch.matmul(dqkv, w) if ctx.needs_input_grad[0] else None   # [B, T, 3K] x [3K, K]
+    dw = weight_grad(dqkv, x, wdtype) if need_w else None             # [3K, K]
     return dx, dw, (dtheta[: H // 2] if ctx.has_theta else None), dn1, dn2
 
 
 def _qr_backward(ctx, dp1, dp2, dinfo, _diraw, _dqkraw):
-    dx, dw, dtheta, dn1, dn2 = _qr_grads(ctx, dp1, dp2, dinfo, None)
+    dx, dw, dtheta, dn1, dn2 = _qr_grads(ctx, dp1, dp2, dinfo, None, ctx.needs_input_grad[1])
     return dx, dw, None, dtheta, None, None, None, None, dn1, dn2, None
 
 
@@ -485,8 +487,8 @@ def _qrm_backward(ctx, dp1, dp2, dinfo, _diraw, _dqkraw, _dw):
     if not ctx.train:
         raise RuntimeError("mote::qkv_rope_master: the backward needs train=True")
     wdtype = torch.float32 if torch.float32 in ctx.w_dtypes else None
-    dx, dw, dtheta, dn1, dn2 = _qr_grads(ctx, dp1, dp2, dinfo, wdtype)
-    dws = (d.to(t) for d, t in zip(dw.chunk(3), ctx.w_dtypes))
+    dx, dw, dtheta, dn1, dn2 = _qr_grads(ctx, dp1, dp2, dinfo, wdtype, any(ctx.needs_input_grad[1:4]))
+    dws = (None,) * 3 if dw is None else (d.to(t) for d, t in zip(dw.chunk(3), ctx.w_dtypes))
     return (dx, *dws, None, dtheta, None, None, None, None, None, dn1, dn2, None)
 
 

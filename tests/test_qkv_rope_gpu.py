@@ -419,6 +419,46 @@ def test_prologue_head_dim_48(cuda, monkeypatch, T, B, layer):
         assert a.dtype == b.dtype and rel_err(a, b) < 1.6e-2, rel_err(a, b)
 
 
+def test_prologue_backward_computes_only_what_is_taken(cuda):
+    """A first layer's input and frozen weights take no gradient: no product runs for them (head dim 48 ran
+    without them before it was fused), the other gradients keep their bits."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from mote_amd.relation import qkv_rope, rope_inv_freq
+
+    print("case prologue backward, gradients not taken", flush=True)
+
+    class Products(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if func.__name__.split(".")[0] in ("mm", "bmm", "linear_wgrad"):
+                self.names.append(func.__name__.split(".")[0])
+            return func(*args, **(kwargs or {}))
+
+    g = torch.Generator().manual_seed(12)
+    inv = rope_inv_freq(48, 10000.0).to(cuda)
+    theta = torch.rand(2, generator=g).to(cuda).requires_grad_(True)
+    x = torch.randn(1, 70, 192, generator=g).bfloat16().to(cuda).requires_grad_(True)
+    ws = [(torch.randn(192, 192, generator=g) / 14).to(cuda).requires_grad_(True) for _ in range(3)]
+    dy = [torch.randn(1, 4, 70, 48, generator=g).bfloat16().to(cuda) for _ in range(3)]
+
+    def grads(x, ws, want):
+        out = qkv_rope(x, tuple(ws), 4, inv, theta, 1)
+        with Products() as seen:
+            got = torch.autograd.grad(out, want, dy)
+        return got, sorted(seen.names)
+
+    full, names = grads(x, ws, [x, *ws, theta])
+    assert len(names) == 2 and "linear_wgrad" in names
+    got, names = grads(x.detach(), ws, [*ws, theta])
+    assert names == ["linear_wgrad"] and all(torch.equal(a, b) for a, b in zip(got, full[1:]))
+    got, names = grads(x, [w.detach() for w in ws], [x, theta])
+    assert names in (["mm"], ["bmm"]) and torch.equal(got[0], full[0]) and torch.equal(got[1], full[4])
+
+
 @pytest.mark.parametrize("d,H", [(192, 4), (256, 4)])
 @pytest.mark.parametrize("T", [1, 33])
 def test_prologue_takes_x_off_a_boundary(cuda, d, H, T):
