@@ -334,9 +334,13 @@ def _linear_wgrad_fake(a, x, dtype):
 
 
 def _wgrad_serves(a_dtype: torch.dtype, x_dtype: torch.dtype, N: int, K: int) -> bool:
-    """bf16 operands, both widths multiples of 64 (the kernel's smallest tile of dW). Below 128 the
-    library's product, whose reduction runs over the token rows, is the slower one too: 576 x 192 over
-    19,856 rows 18 us here, 110 us there."""
+    """bf16 operands, both widths multiples of 64 (the kernel's smallest tile of dW), any number of rows.
+    Widths that are not multiples of 128 are faster here from one row on (576 x 192: 3.6 us here and 4.5 on
+    the library, whose reduction runs over the token rows, at 1 row, 6.6 and 13.1 at 1000, 18 and 110 at
+    19,856). Multiples of 128 are within a microsecond up to 256 rows and faster here from about 2500 (2304 x 768:
+    5.9 and 5.8 us at 1 row, 25.7 and 33.3 at 3000), but slower in between, where two to four splits of the rows
+    are summed by a second launch (1000 rows: 24.2 and 15.5, or 24.4 and 19.4 with the cast to fp32; 512 x 512:
+    10.6 and 13.1): they stay here, since the library's fp32 gradient would be rounded to bf16 first."""
     return USE_WGRAD and a_dtype == torch.bfloat16 and x_dtype == torch.bfloat16 and N % 64 == 0 and K % 64 == 0
 
 
@@ -388,7 +392,8 @@ def linear_wgrad(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     wb = w
     if torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") == torch.bfloat16 and x.is_cuda:
         x, wb = x.to(torch.bfloat16), w.to(torch.bfloat16)  # (F.linear itself would not cast fp64)
-    # (without a backward the function would only cost 2 us of host time)
+    # without a backward the function would only cost host time: 2 us with the checks before it, which a short
+    # extension feels (311 rows after 4096 cached ones: 126.8 us a call with them, 116.5 so)
     if torch.is_grad_enabled() and x.is_cuda and w.is_cuda and _wgrad_serves(x.dtype, wb.dtype, *w.shape) and not _transformed():
         # fp32 weights take dW from the function itself, others through their cast
         return _LinearWgrad.apply(x, w if w.dtype == torch.float32 else wb, wb)
