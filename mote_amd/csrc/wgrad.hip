@@ -22,8 +22,8 @@
 // What bounds it: the two transposed fragment reads per pair of products (LDS), and for the narrow
 // widths the bytes of the two operands. 576 x 192 over 19,856 rows (the 192-wide layer's stacked
 // projections, 30 MB of operands): 17.8 us with the sum, against 110 us for the GEMM library's product;
-// 2304 x 768 over 4964 rows 32.3 us (544 TFLOP/s), library 50; over 79,424 rows 336 us (837 TFLOP/s), library
-// 524 (as graphs of ten calls).
+// 2304 x 768 over 4964 rows 32.3 us (544 TFLOP/s; 36.1 over eight input sets in turn), library 50; over 79,424
+// rows 336 us (837 TFLOP/s), library 524 (as graphs of ten calls).
 #include "common.hpp"
 #include "params.hpp"
 #include "tiles.hpp"
